@@ -60,10 +60,10 @@ int order_rows_by_degree(ent_graph *g) {
       return rc;                                                                   \
     }                                                                              \
   } while (0)
-  ORD_TRY(hipMalloc(&vclass, size_t(n)));
-  ORD_TRY(hipMalloc(&keys, size_t(m)));
-  ORD_TRY(hipMalloc(&keys_out, size_t(m)));
-  ORD_TRY(hipMalloc(&adj_out, sizeof(int) * size_t(m)));
+  ORD_TRY(device_malloc(g->device, reinterpret_cast<void **>(&vclass), size_t(n)));
+  ORD_TRY(device_malloc(g->device, reinterpret_cast<void **>(&keys), size_t(m)));
+  ORD_TRY(device_malloc(g->device, reinterpret_cast<void **>(&keys_out), size_t(m)));
+  ORD_TRY(device_malloc(g->device, reinterpret_cast<void **>(&adj_out), sizeof(int) * size_t(m)));
   const int grid = std::max(1, g->cus) * 8;
   hipLaunchKernelGGL(k_vertex_class, dim3(grid), dim3(256), 0, s, st.off, (long long)n, vclass);
   ORD_TRY(hipGetLastError());
@@ -72,7 +72,7 @@ int order_rows_by_degree(ent_graph *g) {
   const long long *beg = st.off, *end = st.off + 1;
   ORD_TRY(rocprim::segmented_radix_sort_pairs_desc(nullptr, tmp_bytes, keys, keys_out, st.adj, adj_out,
                                                    unsigned(m), unsigned(n), beg, end, 0, 6, s));
-  ORD_TRY(hipMalloc(&tmp, std::max<size_t>(tmp_bytes, 1)));
+  ORD_TRY(device_malloc(g->device, reinterpret_cast<void **>(&tmp), std::max<size_t>(tmp_bytes, 1)));
   ORD_TRY(rocprim::segmented_radix_sort_pairs_desc(tmp, tmp_bytes, keys, keys_out, st.adj, adj_out, unsigned(m),
                                                    unsigned(n), beg, end, 0, 6, s));
   ORD_TRY(hipStreamSynchronize(s));

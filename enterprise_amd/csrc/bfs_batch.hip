@@ -1735,7 +1735,7 @@ int ent_device_alloc(ent_graph *g, int64_t bytes, void **out) {
   if (!g || !out || bytes < 0) return set_error(ENT_EINVAL, "bad argument");
   HIP_TRY(hipSetDevice(g->device));
   *out = nullptr;
-  hipError_t e = hipMalloc(out, size_t(std::max<int64_t>(bytes, 8)));
+  hipError_t e = device_malloc(g->device, out, size_t(std::max<int64_t>(bytes, 8)));
   if (e != hipSuccess) {
     ignore(hipGetLastError());
     return set_error(ENT_ENOMEM, "hipMalloc(%lld) failed: %s", (long long)bytes, hipGetErrorString(e));

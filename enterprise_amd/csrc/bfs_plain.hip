@@ -1900,7 +1900,9 @@ int ent_graph_free(ent_graph *g) {
     ignore(hipSetDevice(g->device));
     ignore(hipStreamSynchronize(g->stream));
   }
+  const int device = g->device;
   release(g);
+  build_give_back(device);
   return ENT_OK;
 }
 

@@ -27,6 +27,9 @@
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <mutex>
+#include <new>
 #include <vector>
 
 #include "ent_bfs.h"
@@ -191,6 +194,14 @@ __global__ __launch_bounds__(kBuildBlock) void k_fill_gaps(const Gap *gaps, cons
   }
 }
 
+}  // namespace
+}  // namespace ent
+
+#include "csr_msd.h"
+
+namespace ent {
+namespace {
+
 int grid_for(long long items, int cus) {
   return int(std::max<long long>(1, std::min<long long>((long long)cus * 16, (items + kBuildBlock - 1) / kBuildBlock)));
 }
@@ -200,8 +211,8 @@ struct DevBuf {
   ~DevBuf() {
     if (p) ignore(hipFree(p));
   }
-  int alloc(size_t bytes, const char *what) {
-    if (hipMalloc(&p, std::max<size_t>(bytes, 16)) != hipSuccess) {
+  int alloc(int device, size_t bytes, const char *what) {
+    if (device_malloc(device, &p, std::max<size_t>(bytes, 16)) != hipSuccess) {
       ignore(hipGetLastError());
       p = nullptr;
       return set_error(ENT_ENOMEM, "hipMalloc of %zu bytes (%s) failed", bytes, what);
@@ -214,8 +225,304 @@ struct DevBuf {
   }
 };
 
-// The whole construction on `stream`; w_in/w_out may be null. Returns m.
-int build_csr(int device, hipStream_t stream, long long n, long long ne, const int *src, const int *dst,
+// What one construction needs on a device: a stream, two events and a block
+// of scratch memory. The calls take no handle, so the last idle context of
+// each device waits here for the next one: allocating and freeing the scratch
+// costs 0.6 ms a call at 1.6 GB, and the driver's clearing of freed memory
+// stalls calls in a row for 10 to 1,000 ms. Bounded: one context per device,
+// of at most kIdleBytes; concurrent calls make their own. Given back when a
+// library allocation fails and when a graph handle of the device is freed.
+constexpr size_t kIdleBytes = size_t(4) << 30;
+
+struct BuildContext {
+  int device = 0, cus = 0;
+  hipStream_t stream = nullptr;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  void *mem = nullptr;
+  size_t bytes = 0;
+
+  ~BuildContext() {
+    if (hipSetDevice(device) != hipSuccess) return;
+    if (e0) ignore(hipEventDestroy(e0));
+    if (e1) ignore(hipEventDestroy(e1));
+    if (stream) ignore(hipStreamDestroy(stream));
+    if (mem) ignore(hipFree(mem));
+  }
+  int init(int dev) {
+    device = dev;
+    HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+    HIP_TRY(hipEventCreate(&e0));
+    HIP_TRY(hipEventCreate(&e1));
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    return ENT_OK;
+  }
+  int reserve(size_t want) {
+    if (want <= bytes) return ENT_OK;
+    if (mem) ignore(hipFree(mem));
+    mem = nullptr;
+    bytes = 0;
+    if (device_malloc(device, &mem, want) != hipSuccess) {
+      ignore(hipGetLastError());
+      mem = nullptr;
+      return set_error(ENT_ENOMEM, "hipMalloc of %zu bytes (construction scratch) failed", want);
+    }
+    bytes = want;
+    return ENT_OK;
+  }
+};
+
+std::mutex g_idle_mu;
+std::vector<std::unique_ptr<BuildContext>> &idle_contexts() {
+  // Never destroyed: the runtime may be gone when static objects are.
+  static auto *v = new std::vector<std::unique_ptr<BuildContext>>();
+  return *v;
+}
+
+// A call's hold on a context. The stream is drained before the context is
+// idle again, also after an error.
+struct ContextLease {
+  std::unique_ptr<BuildContext> c;
+  int take(int device) {
+    {
+      std::lock_guard<std::mutex> lk(g_idle_mu);
+      auto &v = idle_contexts();
+      for (size_t i = 0; i < v.size(); ++i)
+        if (v[i]->device == device) {
+          c = std::move(v[i]);
+          v.erase(v.begin() + long(i));
+          return ENT_OK;
+        }
+    }
+    c.reset(new (std::nothrow) BuildContext());
+    if (!c) return set_error(ENT_ENOMEM, "out of host memory");
+    return c->init(device);
+  }
+  ~ContextLease() { give(); }
+  void give() {
+    std::unique_ptr<BuildContext> c = std::move(this->c);
+    if (!c) return;
+    if (!c->stream || !c->e1 || hipStreamSynchronize(c->stream) != hipSuccess || c->bytes > kIdleBytes) return;
+    std::lock_guard<std::mutex> lk(g_idle_mu);
+    auto &v = idle_contexts();
+    for (auto &x : v)
+      if (x->device == c->device) {  // another call came back first: keep the larger block
+        if (x->bytes < c->bytes) std::swap(x, c);
+        return;
+      }
+    v.push_back(std::move(c));
+  }
+};
+
+// Offsets of a scratch block, 256-byte aligned.
+struct Carver {
+  size_t at = 0;
+  size_t take(size_t bytes) {
+    const size_t o = at;
+    at += (std::max<size_t>(bytes, 16) + 255) / 256 * 256;
+    return o;
+  }
+};
+
+// Leaf bits and partition passes for sorted rows without weights. False
+// when the rest of a key would not fit 32 bits (n above 2^24): those keys
+// take the radix sort.
+bool msd_plan(const BuildShape &s, MsdPlan *p) {
+  p->cb = s.cb;
+  const int least = std::max(0, 2 * s.cb - 32), most = std::min(s.cb, kMaxLeafBits);
+  if (least > most) return false;
+  int b = 0;
+  while (b < most && (s.records >> b) > kLeafTarget) ++b;
+  p->b = std::max(b, least);
+  p->b1 = std::min(p->b, 8);
+  p->b2 = p->b - p->b1;
+  p->rem = 2 * s.cb - p->b;
+  p->nb = int(std::min<long long>(256, (s.ne + (1 << 14) - 1) >> 14));
+  p->halves = p->b > kHistBits ? 2 : 1;
+  return true;
+}
+
+hipError_t allow_lds(const void *fn, size_t bytes) {
+  return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
+}
+
+// Sorted rows without weights by partition (csr_msd.h). plan() sizes the
+// scratch, run() queues the kernels.
+struct MsdBuild {
+  MsdPlan p;
+  unsigned tiles = 0;
+  size_t o_wide = 0, o_keys = 0, o_mc = 0, o_counts = 0, o_off = 0, o_cur1 = 0, o_cur2 = 0, o_lists = 0, o_crowded = 0,
+         o_chunks = 0, o_tc = 0, o_to = 0, o_hist = 0;
+
+  void plan(const BuildShape &s, Carver &cv) {
+    const size_t R = size_t(s.records), L = size_t(1) << p.b;
+    tiles = unsigned((s.records + kEmitTile - 1) >> kEmitShift);
+    o_keys = cv.take(4 * R);
+    // 64-bit keys between the passes; afterwards the merge buffer.
+    o_wide = cv.take(p.b2 ? 8 * R : R > size_t(kChunk) ? 4 * R : 0);
+    o_mc = cv.take(sizeof(MsdCounts));
+    o_counts = cv.take(4 * L);
+    o_off = cv.take(4 * (L + 1));
+    o_cur1 = cv.take(4 * kMaxFan);
+    o_cur2 = cv.take(4 * L);
+    o_lists = cv.take(4 * L * kLeafClasses);
+    o_crowded = cv.take(4 * L);
+    o_chunks = cv.take(sizeof(Chunk) * (2 * (R / kChunk) + 1));
+    o_tc = cv.take(4 * size_t(tiles));
+    o_to = cv.take(4 * (size_t(tiles) + 1));
+    o_hist = cv.take(4 * L * size_t(p.nb));
+  }
+
+  template <int T>
+  void sort_class(int k, hipStream_t stream, int cus, const BuildShape &s, const unsigned *lists, MsdCounts *mc,
+                  const unsigned *off, unsigned *k32, unsigned *tile_cnt, unsigned *crowded) const {
+    if (k && s.records <= (long long)kLeafSmall << (k - 1)) return;
+    // Blocks that fit the LDS at once (27, 51 and 99 KB each).
+    const unsigned grid = std::min(1u << p.b, unsigned(cus) * (k == 0 ? 6u : k == 1 ? 3u : 1u));
+    hipLaunchKernelGGL(k_leaf_bins<T>, dim3(grid), dim3(T), 0, stream, p, s.dedup, lists + (size_t(k) << p.b),
+                       &mc->leaves[k], off, k32, tile_cnt, crowded, &mc->crowded);
+  }
+
+  int run(BuildContext &c, const BuildShape &s, const int *src, const int *dst, long long *beg, int *adj, Gap *gaps,
+          unsigned long long *ngaps) const {
+    char *base = static_cast<char *>(c.mem);
+    auto u = [&](size_t o) { return reinterpret_cast<unsigned *>(base + o); };
+    unsigned *k32 = u(o_keys), *counts = u(o_counts), *off = u(o_off), *cur1 = u(o_cur1), *cur2 = u(o_cur2),
+             *lists = u(o_lists), *crowded = u(o_crowded), *tile_cnt = u(o_tc), *tile_off = u(o_to), *hist = u(o_hist);
+    unsigned long long *k64 = reinterpret_cast<unsigned long long *>(base + o_wide);
+    MsdCounts *mc = reinterpret_cast<MsdCounts *>(base + o_mc);
+    Chunk *chunks = reinterpret_cast<Chunk *>(base + o_chunks);
+    hipStream_t stream = c.stream;
+    const unsigned L = 1u << p.b;
+    const size_t hist_lds = size_t(4) << std::min(p.b, kHistBits);
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_msd_hist), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(hist_lds)));
+    hipLaunchKernelGGL(k_msd_hist, dim3(unsigned(p.nb), unsigned(p.halves)), dim3(kHistThreads), hist_lds, stream, s,
+                       p, src, dst, hist, mc, tile_cnt, tiles, ngaps);
+    hipLaunchKernelGGL(k_msd_reduce, dim3((L + kWave - 1) / kWave), dim3(256), 0, stream, p, hist, counts, lists,
+                       chunks, mc);
+    hipLaunchKernelGGL(k_scan, dim3(1), dim3(kScanThreads), 0, stream, counts, off, L, cur1, cur2, p.b2);
+    const long long per = (s.rev ? kPartItems / 2 : kPartItems) * (long long)kPartThreads;
+    const unsigned t1 = unsigned((s.ne + per - 1) / per);
+    if (p.b2) {
+      hipLaunchKernelGGL(k_msd_part1<unsigned long long>, dim3(t1), dim3(kPartThreads), 0, stream, s, p, src, dst,
+                         cur1, k64);
+      const unsigned t2 = unsigned(s.records / kPartTile) + (1u << p.b1);
+      hipLaunchKernelGGL(k_msd_part2, dim3(t2), dim3(kPartThreads), 0, stream, p, k64, off, cur2, k32);
+    } else {
+      hipLaunchKernelGGL(k_msd_part1<unsigned>, dim3(t1), dim3(kPartThreads), 0, stream, s, p, src, dst, cur1, k32);
+    }
+    sort_class<256>(0, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
+    sort_class<512>(1, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
+    sort_class<1024>(2, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
+    HIP_TRY(hipGetLastError());
+    MsdCounts h{};
+    h.crowded = L;  // up to kChunk records nothing but this can be left over
+    if (s.records > kChunk) {
+      HIP_TRY(hipMemcpyAsync(&h, mc, sizeof h, hipMemcpyDeviceToHost, stream));
+      HIP_TRY(hipStreamSynchronize(stream));
+    }
+    if (h.crowded)
+      hipLaunchKernelGGL((k_leaf_sort<1024, kLeafItems>), dim3(std::min(h.crowded, unsigned(c.cus) * 2)), dim3(1024), 0,
+                         stream, p, s.dedup, crowded, &mc->crowded, off, k32, tile_cnt);
+    if (h.chunks) {
+      // The number of merge passes follows from the largest leaf; the sorted
+      // chunks go where it leaves the result in k32.
+      unsigned *other = reinterpret_cast<unsigned *>(k64);
+      int passes = 0;
+      while (((unsigned long long)kChunk << passes) < h.max_size) ++passes;
+      hipLaunchKernelGGL(k_chunk_place, dim3(std::min((h.chunks + 255) / 256, 1024u)), dim3(256), 0, stream, mc, off,
+                         chunks);
+      unsigned *from = (passes & 1) ? other : k32, *to = (passes & 1) ? k32 : other;
+      hipLaunchKernelGGL((k_chunk_sort<1024, kLeafItems>), dim3(std::min(h.chunks, unsigned(c.cus) * 2)), dim3(1024),
+                         0, stream, p, chunks, mc, k32, from);
+      for (int i = 0; i < passes; ++i) {
+        hipLaunchKernelGGL(k_leaf_merge, dim3(h.chunks, kChunk / kMergeTile), dim3(kMergeThreads), 0, stream, chunks,
+                           from, to, (unsigned long long)kChunk << i, s.dedup && i == passes - 1 ? tile_cnt : nullptr);
+        std::swap(from, to);
+      }
+    }
+    if (s.dedup)
+      hipLaunchKernelGGL(k_scan, dim3(1), dim3(kScanThreads), 0, stream, tile_cnt, tile_off, tiles, nullptr, nullptr,
+                         0);
+    hipLaunchKernelGGL(k_emit, dim3((tiles + 3) / 4), dim3(kEmitThreads), 0, stream, s, p, k32, off, tile_off, tiles,
+                       beg, adj, gaps, ngaps);
+    HIP_TRY(hipGetLastError());
+    return ENT_OK;
+  }
+};
+
+// Every other form: a least-significant-digit radix sort of 64-bit keys, with
+// the record index where rows keep the tuples' order or carry weights.
+struct RadixBuild {
+  bool keys_only = false;
+  int kbits = 0;
+  long long ntiles = 1;
+  size_t o_k0 = 0, o_k1 = 0, o_i0 = 0, o_i1 = 0, o_tiles = 0, o_tmp = 0, sort_bytes = 0, scan_bytes = 0;
+
+  int plan(const BuildShape &s, int bits, bool weights, hipStream_t stream, Carver &cv) {
+    const size_t R = size_t(s.records);
+    keys_only = s.sorted && !weights;
+    kbits = bits;
+    ntiles = std::max<long long>(1, (s.records + kTile - 1) / kTile);
+    o_k0 = cv.take(8 * R);
+    o_k1 = cv.take(8 * R);
+    o_i0 = cv.take(keys_only ? 0 : 4 * R);
+    o_i1 = cv.take(keys_only ? 0 : 4 * R);
+    o_tiles = cv.take(8 * size_t(2 * ntiles + 1));
+    // Scratch for the sort and the scan of tile counts.
+    rocprim::double_buffer<unsigned long long> kb(nullptr, nullptr);
+    rocprim::double_buffer<unsigned> vb(nullptr, nullptr);
+    unsigned long long *none = nullptr;
+    if (keys_only)
+      HIP_TRY(rocprim::radix_sort_keys(nullptr, sort_bytes, kb, R, 0u, unsigned(kbits), stream));
+    else
+      HIP_TRY(rocprim::radix_sort_pairs(nullptr, sort_bytes, kb, vb, R, 0u, unsigned(kbits), stream));
+    HIP_TRY(rocprim::inclusive_scan(nullptr, scan_bytes, none, none, size_t(ntiles),
+                                    rocprim::plus<unsigned long long>(), stream));
+    o_tmp = cv.take(std::max(sort_bytes, scan_bytes));
+    return ENT_OK;
+  }
+
+  int run(BuildContext &c, const BuildShape &s, const int *src, const int *dst, const int *w_in, long long *beg,
+          int *adj, int *w_out, Gap *gaps, unsigned long long *ngaps) const {
+    hipStream_t stream = c.stream;
+    // beg starts at zero: with no kept record nothing else writes it.
+    HIP_TRY(hipMemsetAsync(ngaps, 0, 8, stream));
+    HIP_TRY(hipMemsetAsync(beg, 0, 8 * size_t(s.n + 1ll), stream));
+    const size_t R = size_t(s.records);
+    if (!R) return ENT_OK;
+    char *base = static_cast<char *>(c.mem);
+    auto u64 = [&](size_t o) { return reinterpret_cast<unsigned long long *>(base + o); };
+    auto u32 = [&](size_t o) { return reinterpret_cast<unsigned *>(base + o); };
+    rocprim::double_buffer<unsigned long long> kb(u64(o_k0), u64(o_k1));
+    rocprim::double_buffer<unsigned> vb(u32(o_i0), u32(o_i1));
+    void *tmp = base + o_tmp;
+    hipLaunchKernelGGL(k_records, dim3(grid_for(s.records, c.cus)), dim3(kBuildBlock), 0, stream, s, src, dst,
+                       kb.current(), keys_only ? nullptr : vb.current());
+    HIP_TRY(hipGetLastError());
+    size_t tb = sort_bytes;
+    if (keys_only)
+      HIP_TRY(rocprim::radix_sort_keys(tmp, tb, kb, R, 0u, unsigned(kbits), stream));
+    else
+      HIP_TRY(rocprim::radix_sort_pairs(tmp, tb, kb, vb, R, 0u, unsigned(kbits), stream));
+    // Kept records per tile, their running sum, then every kept record at its
+    // rank.
+    unsigned long long *tile_cnt = u64(o_tiles), *tile_off = tile_cnt + ntiles;
+    HIP_TRY(hipMemsetAsync(tile_cnt, 0, 8 * size_t(2 * ntiles + 1), stream));
+    hipLaunchKernelGGL(k_tile_count, dim3(unsigned(ntiles)), dim3(kBuildBlock), 0, stream, s, kb.current(), tile_cnt);
+    HIP_TRY(hipGetLastError());
+    tb = scan_bytes;
+    HIP_TRY(rocprim::inclusive_scan(tmp, tb, tile_cnt, tile_off + 1, size_t(ntiles),
+                                    rocprim::plus<unsigned long long>(), stream));
+    hipLaunchKernelGGL(k_tile_assemble, dim3(unsigned(ntiles)), dim3(kBuildBlock), 0, stream, s, kb.current(),
+                       keys_only ? nullptr : vb.current(), tile_off, src, dst, w_in, beg, adj, w_out, gaps, ngaps);
+    HIP_TRY(hipGetLastError());
+    return ENT_OK;
+  }
+};
+
+// The whole construction on the context's stream; w_in/w_out may be null.
+int build_csr(BuildContext &c, long long n, long long ne, const int *src, const int *dst,
               const int *w_in, int flags, long long *beg, int *adj, long long adj_cap, int *w_out,
               long long *m_out, ent_build_stats *st) {
   if (n < 0 || n > INT32_MAX || ne < 0) return set_error(ENT_EINVAL, "bad sizes n=%lld ne=%lld", n, ne);
@@ -234,73 +541,26 @@ int build_csr(int device, hipStream_t stream, long long n, long long ne, const i
   if (adj_cap < s.records) return set_error(ENT_EINVAL, "adjacency capacity %lld < %lld records", adj_cap, s.records);
   const int kbits = s.sorted ? s.cb + bits_for(uint64_t(n)) : bits_for(uint64_t(n));
   if (kbits > 64) return set_error(ENT_EINVAL, "key of %d bits", kbits);
-  int cus = 0;
-  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-  const bool keys_only = s.sorted && !w_in;
-  const size_t R = size_t(s.records);
-  DevBuf k0, k1, i0, i1, cnt, tmp, gaps;
-  int rc;
-  if ((rc = k0.alloc(8 * R, "keys")) || (rc = k1.alloc(8 * R, "keys")) || (rc = cnt.alloc(16, "counts")) ||
-      (rc = gaps.alloc(sizeof(Gap) * kGapCap, "row gaps")))
+  Carver cv;
+  const size_t o_cnt = cv.take(16), o_gaps = cv.take(sizeof(Gap) * kGapCap);
+  MsdBuild msd;
+  RadixBuild radix;
+  const bool part = s.records && s.sorted && !w_in && msd_plan(s, &msd.p);
+  int rc = ENT_OK;
+  if (part) msd.plan(s, cv);
+  else if ((rc = radix.plan(s, kbits, w_in != nullptr, c.stream, cv))) return rc;
+  if ((rc = c.reserve(cv.at))) return rc;
+  char *mem = static_cast<char *>(c.mem);
+  unsigned long long *ngaps = reinterpret_cast<unsigned long long *>(mem + o_cnt);
+  Gap *gaps = reinterpret_cast<Gap *>(mem + o_gaps);
+  hipStream_t stream = c.stream;
+  HIP_TRY(hipEventRecord(c.e0, stream));
+  if ((rc = part ? msd.run(c, s, src, dst, beg, adj, gaps, ngaps)
+                 : radix.run(c, s, src, dst, w_in, beg, adj, w_out, gaps, ngaps)))
     return rc;
-  if (!keys_only && ((rc = i0.alloc(4 * R, "record indices")) || (rc = i1.alloc(4 * R, "record indices")))) return rc;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  HIP_TRY(hipEventCreate(&e0));
-  HIP_TRY(hipEventCreate(&e1));
-  struct EvGuard {
-    hipEvent_t a, b;
-    ~EvGuard() {
-      ignore(hipEventDestroy(a));
-      ignore(hipEventDestroy(b));
-    }
-  } evg{e0, e1};
-  rocprim::double_buffer<unsigned long long> keys(k0.as<unsigned long long>(), k1.as<unsigned long long>());
-  rocprim::double_buffer<unsigned> vals(i0.as<unsigned>(), i1.as<unsigned>());
-  // Scratch for the sort and the scan of tile counts, sized once.
-  const long long ntiles = std::max<long long>(1, (s.records + kTile - 1) / kTile);
-  DevBuf tiles;
-  if ((rc = tiles.alloc(8 * size_t(2 * ntiles + 1), "tile counts"))) return rc;
-  unsigned long long *tile_cnt = tiles.as<unsigned long long>(), *tile_off = tile_cnt + ntiles;
-  size_t tb_sort = 0, tb_scan = 0;
-  if (keys_only)
-    HIP_TRY(rocprim::radix_sort_keys(nullptr, tb_sort, keys, R, 0u, unsigned(kbits), stream));
-  else
-    HIP_TRY(rocprim::radix_sort_pairs(nullptr, tb_sort, keys, vals, R, 0u, unsigned(kbits), stream));
-  HIP_TRY(rocprim::inclusive_scan(nullptr, tb_scan, tile_cnt, tile_off + 1, size_t(ntiles),
-                                  rocprim::plus<unsigned long long>(), stream));
-  if ((rc = tmp.alloc(std::max(tb_sort, tb_scan), "sort scratch"))) return rc;
-  HIP_TRY(hipEventRecord(e0, stream));
-  if (R) {
-    hipLaunchKernelGGL(k_records, dim3(grid_for(s.records, cus)), dim3(kBuildBlock), 0, stream, s, src, dst,
-                       keys.current(), keys_only ? nullptr : vals.current());
-    HIP_TRY(hipGetLastError());
-    size_t tb = tb_sort;
-    if (keys_only)
-      HIP_TRY(rocprim::radix_sort_keys(tmp.p, tb, keys, R, 0u, unsigned(kbits), stream));
-    else
-      HIP_TRY(rocprim::radix_sort_pairs(tmp.p, tb, keys, vals, R, 0u, unsigned(kbits), stream));
-  }
-  // Kept records per tile, their running sum, then every kept record at its
-  // rank. beg starts at zero: with no kept record nothing else writes it.
-  unsigned long long *ngaps = cnt.as<unsigned long long>() + 1;
-  HIP_TRY(hipMemsetAsync(ngaps, 0, 8, stream));
-  HIP_TRY(hipMemsetAsync(tiles.p, 0, 8 * size_t(2 * ntiles + 1), stream));
-  HIP_TRY(hipMemsetAsync(beg, 0, 8 * size_t(n + 1), stream));
-  if (R) {
-    hipLaunchKernelGGL(k_tile_count, dim3(unsigned(ntiles)), dim3(kBuildBlock), 0, stream, s, keys.current(),
-                       tile_cnt);
-    HIP_TRY(hipGetLastError());
-    size_t tb = tb_scan;
-    HIP_TRY(rocprim::inclusive_scan(tmp.p, tb, tile_cnt, tile_off + 1, size_t(ntiles),
-                                    rocprim::plus<unsigned long long>(), stream));
-    hipLaunchKernelGGL(k_tile_assemble, dim3(unsigned(ntiles)), dim3(kBuildBlock), 0, stream, s, keys.current(),
-                       keys_only ? nullptr : vals.current(), tile_off, src, dst, w_in, beg, adj, w_out,
-                       gaps.as<Gap>(), ngaps);
-    HIP_TRY(hipGetLastError());
-  }
-  hipLaunchKernelGGL(k_fill_gaps, dim3(cus * 4), dim3(kBuildBlock), 0, stream, gaps.as<Gap>(), ngaps, beg);
+  hipLaunchKernelGGL(k_fill_gaps, dim3(c.cus * 4), dim3(kBuildBlock), 0, stream, gaps, ngaps, beg);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipEventRecord(e1, stream));
+  HIP_TRY(hipEventRecord(c.e1, stream));
   long long m = 0;
   HIP_TRY(hipMemcpyAsync(&m, beg + n, 8, hipMemcpyDeviceToHost, stream));
   HIP_TRY(hipStreamSynchronize(stream));
@@ -311,7 +571,7 @@ int build_csr(int device, hipStream_t stream, long long n, long long ne, const i
     st->m = m;
     st->key_bits = kbits;
     float ms = 0.f;
-    if (hipEventElapsedTime(&ms, e0, e1) == hipSuccess) st->device_ms = ms;
+    if (hipEventElapsedTime(&ms, c.e0, c.e1) == hipSuccess) st->device_ms = ms;
   }
   return ENT_OK;
 }
@@ -336,10 +596,10 @@ int check_tuples(int64_t n, int64_t ne, const int32_t *src, const int32_t *dst) 
 // Copies host tuples (and weights) to new device buffers on `stream`.
 struct DevTuples {
   DevBuf s, d, w;
-  int upload(hipStream_t stream, int64_t ne, const int32_t *src, const int32_t *dst, const int32_t *weight) {
+  int upload(int device, hipStream_t stream, int64_t ne, const int32_t *src, const int32_t *dst, const int32_t *weight) {
     int rc;
-    if ((rc = s.alloc(4 * size_t(ne), "tuples")) || (rc = d.alloc(4 * size_t(ne), "tuples"))) return rc;
-    if (weight && (rc = w.alloc(4 * size_t(ne), "weights"))) return rc;
+    if ((rc = s.alloc(device, 4 * size_t(ne), "tuples")) || (rc = d.alloc(device, 4 * size_t(ne), "tuples"))) return rc;
+    if (weight && (rc = w.alloc(device, 4 * size_t(ne), "weights"))) return rc;
     if (ne) {
       HIP_TRY(hipMemcpyAsync(s.p, src, 4 * size_t(ne), hipMemcpyHostToDevice, stream));
       HIP_TRY(hipMemcpyAsync(d.p, dst, 4 * size_t(ne), hipMemcpyHostToDevice, stream));
@@ -349,14 +609,15 @@ struct DevTuples {
   }
 };
 
-struct StreamGuard {
-  hipStream_t s = nullptr;
-  ~StreamGuard() {
-    if (s) ignore(hipStreamDestroy(s));
-  }
-};
-
 }  // namespace
+
+void build_give_back(int device) {
+  std::lock_guard<std::mutex> lk(g_idle_mu);
+  auto &v = idle_contexts();
+  for (size_t i = v.size(); i-- > 0;)
+    if (v[i]->device == device) v.erase(v.begin() + long(i));
+}
+
 }  // namespace ent
 
 using namespace ent;
@@ -370,10 +631,11 @@ int ent_csr_build_device(int32_t device, int64_t n, int64_t ne, const int32_t *s
   if (!beg_pos_dev || !m_out || (ne > 0 && (!src_dev || !dst_dev || !adj_dev)))
     return set_error(ENT_EINVAL, "NULL argument");
   HIP_TRY(hipSetDevice(device));
-  StreamGuard sg;
-  HIP_TRY(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
+  ContextLease ctx;
+  int rc = ctx.take(device);
+  if (rc) return rc;
   long long m = 0;
-  const int rc = build_csr(device, sg.s, n, ne, src_dev, dst_dev, nullptr, flags,
+  rc = build_csr(*ctx.c, n, ne, src_dev, dst_dev, nullptr, flags,
                            reinterpret_cast<long long *>(beg_pos_dev), adj_dev, adj_capacity, nullptr, &m, st);
   if (rc) return rc;
   *m_out = m;
@@ -389,16 +651,17 @@ int ent_csr_build(int32_t device, int64_t n, int64_t ne, const int32_t *src, con
   std::memset(out, 0, sizeof *out);
   if (weight_out) *weight_out = nullptr;
   HIP_TRY(hipSetDevice(device));
-  StreamGuard sg;
-  HIP_TRY(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
+  ContextLease ctx;
+  if ((rc = ctx.take(device))) return rc;
+  hipStream_t stream = ctx.c->stream;
   const int64_t records = ne * ((flags & ENT_CSR_REVERSE) ? 2 : 1);
   DevTuples dt;
   DevBuf db, da, dwo;
-  if ((rc = dt.upload(sg.s, ne, src, dst, weight)) || (rc = db.alloc(8 * size_t(n + 1), "offsets")) ||
-      (rc = da.alloc(4 * size_t(records), "adjacency")) || (weight && (rc = dwo.alloc(4 * size_t(records), "weights"))))
+  if ((rc = dt.upload(device, stream, ne, src, dst, weight)) || (rc = db.alloc(device, 8 * size_t(n + 1), "offsets")) ||
+      (rc = da.alloc(device, 4 * size_t(records), "adjacency")) || (weight && (rc = dwo.alloc(device, 4 * size_t(records), "weights"))))
     return rc;
   long long m = 0;
-  if ((rc = build_csr(device, sg.s, n, ne, dt.s.as<int>(), dt.d.as<int>(), weight ? dt.w.as<int>() : nullptr, flags,
+  if ((rc = build_csr(*ctx.c, n, ne, dt.s.as<int>(), dt.d.as<int>(), weight ? dt.w.as<int>() : nullptr, flags,
                       db.as<long long>(), da.as<int>(), records, weight ? dwo.as<int>() : nullptr, &m, st)))
     return rc;
   int64_t *beg = static_cast<int64_t *>(std::malloc(8 * size_t(n + 1)));
@@ -412,10 +675,10 @@ int ent_csr_build(int32_t device, int64_t n, int64_t ne, const int32_t *src, con
   };
   if (!beg || !adj || (weight_out && weight && !wh))
     return fail(set_error(ENT_ENOMEM, "out of host memory (%lld entries)", m));
-  hipError_t e = hipMemcpyAsync(beg, db.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, sg.s);
-  if (e == hipSuccess && m) e = hipMemcpyAsync(adj, da.p, 4 * size_t(m), hipMemcpyDeviceToHost, sg.s);
-  if (e == hipSuccess && wh && m) e = hipMemcpyAsync(wh, dwo.p, 4 * size_t(m), hipMemcpyDeviceToHost, sg.s);
-  if (e == hipSuccess) e = hipStreamSynchronize(sg.s);
+  hipError_t e = hipMemcpyAsync(beg, db.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, stream);
+  if (e == hipSuccess && m) e = hipMemcpyAsync(adj, da.p, 4 * size_t(m), hipMemcpyDeviceToHost, stream);
+  if (e == hipSuccess && wh && m) e = hipMemcpyAsync(wh, dwo.p, 4 * size_t(m), hipMemcpyDeviceToHost, stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (e != hipSuccess) return fail(set_error(ENT_EDEVICE, "copy of the CSR to the host failed: %s", hipGetErrorString(e)));
   out->n = n;
   out->m = m;
@@ -435,23 +698,25 @@ int ent_graph_upload_edges(const int32_t *src, const int32_t *dst, int64_t n, in
   int rc = check_tuples(n, ne, src, dst);
   if (rc) return rc;
   HIP_TRY(hipSetDevice(device));
-  StreamGuard sg;
-  HIP_TRY(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
+  ContextLease ctx;
+  if ((rc = ctx.take(device))) return rc;
+  hipStream_t stream = ctx.c->stream;
   const int64_t records = ne * ((flags & ENT_CSR_REVERSE) ? 2 : 1);
   DevTuples dt;
   DevBuf db, da;
-  if ((rc = dt.upload(sg.s, ne, src, dst, nullptr)) || (rc = db.alloc(8 * size_t(n + 1), "offsets")) ||
-      (rc = da.alloc(4 * size_t(records), "adjacency")))
+  if ((rc = dt.upload(device, stream, ne, src, dst, nullptr)) || (rc = db.alloc(device, 8 * size_t(n + 1), "offsets")) ||
+      (rc = da.alloc(device, 4 * size_t(records), "adjacency")))
     return rc;
   long long m = 0;
-  if ((rc = build_csr(device, sg.s, n, ne, dt.s.as<int>(), dt.d.as<int>(), nullptr, flags, db.as<long long>(),
+  if ((rc = build_csr(*ctx.c, n, ne, dt.s.as<int>(), dt.d.as<int>(), nullptr, flags, db.as<long long>(),
                       da.as<int>(), records, nullptr, &m, nullptr)))
     return rc;
   // The offsets come back for the host-side degree tables; the adjacency is
   // copied device to device into the handle's CSR.
   std::vector<int64_t> beg(size_t(n) + 1);
-  HIP_TRY(hipMemcpyAsync(beg.data(), db.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, sg.s));
-  HIP_TRY(hipStreamSynchronize(sg.s));
+  HIP_TRY(hipMemcpyAsync(beg.data(), db.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, stream));
+  HIP_TRY(hipStreamSynchronize(stream));
+  ctx.give();
   return upload_graph(beg.data(), da.as<int32_t>(), true, n, m, device, upload_flags, out);
 }
 

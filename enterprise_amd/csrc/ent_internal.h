@@ -111,9 +111,21 @@ namespace ent {
 // Rows one ent_device_row_hash launch sums (its per-handle buffer's length).
 constexpr int kHashRows = 512;
 
+// Frees the idle construction context of `device` (csr_build.hip).
+void build_give_back(int device);
+
+// hipMalloc that gives the idle construction context back before it fails.
+inline hipError_t device_malloc(int device, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  ignore(hipGetLastError());
+  build_give_back(device);
+  return hipMalloc(p, bytes);
+}
+
 inline int dev_alloc(ent_graph *g, void **p, size_t bytes) {
   if (bytes == 0) bytes = 8;
-  hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = device_malloc(g->device, p, bytes);
   if (e != hipSuccess) {
     *p = nullptr;
     ignore(hipGetLastError());

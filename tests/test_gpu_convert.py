@@ -165,3 +165,51 @@ def test_upload_edges_bfs(oracle):
         for r in h.pick_roots(4, 77):
             got, _ = dg.bfs(int(r))
             assert np.array_equal(got, oracle.bfs(h.beg_pos, h.adj, int(r))), r
+
+
+def _one_row(n, ne, seed):
+    """Every tuple in row 0 (one leaf holds them all), columns repeating."""
+    rng = np.random.default_rng(seed)
+    return np.zeros(ne, np.int32), rng.integers(0, n, ne).astype(np.int32)
+
+
+PARTITION_CASES = {
+    # Largest leaf of each sort kernel, one record less and more, and merged
+    # leaves of 2, 3 and 7 chunks (odd and even numbers of merge passes).
+    **{f"row0_{ne}": (lambda ne=ne: (1000, *_one_row(1000, ne, ne)))
+       for ne in (1, 2, 63, 64, 65, 4095, 4096, 4097, 16383, 16384, 16385, 32769, 49153, 100001)},
+    # A hub among ordinary rows, its columns spread over 2^20 ids.
+    "hub": lambda: (1 << 20, *(np.concatenate(x) for x in zip(_one_row(1 << 20, 70000, 5), _tuples(6, 1 << 20, 50000)))),
+    # Tile edges of the partition passes.
+    **{f"tile_{ne}": (lambda ne=ne: (5000, *_tuples(ne, 5000, ne)))
+       for ne in (3510, 3511, 4095, 4096, 4097, 8191, 8192, 8193)},
+    # One pass and two, every vertex count around a power of two.
+    **{f"n_{n}": (lambda n=n: (n, *_tuples(n, n, 20000)))
+       for n in (1, 2, 255, 256, 257, 65535, 65536, 65537, (1 << 20) + 1, 1 << 22, (1 << 23) + 5, 1 << 24,
+                 (1 << 24) + 1)},
+    # Columns close together in an id range of 2^20: bins above their limit.
+    **{f"crowded_{ne}": (lambda ne=ne: (1 << 20, *(np.concatenate(x) for x in zip(
+        _one_row(512, ne, ne), _tuples(9, 1 << 20, 9000))))) for ne in (700, 9000, 16384, 40000)},
+    "two_passes": lambda: (1 << 16, *_tuples(3, 1 << 16, 1200000)),
+}
+
+
+@pytest.mark.parametrize("case", list(PARTITION_CASES))
+def test_sorted_rows_by_partition(oracle, case):
+    """Sorted rows without weights at the edges of the partition build (leaf
+    and tile sizes, passes, key widths; the largest n takes the radix sort):
+    the oracle's CSR, bit for bit."""
+    n, src, dst = PARTITION_CASES[case]()
+    for flags in (L.CSR_SORT, L.CSR_SORT | L.CSR_REVERSE, L.CSR_DEDUP | L.CSR_NO_LOOPS, L.CSR_SIMPLE):
+        _say(f"[gpu] csr_build {case} n={n} ne={src.size} flags={flags}")
+        g, _, st = convert.csr_build(n, src, dst, flags)
+        b, a, _ = oracle.csr_build(n, src, dst, flags)
+        assert np.array_equal(g.beg_pos, b) and np.array_equal(g.adj, a), flags
+        assert st["m"] == a.size
+
+
+def test_partition_drops_every_record():
+    """Loops alone, all dropped: an empty CSR."""
+    ids = np.arange(3000, dtype=np.int32)
+    g, _, st = convert.csr_build(3000, ids, ids, L.CSR_SIMPLE)
+    assert g.m == 0 and st["m"] == 0 and not g.beg_pos.any()
