@@ -237,7 +237,11 @@ constexpr size_t kIdleBytes = size_t(4) << 30;
 struct BuildContext {
   int device = 0, cus = 0;
   hipStream_t stream = nullptr;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
+  hipEvent_t e0 = nullptr, e1 = nullptr, e_counts = nullptr;
+  struct Host {  // pinned
+    long long m;
+    MsdCounts counts;
+  } *host = nullptr;
   void *mem = nullptr;
   size_t bytes = 0;
 
@@ -245,6 +249,8 @@ struct BuildContext {
     if (hipSetDevice(device) != hipSuccess) return;
     if (e0) ignore(hipEventDestroy(e0));
     if (e1) ignore(hipEventDestroy(e1));
+    if (e_counts) ignore(hipEventDestroy(e_counts));
+    if (host) ignore(hipHostFree(host));
     if (stream) ignore(hipStreamDestroy(stream));
     if (mem) ignore(hipFree(mem));
   }
@@ -253,6 +259,8 @@ struct BuildContext {
     HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
+    HIP_TRY(hipEventCreateWithFlags(&e_counts, hipEventDisableTiming));
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&host), sizeof(Host), hipHostMallocDefault));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     return ENT_OK;
   }
@@ -301,7 +309,7 @@ struct ContextLease {
   void give() {
     std::unique_ptr<BuildContext> c = std::move(this->c);
     if (!c) return;
-    if (!c->stream || !c->e1 || hipStreamSynchronize(c->stream) != hipSuccess || c->bytes > kIdleBytes) return;
+    if (!c->stream || !c->host || hipStreamSynchronize(c->stream) != hipSuccess || c->bytes > kIdleBytes) return;
     std::lock_guard<std::mutex> lk(g_idle_mu);
     auto &v = idle_contexts();
     for (auto &x : v)
@@ -351,7 +359,7 @@ struct MsdBuild {
   MsdPlan p;
   unsigned tiles = 0;
   size_t o_wide = 0, o_keys = 0, o_mc = 0, o_counts = 0, o_off = 0, o_cur1 = 0, o_cur2 = 0, o_lists = 0, o_crowded = 0,
-         o_chunks = 0, o_tc = 0, o_to = 0, o_hist = 0;
+         o_crowded2 = 0, o_chunks = 0, o_tc = 0, o_to = 0, o_hist = 0;
 
   void plan(const BuildShape &s, Carver &cv) {
     const size_t R = size_t(s.records), L = size_t(1) << p.b;
@@ -367,6 +375,7 @@ struct MsdBuild {
     o_lists = cv.take(4 * L * kLeafClasses);
     o_crowded = cv.take(4 * L);
     o_chunks = cv.take(sizeof(Chunk) * (2 * (R / kChunk) + 1));
+    o_crowded2 = cv.take(4 * (2 * (R / kChunk) + 1));
     o_tc = cv.take(4 * size_t(tiles));
     o_to = cv.take(4 * (size_t(tiles) + 1));
     o_hist = cv.take(4 * L * size_t(p.nb));
@@ -379,7 +388,7 @@ struct MsdBuild {
     // Blocks that fit the LDS at once (27, 51 and 99 KB each).
     const unsigned grid = std::min(1u << p.b, unsigned(cus) * (k == 0 ? 6u : k == 1 ? 3u : 1u));
     hipLaunchKernelGGL(k_leaf_bins<T>, dim3(grid), dim3(T), 0, stream, p, s.dedup, lists + (size_t(k) << p.b),
-                       &mc->leaves[k], off, k32, tile_cnt, crowded, &mc->crowded);
+                       nullptr, &mc->leaves[k], off, k32, k32, tile_cnt, crowded, &mc->crowded[0]);
   }
 
   int run(BuildContext &c, const BuildShape &s, const int *src, const int *dst, long long *beg, int *adj, Gap *gaps,
@@ -400,45 +409,54 @@ struct MsdBuild {
                        p, src, dst, hist, mc, tile_cnt, tiles, ngaps);
     hipLaunchKernelGGL(k_msd_reduce, dim3((L + kWave - 1) / kWave), dim3(256), 0, stream, p, hist, counts, lists,
                        chunks, mc);
+    if (s.records > kChunk) {
+      HIP_TRY(hipMemcpyAsync(&c.host->counts, mc, sizeof(MsdCounts), hipMemcpyDeviceToHost, stream));
+      HIP_TRY(hipEventRecord(c.e_counts, stream));
+    }
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(kScanThreads), 0, stream, counts, off, L, cur1, cur2, p.b2);
-    const long long per = (s.rev ? kPartItems / 2 : kPartItems) * (long long)kPartThreads;
+    const long long per = (s.rev ? kPart1Items / 2 : kPart1Items) * (long long)kPart1Threads;
     const unsigned t1 = unsigned((s.ne + per - 1) / per);
     if (p.b2) {
-      hipLaunchKernelGGL(k_msd_part1<unsigned long long>, dim3(t1), dim3(kPartThreads), 0, stream, s, p, src, dst,
+      hipLaunchKernelGGL(k_msd_part1<unsigned long long>, dim3(t1), dim3(kPart1Threads), 0, stream, s, p, src, dst,
                          cur1, k64);
-      const unsigned t2 = unsigned(s.records / kPartTile) + (1u << p.b1);
-      hipLaunchKernelGGL(k_msd_part2, dim3(t2), dim3(kPartThreads), 0, stream, p, k64, off, cur2, k32);
+      const unsigned t2 = unsigned(s.records / kPart2Tile) + (1u << p.b1);
+      hipLaunchKernelGGL(k_msd_part2, dim3(t2), dim3(kPart2Threads), 0, stream, p, k64, off, cur2, k32);
     } else {
-      hipLaunchKernelGGL(k_msd_part1<unsigned>, dim3(t1), dim3(kPartThreads), 0, stream, s, p, src, dst, cur1, k32);
+      hipLaunchKernelGGL(k_msd_part1<unsigned>, dim3(t1), dim3(kPart1Threads), 0, stream, s, p, src, dst, cur1, k32);
     }
     sort_class<256>(0, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
     sort_class<512>(1, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
     sort_class<1024>(2, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
     HIP_TRY(hipGetLastError());
-    MsdCounts h{};
-    h.crowded = L;  // up to kChunk records nothing but this can be left over
+    hipLaunchKernelGGL((k_leaf_sort<1024, kLeafItems>), dim3(std::min(L, unsigned(c.cus) * 2)), dim3(1024), 0, stream,
+                       p, s.dedup, crowded, &mc->crowded[0], off, k32, tile_cnt);
+    HIP_TRY(hipGetLastError());
     if (s.records > kChunk) {
-      HIP_TRY(hipMemcpyAsync(&h, mc, sizeof h, hipMemcpyDeviceToHost, stream));
-      HIP_TRY(hipStreamSynchronize(stream));
-    }
-    if (h.crowded)
-      hipLaunchKernelGGL((k_leaf_sort<1024, kLeafItems>), dim3(std::min(h.crowded, unsigned(c.cus) * 2)), dim3(1024), 0,
-                         stream, p, s.dedup, crowded, &mc->crowded, off, k32, tile_cnt);
-    if (h.chunks) {
-      // The number of merge passes follows from the largest leaf; the sorted
-      // chunks go where it leaves the result in k32.
-      unsigned *other = reinterpret_cast<unsigned *>(k64);
-      int passes = 0;
-      while (((unsigned long long)kChunk << passes) < h.max_size) ++passes;
-      hipLaunchKernelGGL(k_chunk_place, dim3(std::min((h.chunks + 255) / 256, 1024u)), dim3(256), 0, stream, mc, off,
-                         chunks);
-      unsigned *from = (passes & 1) ? other : k32, *to = (passes & 1) ? k32 : other;
-      hipLaunchKernelGGL((k_chunk_sort<1024, kLeafItems>), dim3(std::min(h.chunks, unsigned(c.cus) * 2)), dim3(1024),
-                         0, stream, p, chunks, mc, k32, from);
-      for (int i = 0; i < passes; ++i) {
-        hipLaunchKernelGGL(k_leaf_merge, dim3(h.chunks, kChunk / kMergeTile), dim3(kMergeThreads), 0, stream, chunks,
-                           from, to, (unsigned long long)kChunk << i, s.dedup && i == passes - 1 ? tile_cnt : nullptr);
-        std::swap(from, to);
+      // The copy was queued before the partition passes, so the device is
+      // still busy with them when the host has it.
+      HIP_TRY(hipEventSynchronize(c.e_counts));
+      const MsdCounts h = c.host->counts;
+      if (h.chunks) {
+        // The number of merge passes follows from the largest leaf; the
+        // sorted chunks go where it leaves the result in k32.
+        unsigned *other = reinterpret_cast<unsigned *>(k64);
+        int passes = 0;
+        while (((unsigned long long)kChunk << passes) < h.max_size) ++passes;
+        hipLaunchKernelGGL(k_chunk_place, dim3(std::min((h.chunks + 255) / 256, 1024u)), dim3(256), 0, stream, mc, off,
+                           chunks);
+        unsigned *from = (passes & 1) ? other : k32, *to = (passes & 1) ? k32 : other;
+        unsigned *crowded_chunks = u(o_crowded2);
+        hipLaunchKernelGGL(k_leaf_bins<1024>, dim3(std::min(h.chunks, unsigned(c.cus))), dim3(1024), 0, stream, p, 0,
+                           nullptr, chunks, &mc->chunks, off, k32, from, nullptr, crowded_chunks, &mc->crowded[1]);
+        hipLaunchKernelGGL((k_chunk_sort<1024, kLeafItems>), dim3(std::min(h.chunks, unsigned(c.cus) * 2)),
+                           dim3(1024), 0, stream, p, chunks, crowded_chunks, &mc->crowded[1], k32, from);
+        for (int i = 0; i < passes; ++i) {
+          hipLaunchKernelGGL(k_leaf_merge, dim3(h.chunks, kChunk / kMergeTile), dim3(kMergeThreads), 0, stream, chunks,
+                             from, to, (unsigned long long)kChunk << i,
+                             s.dedup && i == passes - 1 ? tile_cnt : nullptr);
+          std::swap(from, to);
+        }
+        HIP_TRY(hipGetLastError());
       }
     }
     if (s.dedup)
@@ -561,9 +579,9 @@ int build_csr(BuildContext &c, long long n, long long ne, const int *src, const 
   hipLaunchKernelGGL(k_fill_gaps, dim3(c.cus * 4), dim3(kBuildBlock), 0, stream, gaps, ngaps, beg);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(c.e1, stream));
-  long long m = 0;
-  HIP_TRY(hipMemcpyAsync(&m, beg + n, 8, hipMemcpyDeviceToHost, stream));
+  HIP_TRY(hipMemcpyAsync(&c.host->m, beg + n, 8, hipMemcpyDeviceToHost, stream));
   HIP_TRY(hipStreamSynchronize(stream));
+  const long long m = c.host->m;
   *m_out = m;
   if (st) {
     std::memset(st, 0, sizeof *st);

@@ -15,24 +15,29 @@
 //                 keys -> 32-bit leaf keys by the next b2; one pass when
 //                 b <= 8
 //   k_leaf_bins   a leaf of at most kChunk records sorted in LDS, in place
-//   k_leaf_sort   the same by radix passes, for leaves with crowded bins
-//   k_chunk_sort, k_leaf_merge   leaves above kChunk: sorted chunks, merged
+//   k_leaf_sort, k_chunk_sort   the same by radix passes, where bins are crowded
+//   k_leaf_merge  leaves above kChunk: their sorted chunks merged
 //   k_scan, k_emit  duplicates dropped, columns and offsets out
 //
 // The sorts also count the records each emission tile keeps (the duplicates
 // are seen there), so emission reads the keys once.
 //
 // Bound: passes over the records. 134 M records (R-MAT 22 tuples, both
-// directions): 3.1 ms a call, against 7.0 ms for the six-pass
+// directions): 2.5 ms a call, against 7.0 ms for the six-pass
 // least-significant-digit sort of 45-bit keys that the other forms take.
 #pragma once
 
 namespace ent {
 namespace {
 
-constexpr int kPartThreads = 512;
-constexpr int kPartItems = 16;
-constexpr int kPartTile = kPartThreads * kPartItems;  // records staged per tile (64 KiB of keys)
+// Threads and records per thread of the partition passes (a tile of keys
+// staged in LDS each). R-MAT 22, 134 M records: the first pass takes 400 us
+// with 16,384 records a tile, 490 with 8,192 and 680 with 4,096 (its 256
+// buckets get longer runs); the second, to 128 leaves a bucket, 450 us with
+// 4,096 (four blocks fit a CU) and 570 with 8,192.
+constexpr int kPart1Threads = 1024, kPart1Items = 16;
+constexpr int kPart2Threads = 512, kPart2Items = 8;
+constexpr int kPart2Tile = kPart2Threads * kPart2Items;
 constexpr int kMaxFan = 256;                          // buckets of one partition pass
 constexpr int kHistBits = 15;                         // leaf counters one block holds (128 KiB of LDS)
 constexpr int kMaxLeafBits = 16;
@@ -66,7 +71,7 @@ struct Chunk {
 // Counters the reduce pass leaves for the host and the later kernels.
 struct MsdCounts {
   unsigned leaves[kLeafClasses];  // leaves by sort class
-  unsigned crowded;               // leaves left to k_leaf_sort
+  unsigned crowded[2];            // leaves, chunks left to the radix sort
   unsigned chunks;                // chunks of the leaves above kChunk
   unsigned max_size;              // largest leaf
 };
@@ -188,24 +193,26 @@ __global__ __launch_bounds__(256) void k_chunk_place(const MsdCounts *mc, const 
 }
 
 // Exclusive sums of cnt[0 .. n) into off[0 .. n] (off[n] = total), by one
-// block: n is at most some ten thousand per step of 32 entries a thread. With
-// cur1, also the partition cursors: cur2 = off, cur1[q] = off[q << b2].
+// block of 16 wavefronts with kScanItems coalesced rows of 64 entries each in
+// flight (32,768 entries a step; n is at most some 100,000 at the benchmark
+// sizes). With cur1, also the partition cursors: cur2 = off,
+// cur1[q] = off[q << b2].
 __global__ __launch_bounds__(kScanThreads) void k_scan(const unsigned *cnt, unsigned *off, unsigned n, unsigned *cur1,
                                                        unsigned *cur2, int b2) {
   __shared__ unsigned part[kScanThreads / kWave];
   const int wid = threadIdx.x / kWave, lane = lane_id();
   unsigned run = 0;
   for (unsigned base = 0; base < n; base += kScanThreads * kScanItems) {
-    const unsigned per = min(unsigned(kScanItems), (n - base + kScanThreads - 1) / kScanThreads);
-    const unsigned i0 = base + threadIdx.x * per;
+    const unsigned i0 = base + unsigned(wid) * kWave * kScanItems + lane;
     unsigned x[kScanItems], t = 0;
 #pragma unroll
-    for (unsigned j = 0; j < unsigned(kScanItems); ++j) {
-      x[j] = j < per && i0 + j < n ? cnt[i0 + j] : 0u;
-      t += x[j];
+    for (int j = 0; j < kScanItems; ++j) x[j] = i0 + j * kWave < n ? cnt[i0 + j * kWave] : 0u;
+#pragma unroll
+    for (int j = 0; j < kScanItems; ++j) {  // x[j] becomes its inclusive sum within the wavefront's entries
+      x[j] = t + unsigned(wave_incl_scan(int(x[j])));
+      t = unsigned(wave_read(int(x[j]), kWave - 1));
     }
-    const unsigned incl = unsigned(wave_incl_scan(int(t)));
-    if (lane == kWave - 1) part[wid] = incl;
+    if (lane == 0) part[wid] = t;
     __syncthreads();
     unsigned before = run, all = 0;
 #pragma unroll
@@ -214,18 +221,19 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(const unsigned *cnt, unsi
       if (k < wid) before += y;
       all += y;
     }
-    unsigned e = before + incl - t;
 #pragma unroll
-    for (unsigned j = 0; j < unsigned(kScanItems); ++j) {
-      const unsigned i = i0 + j;
-      if (j < per && i < n) {
+    for (int j = 0; j < kScanItems; ++j) {
+      const unsigned i = i0 + j * kWave;
+      unsigned e = unsigned(__shfl_up(int(x[j]), 1));
+      if (lane == 0) e = j ? unsigned(wave_read(int(x[j ? j - 1 : 0]), kWave - 1)) : 0u;
+      e += before;
+      if (i < n) {
         off[i] = e;
         if (cur1) {
           cur2[i] = e;
           if ((i & ((1u << b2) - 1)) == 0) cur1[i >> b2] = e;
         }
       }
-      e += x[j];
     }
     run += all;
     __syncthreads();
@@ -236,23 +244,23 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(const unsigned *cnt, unsi
 // One staged tile of a partition pass: item(j, key) gives the thread's j-th
 // record (false: none), key -> bucket (key >> shift) & (fan - 1), out[...] =
 // Out(key & mask). A bucket's records of the tile leave LDS as one run.
-template <class Out>
+template <int T, int I>
 struct PartSmem {
-  unsigned long long stage[kPartTile];
+  unsigned long long stage[T * I];
   unsigned cnt[kMaxFan], loc[kMaxFan], gb[kMaxFan];
   unsigned part[kMaxFan / kWave];
 };
 
-template <class Out, class Item>
-__device__ __forceinline__ void part_tile(PartSmem<Out> &sm, int shift, int fan, unsigned long long mask,
+template <int T, int I, class Out, class Item>
+__device__ __forceinline__ void part_tile(PartSmem<T, I> &sm, int shift, int fan, unsigned long long mask,
                                           unsigned *cursor, Out *out, Item item) {
   const int t = threadIdx.x;
-  for (int k = t; k < kMaxFan; k += kPartThreads) sm.cnt[k] = 0;
+  for (int k = t; k < kMaxFan; k += T) sm.cnt[k] = 0;
   __syncthreads();
-  unsigned long long key[kPartItems];
-  int rank[kPartItems];
+  unsigned long long key[I];
+  int rank[I];
 #pragma unroll
-  for (int j = 0; j < kPartItems; ++j) {
+  for (int j = 0; j < I; ++j) {
     const bool in = item(j, key[j]);
     rank[j] = in ? int(atomicAdd(&sm.cnt[(key[j] >> shift) & (fan - 1)], 1u)) : -1;
   }
@@ -272,13 +280,13 @@ __device__ __forceinline__ void part_tile(PartSmem<Out> &sm, int shift, int fan,
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kPartItems; ++j)
+  for (int j = 0; j < I; ++j)
     if (rank[j] >= 0) sm.stage[sm.loc[(key[j] >> shift) & (fan - 1)] + unsigned(rank[j])] = key[j];
   unsigned total = 0;
 #pragma unroll
   for (int k = 0; k < kMaxFan / kWave; ++k) total += sm.part[k];
   __syncthreads();
-  for (unsigned i = t; i < total; i += kPartThreads) {
+  for (unsigned i = t; i < total; i += T) {
     const unsigned long long k = sm.stage[i];
     const unsigned d = unsigned(k >> shift) & unsigned(fan - 1);
     out[sm.gb[d] + (i - sm.loc[d])] = Out(k & mask);
@@ -287,21 +295,21 @@ __device__ __forceinline__ void part_tile(PartSmem<Out> &sm, int shift, int fan,
 
 // First pass: tuples to buckets of the first b1 key bits.
 template <class Out>
-__global__ __launch_bounds__(kPartThreads) void k_msd_part1(BuildShape s, MsdPlan p, const int *src, const int *dst,
+__global__ __launch_bounds__(kPart1Threads) void k_msd_part1(BuildShape s, MsdPlan p, const int *src, const int *dst,
                                                             unsigned *cursor, Out *out) {
-  __shared__ PartSmem<Out> sm;
-  const int per = s.rev ? kPartItems / 2 : kPartItems;
-  const long long t0 = (long long)blockIdx.x * per * kPartThreads + threadIdx.x;
-  unsigned u[kPartItems], v[kPartItems];
+  __shared__ PartSmem<kPart1Threads, kPart1Items> sm;
+  const int per = s.rev ? kPart1Items / 2 : kPart1Items;
+  const long long t0 = (long long)blockIdx.x * per * kPart1Threads + threadIdx.x;
+  unsigned u[kPart1Items], v[kPart1Items];
 #pragma unroll
-  for (int j = 0; j < kPartItems; ++j) {
-    const long long i = t0 + (long long)j * kPartThreads;
+  for (int j = 0; j < kPart1Items; ++j) {
+    const long long i = t0 + (long long)j * kPart1Threads;
     const bool in = j < per && i < s.ne;
     u[j] = in ? unsigned(src[i]) : ~0u;
     v[j] = in ? unsigned(dst[i]) : ~0u;
   }
   const unsigned long long mask = sizeof(Out) == 8 ? ~0ull : (1ull << p.rem) - 1;
-  part_tile<Out>(sm, 2 * p.cb - p.b1, 1 << p.b1, mask, cursor, out, [&](int j, unsigned long long &key) {
+  part_tile<kPart1Threads, kPart1Items, Out>(sm, 2 * p.cb - p.b1, 1 << p.b1, mask, cursor, out, [&](int j, unsigned long long &key) {
     // With the reverse entries, item 2i is (u, v) and item 2i + 1 is (v, u).
     const bool back = s.rev && (j & 1);
     const unsigned a = s.rev ? u[j / 2] : u[j], c = s.rev ? v[j / 2] : v[j];
@@ -311,15 +319,15 @@ __global__ __launch_bounds__(kPartThreads) void k_msd_part1(BuildShape s, MsdPla
 }
 
 // Second pass: a tile of one first-pass bucket to its leaves.
-__global__ __launch_bounds__(kPartThreads) void k_msd_part2(MsdPlan p, const unsigned long long *in,
+__global__ __launch_bounds__(kPart2Threads) void k_msd_part2(MsdPlan p, const unsigned long long *in,
                                                             const unsigned *off, unsigned *cursor, unsigned *out) {
-  __shared__ PartSmem<unsigned> sm;
+  __shared__ PartSmem<kPart2Threads, kPart2Items> sm;
   __shared__ unsigned first[kMaxFan + 1];
   __shared__ int bucket;
   const int t = threadIdx.x, fan1 = 1 << p.b1;
   unsigned c = 0, incl = 0;
   if (t < kMaxFan) {
-    if (t < fan1) c = (off[(t + 1) << p.b2] - off[t << p.b2] + kPartTile - 1) / kPartTile;
+    if (t < fan1) c = (off[(t + 1) << p.b2] - off[t << p.b2] + kPart2Tile - 1) / kPart2Tile;
     incl = unsigned(wave_incl_scan(int(c)));
     if (lane_id() == kWave - 1) sm.part[t / kWave] = incl;
   }
@@ -335,11 +343,11 @@ __global__ __launch_bounds__(kPartThreads) void k_msd_part2(MsdPlan p, const uns
   const int q = bucket;
   if (q < 0) return;  // past the last tile
   const unsigned e = off[(q + 1) << p.b2];
-  const unsigned s0 = off[q << p.b2] + (blockIdx.x - first[q]) * kPartTile;
+  const unsigned s0 = off[q << p.b2] + (blockIdx.x - first[q]) * kPart2Tile;
   __syncthreads();  // sm.part is written again
-  part_tile<unsigned>(sm, 2 * p.cb - p.b, 1 << p.b2, (1ull << p.rem) - 1, cursor + ((long long)q << p.b2), out,
+  part_tile<kPart2Threads, kPart2Items, unsigned>(sm, 2 * p.cb - p.b, 1 << p.b2, (1ull << p.rem) - 1, cursor + ((long long)q << p.b2), out,
                       [&](int j, unsigned long long &key) {
-                        const unsigned i = s0 + unsigned(j) * kPartThreads + unsigned(t);
+                        const unsigned i = s0 + unsigned(j) * kPart2Threads + unsigned(t);
                         const bool ok = i < e;
                         key = ok ? in[i] : 0ull;
                         return ok;
@@ -377,16 +385,20 @@ template <int T>
 struct BinSmem {
   unsigned exch[T * kLeafItems];
   uint4 bins[T * kLeafItems / 8 + 1];  // 16-bit counters, then 16-bit starts, in pairs
-  unsigned gcnt[kGroups], gstart[kGroups];
+  unsigned group[kGroups];  // record counts, then first bin | count << 16
   unsigned part[T / kWave];
   unsigned tcnt[kLeafTiles];
   int crowded;
 };
 
+// Work: the leaves of list (off[leaf] on, sorted in place), or, with chunks,
+// the chunks themselves from src to dst. What is crowded is listed by leaf or
+// chunk number.
 template <int T>
-__global__ __launch_bounds__(T) void k_leaf_bins(MsdPlan p, int dedup, const unsigned *list, const unsigned *nlist,
-                                                 const unsigned *off, unsigned *keys, unsigned *tile_cnt,
-                                                 unsigned *crowded, unsigned *ncrowded) {
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(6))) void k_leaf_bins(MsdPlan p, int dedup, const unsigned *list, const Chunk *chunks,
+                                                 const unsigned *nlist, const unsigned *off, const unsigned *src,
+                                                 unsigned *dst, unsigned *tile_cnt, unsigned *crowded,
+                                                 unsigned *ncrowded) {
   __shared__ BinSmem<T> sm;
   const int t = threadIdx.x, wid = t / kWave, lane = lane_id();
   const unsigned n = *nlist;
@@ -395,26 +407,27 @@ __global__ __launch_bounds__(T) void k_leaf_bins(MsdPlan p, int dedup, const uns
   const int low = max(p.rem - 8, 0);                   // key bits below the group
   const int up = low ? 32 - low : 0;                   // ... moved to the top of a word
   for (unsigned li = blockIdx.x; li < n; li += gridDim.x) {
-    const unsigned leaf = list[li], first = off[leaf];
-    const int size = int(off[leaf + 1] - first);
+    const unsigned item = chunks ? li : list[li];
+    const unsigned first = chunks ? chunks[li].start : off[item];
+    const int size = chunks ? int(chunks[li].size) : int(off[item + 1] - first);
     unsigned key[kLeafItems];
 #pragma unroll
     for (int j = 0; j < kLeafItems; ++j) {
       const int i = j * T + t;
-      key[j] = i < size ? keys[first + unsigned(i)] : 0u;
+      key[j] = i < size ? src[first + unsigned(i)] : 0u;
     }
-    for (int k = t; k < kGroups; k += T) sm.gcnt[k] = 0;
+    for (int k = t; k < kGroups; k += T) sm.group[k] = 0;
     for (int k = t; k < T * kLeafItems / 8 + 1; k += T) sm.bins[k] = make_uint4(0u, 0u, 0u, 0u);
     if (t < kLeafTiles) sm.tcnt[t] = 0;
     if (t == 0) sm.crowded = 0;
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kLeafItems; ++j)
-      if (j * T + t < size) atomicAdd(&sm.gcnt[key[j] >> low], 1u);
+      if (j * T + t < size) atomicAdd(&sm.group[key[j] >> low], 1u);
     __syncthreads();
     unsigned c = 0, incl = 0;
     if (t < kGroups) {
-      c = sm.gcnt[t];
+      c = sm.group[t];
       incl = unsigned(wave_incl_scan(int(c)));
       if (lane == kWave - 1) sm.part[wid] = incl;
     }
@@ -422,12 +435,12 @@ __global__ __launch_bounds__(T) void k_leaf_bins(MsdPlan p, int dedup, const uns
     if (t < kGroups) {
       unsigned before = incl - c;
       for (int k = 0; k < wid; ++k) before += sm.part[k];
-      sm.gstart[t] = before;
+      sm.group[t] = before | (c << 16);
     }
     __syncthreads();
     auto bin_of = [&](unsigned k) {
-      const unsigned g = k >> low;
-      return sm.gstart[g] + (up ? __umulhi(k << up, sm.gcnt[g]) : 0u);
+      const unsigned g = sm.group[k >> low];
+      return (g & 0xFFFFu) + (up ? __umulhi(k << up, g >> 16) : 0u);
     };
     unsigned bin[kLeafItems];  // bin | rank among its records << 16
     bool over = false;
@@ -444,7 +457,7 @@ __global__ __launch_bounds__(T) void k_leaf_bins(MsdPlan p, int dedup, const uns
     if (over) sm.crowded = 1;
     __syncthreads();
     if (sm.crowded) {  // the whole block
-      if (t == 0) crowded[atomicAdd(ncrowded, 1u)] = leaf;
+      if (t == 0) crowded[atomicAdd(ncrowded, 1u)] = item;
       __syncthreads();
       continue;
     }
@@ -493,7 +506,7 @@ __global__ __launch_bounds__(T) void k_leaf_bins(MsdPlan p, int dedup, const uns
           at += (y < k || eq) ? 1 : 0;
         }
         pos = first + unsigned(at);
-        keys[pos] = k;
+        dst[pos] = k;
         kept = !dup;
       }
       if (dedup) count_kept(sm.tcnt, tile0, pos, kept);
@@ -624,12 +637,12 @@ __global__ __launch_bounds__(T) void k_leaf_sort(MsdPlan p, int dedup, const uns
 }
 
 template <int T, int ITEMS>
-__global__ __launch_bounds__(T) void k_chunk_sort(MsdPlan p, const Chunk *chunks, const MsdCounts *mc,
-                                                  const unsigned *src, unsigned *dst) {
+__global__ __launch_bounds__(T) void k_chunk_sort(MsdPlan p, const Chunk *chunks, const unsigned *list,
+                                                  const unsigned *nlist, const unsigned *src, unsigned *dst) {
   __shared__ LeafSmem<T, ITEMS> sm;
-  const unsigned n = mc->chunks;
+  const unsigned n = *nlist;
   for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
-    const Chunk c = chunks[i];
+    const Chunk c = chunks[list[i]];
     leaf_sort<T, ITEMS>(sm, src, dst, c.start, int(c.size), p.rem, nullptr);
   }
 }
