@@ -49,6 +49,7 @@
 #include "ent_batch.h"
 #include "ent_bfs.h"
 #include "ent_common.h"
+#include "ent_deep.h"
 #include "ent_device.h"
 #include "ent_internal.h"
 
@@ -1439,6 +1440,29 @@ BKernels blevel_for(int W) {
   }
 }
 
+// Sources are placed at mask bits in descending order of root degree
+// (ties by vertex id), so each 64-source word holds roots whose frontiers
+// grow alike and the per-word direction can push the lagging words while it
+// pulls the others, whatever order the caller gave; the same set of roots
+// always gets the same words, and so the same per-word counts.
+// [0 .. k) are the roots by bit, [512 + p] the caller's index of bit p (its
+// output row).
+std::vector<int32_t> place_sources(const ent_graph *g, const int32_t *roots, int k) {
+  std::vector<int32_t> placed(2 * ENT_BATCH_MAX_SOURCES, 0);
+  std::vector<int> order(static_cast<size_t>(k));
+  for (int s = 0; s < k; ++s) order[size_t(s)] = s;
+  const int32_t *deg = g->store->h_deg.data();
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    const int32_t dx = deg[size_t(roots[x])], dy = deg[size_t(roots[y])];
+    return dx != dy ? dx > dy : roots[x] < roots[y];
+  });
+  for (int p = 0; p < k; ++p) {
+    placed[size_t(p)] = roots[order[size_t(p)]];
+    placed[size_t(ENT_BATCH_MAX_SOURCES + p)] = order[size_t(p)];
+  }
+  return placed;
+}
+
 int run_batch(ent_graph *g, const int32_t *roots, int k, int *out, BState *fin) {
   BatchWorkspace *b = g->batch;
   // The search's own width: a workspace reserved for more sources holds the
@@ -1476,27 +1500,7 @@ int run_batch(ent_graph *g, const int32_t *roots, int k, int *out, BState *fin) 
   a.chunk_words = c.bu_chunk_words;
   a.out16 = ((reinterpret_cast<uintptr_t>(out) & 15) == 0 && (g->n & 3) == 0) ? 1 : 0;
   a.fused = (W <= 4 && c.batch_fused > 0) ? std::max<long long>(1, (long long)g->n / c.batch_fused) : 0;
-  // Sources are placed at mask bits in descending order of root degree
-  // (ties by vertex id), so each 64-source word holds roots whose frontiers
-  // grow alike and the per-word direction can push the lagging words while it
-  // pulls the others, whatever order the caller gave; the same set of roots
-  // always gets the same words, and so the same per-word counts.
-  // placed[0 .. k) are the roots by bit, placed[512 + p] the caller's index
-  // of bit p (its output row).
-  std::vector<int32_t> placed(2 * ENT_BATCH_MAX_SOURCES, 0);
-  {
-    std::vector<int> order(static_cast<size_t>(k));
-    for (int s = 0; s < k; ++s) order[size_t(s)] = s;
-    const int32_t *deg = g->store->h_deg.data();
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-      const int32_t dx = deg[size_t(roots[x])], dy = deg[size_t(roots[y])];
-      return dx != dy ? dx > dy : roots[x] < roots[y];
-    });
-    for (int p = 0; p < k; ++p) {
-      placed[size_t(p)] = roots[order[size_t(p)]];
-      placed[size_t(ENT_BATCH_MAX_SOURCES + p)] = order[size_t(p)];
-    }
-  }
+  const std::vector<int32_t> placed = place_sources(g, roots, k);
   a.rowmap = b->roots + ENT_BATCH_MAX_SOURCES;
   // Level-0 counts on the host: distinct (vertex, word) pairs of the roots.
   std::vector<std::pair<int32_t, int>> vw;
@@ -1616,6 +1620,61 @@ void batch_release(ent_graph *g) {
 
 namespace {
 
+// Whether a batch runs as k searches side by side, several levels per launch
+// (bfs_deep.hip), instead of on joint masks: no vertex of more than
+// kDeepMaxDegree edges, the default kind of configuration, and a graph of at
+// least kDeepBatchVertices (below it, uniform random graphs have no larger
+// degrees either, and those spread too fast). 4-neighbour grids, joint search
+// against this one: 2048 x 2048 with 4, 16 and 64 sources 76, 87 and 151
+// against 6.3, 11.1 and 35.8 ms; 1024 x 1024 with 512 sources 223 against 65;
+// 300 x 300 with 32 sources 14.4 against 1.2. Sources close together, whose
+// joint frontiers coincide, cost the joint search no less than 4 sources do.
+constexpr int64_t kDeepBatchVertices = 1 << 12;
+bool deep_batch_fits(const ent_graph *g, int k) {
+  const ent_bfs_config &c = g->cfg;
+  return g->store->max_deg <= kDeepMaxDegree && g->n >= kDeepBatchVertices &&
+         !g->deep_batch_off && c.launch != ENT_LAUNCH_PERSISTENT && c.batch_fused > 0 &&
+         (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN);
+}
+
+// *ran stays false when a frontier outgrew the queues (the rows are then
+// written again by the joint search).
+int run_deep_batch(ent_graph *g, const int32_t *roots, int k, int *out, bool want_bytes, BState *fin, bool *ran) {
+  int rc = deep_reserve(g, k, kDeepQueue);
+  if (rc) return rc;
+  // The roots by row, and the rows by 64-source group for the byte count.
+  int *droots = g->batch->roots;
+  std::vector<int32_t> placed = place_sources(g, roots, k);
+  std::copy(roots, roots + k, placed.begin());
+  HIP_TRY(hipMemcpyAsync(droots, placed.data(), sizeof(int32_t) * placed.size(), hipMemcpyHostToDevice, g->stream));
+  std::vector<DeepState> st(static_cast<size_t>(k));
+  if ((rc = deep_batch(g, droots, k, out, st.data()))) return rc;
+  for (const DeepState &s : st)
+    if (s.error) {
+      HIP_TRY(hipStreamSynchronize(g->stream));
+      return ENT_OK;
+    }
+  for (const DeepState &s : st) {
+    fin->levels = std::max(fin->levels, s.levels);
+    fin->phases = std::max(fin->phases, s.launches);
+    fin->total_vertices += s.total_nf;
+    fin->total_edges += s.total_mf;
+  }
+  fin->td_mask = fin->levels >= 64 ? ~0ull : (1ull << fin->levels) - 1;
+  fin->done = 1;
+  if (want_bytes) {
+    unsigned long long joint = 0;
+    if ((rc = deep_joint_bytes(g, out, droots + ENT_BATCH_MAX_SOURCES, k, &joint))) return rc;
+    fin->alg_bytes = joint + 4ull * 64ull * (unsigned long long)words_for(k) * (unsigned long long)g->n;
+  }
+  // The level history is not used; the count of times the search outgrew it
+  // follows from the levels all the same.
+  const int kept = g->batch->lcap;
+  if (fin->levels >= kept + 2) fin->flushes = 1 + (fin->levels - 2 - kept) / (kept + 2);
+  *ran = true;
+  return ENT_OK;
+}
+
 // Multi-source search with g->mu held. Any depth fits the reserved
 // workspace: the level ring flushes kept levels to the rows as it goes
 // (st->flushes).
@@ -1626,7 +1685,12 @@ int batch_locked(ent_graph *g, const int32_t *roots, int k, int32_t *depths_dev,
   if (rc) return rc;
   HIP_TRY(hipEventRecord(g->ev0, g->stream));
   BState fin{};
-  rc = run_batch(g, roots, k, depths_dev, &fin);
+  bool ran = false;
+  if (deep_batch_fits(g, k)) {
+    rc = run_deep_batch(g, roots, k, depths_dev, st != nullptr, &fin, &ran);
+    if (!rc && !ran) g->deep_batch_off = true;
+  }
+  if (!rc && !ran) rc = run_batch(g, roots, k, depths_dev, &fin);
   if (rc) {
     ignore(hipStreamSynchronize(g->stream));
     return rc;

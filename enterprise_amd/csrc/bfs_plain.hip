@@ -59,6 +59,7 @@
 
 #include "ent_bfs.h"
 #include "ent_common.h"
+#include "ent_deep.h"
 #include "ent_device.h"
 
 namespace ent {
@@ -1061,6 +1062,60 @@ __global__ __launch_bounds__(BS) void k_level(Args a, long long i) {
   run_phase<BS, HUB, COUNT>(a, sm, i);
 }
 
+// Hands the search over to the several-levels-per-launch form (bfs_deep.hip)
+// after launch i - 1, a queue-driven level: derives the state launch i would
+// have and, if that is another queue-driven level whose frontier does not
+// grow by more than half, makes it the first state of that form (else
+// DEEP_NOT_TAKEN). Writes nothing the ordinary launches read, so launch i can
+// still follow. One wavefront.
+__global__ __launch_bounds__(kWave) void k_deep_take(Args a, long long i, DeepCtl *d) {
+  __shared__ State S;
+  __shared__ unsigned long long tot[8];
+  const int lane = threadIdx.x;
+  const Control *c = a.ctl;
+  const unsigned *s32 = reinterpret_cast<const unsigned *>(&c->st[(i + 1) & 1]);
+  for (int w = lane; w < int(sizeof(State) / 4); w += kWave) reinterpret_cast<unsigned *>(&S)[w] = s32[w];
+  const unsigned long long *src = &c->cnt[(i + 2) % 3].v[lane * kStripeU64];
+  unsigned long long nf = src[K_NF], mf = src[K_MF], md = src[K_MAXDEG], ovf = src[K_QOVF];
+  const unsigned long long qn = src[K_QN];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    nf += __shfl_xor(nf, o);
+    mf += __shfl_xor(mf, o);
+    md = max(md, __shfl_xor(md, o));
+    ovf |= __shfl_xor(ovf, o);
+  }
+  const bool q_fit = __ballot(qn > (unsigned long long)a.qcap_s) == 0;
+  for (int k = lane; k < 3 * kDeepStripes * kDeepStripeU32; k += kWave) (&d->cnt[0][0])[k] = 0;
+  wave_sync();
+  DeepState D{};
+  if (lane == 0) {
+    tot[K_NF] = nf;
+    tot[K_MF] = mf;
+    tot[K_MAXDEG] = md;
+    tot[K_QOVF] = ovf;
+    const bool was_queue = !S.done && S.phase == PH_TDQ;
+    const unsigned long long prev = S.prev_nf;
+    next_state(a, S, tot, q_fit);
+    D.search = S.search;
+    if (was_queue && !S.done && S.phase == PH_TDQ && 2 * nf <= 3 * prev + 16) {
+      D.level = S.level;
+      D.par = S.level & 1;
+      D.total_nf = S.total_nf;
+      D.total_mf = S.total_mf;
+      D.td_levels = S.td_levels;
+    } else {
+      D.done = 1;
+      D.error = DEEP_NOT_TAKEN;
+      D.launches = 1;
+    }
+    for (int w = 0; w < kDeepHostWords; ++w)
+      reinterpret_cast<unsigned *>(&d->st[1])[w] = reinterpret_cast<const unsigned *>(&D)[w];
+  }
+  static_assert(kDeepStripes == kStripes && kStripes == kWave, "one queue stripe per lane");
+  d->st[1].qn[lane] = unsigned(min(qn, (unsigned long long)a.qcap_s));
+}
+
 // Whole search in one cooperative launch: launches 0, 1, 2, ... separated by
 // grid barriers. Stops on completion, or when a barrier wait exceeds ~4 s in
 // any block (the search is then marked failed). Every exit decision is taken
@@ -1116,6 +1171,7 @@ void release(ent_graph *g) {
   ignore(hipSetDevice(g->device));
   if (g->stream) ignore(hipStreamSynchronize(g->stream));  // launches queued behind a finished search
   batch_release(g);
+  deep_release(g);
   if (g->gexec) ignore(hipGraphExecDestroy(g->gexec));
   if (g->graph) ignore(hipGraphDestroy(g->graph));
   g->store.reset();
@@ -1443,6 +1499,60 @@ int wait_state(ent_graph *g, long long last, unsigned search, State *out) {
   }
 }
 
+// Whether searches on g may go on with several levels per launch: no vertex
+// of more than kDeepMaxDegree edges (a lane takes a whole row), and a
+// configuration that neither asks for bottom-up levels, for the reference's
+// switch, for a tally nor for no queues.
+bool deep_fits(const ent_graph *g) {
+  const ent_bfs_config &c = g->cfg;
+  return g->store->max_deg <= kDeepMaxDegree && !g->deep_off && !c.count_examined && g->hub_slots == 0 &&
+         c.queue_small >= 0 && (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN);
+}
+
+// First level at which a search is handed over. Earlier ones spread: a frontier
+// that still doubles at level 8 is refused by k_deep_take.
+constexpr int kDeepFirstLevel = 8;
+
+// After launch `next` - 1, a queue-driven level whose state is *fin: runs the
+// rest of the search with several levels per launch. *taken: 1 done, 0 the
+// frontier is not one for it, -1 it outgrew the queues there (start again).
+int run_deep(ent_graph *g, Args &a, long long next, State *fin, int *taken) {
+  *taken = 0;
+  int rc = deep_reserve(g, 1, 0);
+  if (rc) return rc;
+  DeepArgs d{};
+  d.off = a.off;
+  d.adj = a.adj;
+  d.depth = a.depth;
+  d.q[0] = a.qbuf[0];
+  d.q[1] = a.qbuf[1];
+  d.ctl = g->deep->ctl;
+  d.hmir = g->deep->h_mir_dev;
+  d.qcap_s = a.qcap_s;
+  d.nstripe = kDeepStripes;
+  int width = 0;
+  if ((rc = deep_rows(g, &width, &d.rows))) return rc;
+  void *args[] = {&a, &next, &d.ctl};
+  HIP_TRY(launch(reinterpret_cast<const void *>(&k_deep_take), 1, kWave, args, g->stream));
+  DeepState D;
+  rc = deep_run(g, d, width, 1, g->cus * 2, unsigned(fin->search), &D);
+  if (rc) return rc;
+  if (D.error == DEEP_NOT_TAKEN) return ENT_OK;
+  if (D.error) {
+    *taken = -1;
+    return ENT_OK;
+  }
+  *taken = 1;
+  fin->done = 1;
+  fin->levels = D.levels;
+  fin->td_levels = D.td_levels;
+  fin->total_nf = D.total_nf;
+  fin->total_mf = D.total_mf;
+  fin->phases += D.launches;
+  fin->t_end = D.t_end;
+  return ENT_OK;
+}
+
 // Runs one search; on success *fin holds the final state.
 int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
   const ent_bfs_config &cfg = g->cfg;
@@ -1467,6 +1577,19 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
     HIP_TRY(launch(ks.init, std::max(1, grid), bs, args, g->stream));
   }
   const long long max_launches = 2 * g->n + 16;
+  int deep_tries = deep_fits(g) ? 3 : 0;
+  int taken = 0;
+  auto try_deep = [&](long long next) -> int {
+    taken = 0;
+    if (deep_tries == 0 || fin->phase != PH_TDQ || fin->level < kDeepFirstLevel || next >= kSpinMaxLaunch) return ENT_OK;
+    const int e = run_deep(g, a, next, fin, &taken);
+    if (taken == 0) --deep_tries;
+    if (taken < 0) {
+      g->deep_off = true;
+      HIP_TRY(hipStreamSynchronize(g->stream));
+    }
+    return e;
+  };
   switch (cfg.launch) {
     case ENT_LAUNCH_PERSISTENT: {
       const int per_cu = persistent_blocks_per_cu(g, ks);
@@ -1505,11 +1628,15 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
         if (fin->done) break;
         if (i > max_launches) return set_error(ENT_EINTERNAL, "search did not finish in %lld launches", i);
         if (cfg.launch == ENT_LAUNCH_STREAM) {
+          if ((rc = try_deep(i))) return rc;
+          if (taken > 0) break;
+          if (taken < 0) return run_search(g, root, depth_dev, fin);
           k = follow;
           follow = std::min(2 * follow, 1024);
         }
       }
-      if (cfg.launch == ENT_LAUNCH_STREAM) g->expect_launches = int(std::min<int64_t>(fin->phases, 1 << 16));
+      if (cfg.launch == ENT_LAUNCH_STREAM)
+        g->expect_launches = int(std::min<int64_t>(taken > 0 ? i : fin->phases, 1 << 16));
       return ENT_OK;
     }
     case ENT_LAUNCH_GRAPH: {
@@ -1546,6 +1673,9 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
         if (rc) return rc;
         if (fin->done) break;
         if (i > max_launches) return set_error(ENT_EINTERNAL, "search did not finish in %lld launches", i);
+        if ((rc = try_deep(i + k))) return rc;
+        if (taken > 0) break;
+        if (taken < 0) return run_search(g, root, depth_dev, fin);
       }
       return ENT_OK;
     }
@@ -1725,6 +1855,7 @@ int upload_graph(const int64_t *beg_pos, const int32_t *adj, bool adj_on_device,
   for (int64_t v = 0; v < n; ++v) {
     const int64_t d = beg_pos[v + 1] - beg_pos[v];
     hdeg[size_t(v)] = int32_t(d);
+    g->store->max_deg = std::max(g->store->max_deg, int32_t(d));
     if (d > 0) {
       nz[size_t(v >> 6)] |= 1ull << (v & 63);
       ++active;

@@ -395,7 +395,7 @@ struct BinSmem {
 // the chunks themselves from src to dst. What is crowded is listed by leaf or
 // chunk number.
 template <int T>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(6))) void k_leaf_bins(MsdPlan p, int dedup, const unsigned *list, const Chunk *chunks,
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T < 1024 ? 6 : 4))) void k_leaf_bins(MsdPlan p, int dedup, const unsigned *list, const Chunk *chunks,
                                                  const unsigned *nlist, const unsigned *off, const unsigned *src,
                                                  unsigned *dst, unsigned *tile_cnt, unsigned *crowded,
                                                  unsigned *ncrowded) {

@@ -18,6 +18,7 @@ namespace ent {
 struct Args;
 struct Control;
 struct BatchWorkspace;
+struct DeepWorkspace;
 template <class T>
 inline void ignore(T) {}
 
@@ -29,11 +30,16 @@ struct GraphStore {
   int *adj = nullptr;                    // int32[m]
   unsigned long long *nzmask = nullptr;  // bit v: degree(v) > 0
   std::vector<int32_t> h_deg;            // host copy of degrees (for the static lists)
+  int32_t max_deg = 0;
+  std::mutex rows_mu;                    // guards rows, rows_width (ent_deep.h)
+  int *rows = nullptr;
+  int rows_width = -1;                   // -1: not built yet
   ~GraphStore() {
     if (hipSetDevice(device) != hipSuccess) return;
     ignore(hipFree(off));
     ignore(hipFree(adj));
     ignore(hipFree(nzmask));
+    ignore(hipFree(rows));
   }
 };
 // Reorders every adjacency row by descending floor(log2(neighbour degree)),
@@ -94,6 +100,10 @@ struct ent_graph {
   size_t dev_bytes = 0;
   int last_grid = 0;
   int expect_launches = 12;
+  ent::DeepWorkspace *deep = nullptr;    // several levels per launch (ent_deep.h)
+  // A search (batch) of that form outgrew its queues: the graph spreads too
+  // fast for it, and later ones start in the ordinary form.
+  bool deep_off = false, deep_batch_off = false;
   ent::BatchWorkspace *batch = nullptr;  // lazily allocated multi-source workspace
   std::mutex mu;
 };

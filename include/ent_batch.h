@@ -36,7 +36,7 @@ typedef struct ent_batch_stats {
                                rounded up to 1, 2, 4 or 8, whatever width the
                                workspace was reserved for */
   int32_t levels;           /* joint levels (max over sources of depth + 1) */
-  int32_t phases;           /* kernel phases run */
+  int32_t phases;           /* kernel phases run (side by side: launches) */
   int64_t reached_edges;    /* sum over sources of M_c(s) */
   int64_t reached_vertices; /* sum over sources of N_c(s) */
   int64_t alg_bytes;        /* per 64-source group g: sum over levels l and
@@ -49,9 +49,12 @@ typedef struct ent_batch_stats {
   uint64_t td_level_mask;   /* bit l: level l pushed (top-down) some of its
                                words; both bits set: the level split its words
                                by frontier size */
-  int32_t flushes;          /* passes that wrote the kept levels to the rows
-                               before the search ended (one per max_levels + 1
-                               levels beyond the first max_levels) */
+  int32_t flushes;          /* times the search outgrew the kept levels: one per
+                               max_levels + 2 levels beyond the first
+                               max_levels + 1, each a pass that writes the
+                               kept levels to the rows. Searches that run side
+                               by side (low degree) keep no levels and report
+                               the same count */
   int32_t pad;
 } ent_batch_stats;
 

@@ -107,7 +107,8 @@ typedef struct ent_stats {
   int32_t levels;           /* max depth + 1 */
   int32_t td_levels;        /* levels expanded top-down */
   int32_t bu_levels;        /* levels expanded bottom-up */
-  int32_t phases;           /* kernel phases run (levels + inspections) */
+  int32_t phases;           /* kernel phases run (levels + inspections; a
+                               launch that runs several levels counts once) */
   int64_t reached_vertices; /* N_c */
   int64_t reached_edges;    /* M_c = sum of degrees over reached vertices,
                                the reference's TEPS numerator

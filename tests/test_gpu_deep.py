@@ -1,0 +1,158 @@
+"""GPU parity of the several-levels-per-launch searches (bfs_deep.hip) on
+graphs of low degree and high diameter: depths and counts against the oracle
+at the edges of a launch's levels, on graphs with odd cycles (a block can
+reach a vertex by the longer way first), at the largest degree of the rule,
+and on graphs that spread too fast and fall back; batches of few sources
+against single-source rows and the joint search's counts."""
+import numpy as np
+import pytest
+
+import graphs
+from enterprise_amd import DeviceGraph, HostGraph
+from enterprise_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+LAUNCHES = {"stream": L.LAUNCH_STREAM, "graph": L.LAUNCH_GRAPH}
+COUNTS = ("levels", "reached_vertices", "reached_edges", "td_levels")
+
+
+def _say(msg):
+    print(msg, flush=True)
+
+
+def _random_grid(w, h, diagonals, seed):
+    """Grid with 10% of its edges deleted and random diagonals (odd cycles)."""
+    rng = np.random.default_rng(seed)
+    ids = np.arange(w * h).reshape(h, w)
+    e = np.concatenate([np.stack([ids[:, :-1].ravel(), ids[:, 1:].ravel()], 1),
+                        np.stack([ids[:-1].ravel(), ids[1:].ravel()], 1)])
+    e = e[rng.random(len(e)) > 0.1]
+    d = np.stack([ids[:-1, :-1].ravel(), ids[1:, 1:].ravel()], 1)
+    return graphs.edges_graph(w * h, np.concatenate([e, d[rng.random(len(d)) < diagonals]]))
+
+
+def _caterpillar(spine, legs):
+    """A path whose inner vertices have `legs` leaves each (degree legs + 2)."""
+    e = [(i, i + 1) for i in range(spine - 1)]
+    e += [(i, spine + i * legs + j) for i in range(spine) for j in range(legs)]
+    return graphs.edges_graph(spine + spine * legs, e)
+
+
+def _path_then_tree(length, branch, levels):
+    """A path into a complete tree of `branch` children per vertex: small
+    frontiers first, then ones that outgrow a block's queue in one launch."""
+    e, n, last = [(i, i + 1) for i in range(length - 1)], length, [length - 1]
+    for _ in range(levels):
+        nxt = []
+        for v in last:
+            for _ in range(branch):
+                e.append((v, n))
+                nxt.append(n)
+                n += 1
+        last = nxt
+    return graphs.edges_graph(n, e)
+
+
+CASES = {
+    # Paths that end just before, at and after a launch's last level.
+    **{f"path{n}": (lambda n=n: graphs.path(n)[0]) for n in (13, 20, 21, 22, 23, 28, 29, 30, 31, 37, 300)},
+    "cycle513": lambda: graphs.cycle(513)[0],
+    "disjoint": lambda: graphs.disjoint_paths(100, 77)[0],
+    "grid200x150": lambda: _random_grid(200, 150, 0.0, 1),
+    "diagonals200x150": lambda: _random_grid(200, 150, 0.3, 2),
+    "diagonals700x31": lambda: _random_grid(700, 31, 0.05, 3),
+    "degree16": lambda: _caterpillar(300, 14),
+    "degree17": lambda: _caterpillar(300, 15),  # beyond the rule
+    "spreads": lambda: _path_then_tree(40, 15, 4),
+    "bintree11": lambda: graphs.binary_tree(11)[0],
+}
+
+
+@pytest.mark.parametrize("launch", list(LAUNCHES))
+@pytest.mark.parametrize("name", list(CASES))
+def test_deep_search(oracle, name, launch):
+    g = CASES[name]()
+    rng = np.random.default_rng(5)
+    deg = np.diff(g.beg_pos)
+    roots = [int(np.flatnonzero(deg)[0])] + [int(r) for r in rng.choice(np.flatnonzero(deg), 4)]
+    with DeviceGraph(g) as dg:
+        for direction in (L.DIR_AUTO, L.DIR_TOPDOWN, L.DIR_AUTO):
+            dg.configure(launch=LAUNCHES[launch], direction=direction)
+            for r in roots:
+                want = oracle.bfs(g.beg_pos, g.adj, r)
+                _say(f"[gpu] deep {name} {launch} dir={direction} root={r}")
+                got, st = dg.bfs(r)
+                assert np.array_equal(got, want), (name, r)
+                edges, verts = oracle.report(g.beg_pos, want)
+                assert (st["reached_edges"], st["reached_vertices"]) == (edges, verts), st
+                assert st["levels"] == int(want.max()) + 1, st
+                if direction == L.DIR_TOPDOWN:
+                    assert st["td_levels"] == st["levels"], st
+        if name == "path300":  # the form did run: fewer launches than levels
+            _, st = dg.bfs(0)
+            assert st["levels"] == 300 and st["phases"] < 100, st
+
+
+def test_deep_directed_topdown(oracle):
+    """Forced top-down on a directed ring with chords and vertices that have
+    in-edges only."""
+    n = 900
+    beg, adj = [0], []
+    for v in range(n):
+        row = sorted({(v + 1) % 600, 600 + v % 300} | ({(v + 7) % 600} if v % 3 == 0 else set())) if v < 600 else []
+        adj += row
+        beg.append(len(adj))
+    g = HostGraph.from_arrays(np.array(beg, np.int64), np.array(adj, np.int32))
+    with DeviceGraph(g, keep_order=True) as dg:
+        dg.configure(direction=L.DIR_TOPDOWN)
+        for r in (0, 1, 599):
+            _say(f"[gpu] deep directed root={r}")
+            got, st = dg.bfs(r)
+            assert np.array_equal(got, oracle.bfs(g.beg_pos, g.adj, r))
+            assert st["phases"] < st["levels"]
+
+
+@pytest.mark.parametrize("k", [1, 2, 15, 16, 17, 32, 33, 64, 65, 200])
+def test_deep_batch(oracle, k):
+    """Batches on a 300 x 250 grid with odd cycles: every row equals the
+    oracle's, and the counts equal the joint search's on the same roots.
+    Unaligned output too."""
+    g = _random_grid(300, 250, 0.1, 7)
+    roots = g.pick_roots(k, 11)
+    if k > 2:
+        roots[1] = roots[0]  # a repeated root
+    want = np.stack([oracle.bfs(g.beg_pos, g.adj, int(r)) for r in roots])
+    with DeviceGraph(g) as dg:
+        dg.batch_reserve(k, 40)
+        _say(f"[gpu] deep batch k={k}")
+        out, st = dg.bfs_batch(roots)
+        assert np.array_equal(out, want)
+        dg.configure(batch_fused=0)  # the joint search, one level at a time
+        joint, sj = dg.bfs_batch(roots)
+        assert np.array_equal(joint, want)
+        for key in ("levels", "reached_vertices", "reached_edges", "alg_bytes", "words", "k", "flushes"):
+            assert st[key] == sj[key], (key, st, sj)
+        assert 8 * st["phases"] < sj["phases"]
+        dg.configure(batch_fused=8)
+        single, _ = dg.bfs(int(roots[0]))  # one mirror serves both forms
+        assert np.array_equal(single, want[0])
+        dev = dg.device_alloc(4 * k * g.n + 4)
+        try:
+            dg.bfs_batch_device(roots, dev + 4)
+            assert np.array_equal(dg.copy_depth(dev + 4, k * g.n).reshape(k, g.n), want)
+        finally:
+            dg.device_free(dev)
+
+
+def test_deep_batch_spreading_graph(oracle):
+    """A tree of 15 children per vertex: the frontiers outgrow the queues and
+    the batch runs as a joint search, the second time from the start."""
+    g = _path_then_tree(12000, 15, 4)
+    assert g.n >= 1 << 16
+    with DeviceGraph(g) as dg:
+        for roots in ([11990, 11999], [5, 12040]):
+            _say(f"[gpu] deep batch, spreading graph, roots {roots}")
+            out, st = dg.bfs_batch(np.array(roots, np.int32))
+            for i, r in enumerate(roots):
+                assert np.array_equal(out[i], oracle.bfs(g.beg_pos, g.adj, r))
