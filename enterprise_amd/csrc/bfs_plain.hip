@@ -1702,17 +1702,21 @@ int alloc_workspace(ent_graph *g) {
       (rc = dev_alloc(g, reinterpret_cast<void **>(&g->qbuf[0]), sizeof(int) * size_t(kStripes) * size_t(g->qcap_s))) ||
       (rc = dev_alloc(g, reinterpret_cast<void **>(&g->qbuf[1]), sizeof(int) * size_t(kStripes) * size_t(g->qcap_s))) ||
       (rc = dev_alloc(g, reinterpret_cast<void **>(&g->ctl), sizeof(Control))) ||
-      (rc = dev_alloc(g, &g->aux, 256)) ||
+      (rc = dev_alloc(g, &g->aux, kAuxBytes + kParentCountBytes)) ||
       (rc = dev_alloc(g, reinterpret_cast<void **>(&g->hashbuf), sizeof(unsigned long long) * kHashRows)))
     return rc;
   HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&g->h_ctl), sizeof(Control), hipHostMallocDefault));
   std::memset(g->h_ctl, 0, sizeof(Control));
   // Host-coherent: the level kernels write the tagged state mirror here.
   // Zeroed words carry search 0, which no search uses.
-  const size_t mir_bytes = sizeof(unsigned long long) * 2 * kHostStateWords;
+  const size_t mir_bytes = sizeof(unsigned long long) * (2 * kHostStateWords + 1);
   HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&g->h_mir), mir_bytes, hipHostMallocCoherent));
   std::memset(g->h_mir, 0, mir_bytes);
   HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void **>(&g->h_mir_dev), g->h_mir, 0));
+  g->h_bad = reinterpret_cast<unsigned *>(g->h_mir + 2 * kHostStateWords);
+  g->h_bad_dev = reinterpret_cast<unsigned *>(g->h_mir_dev + 2 * kHostStateWords);
+  // The parent call's result sits behind the mirror's words.
+  HIP_TRY(hipMemset(g->aux, 0, kAuxBytes + kParentCountBytes));
   HIP_TRY(hipMemset(g->ctl, 0, sizeof(Control)));
   HIP_TRY(hipDeviceSynchronize());
   return build_lists(g);

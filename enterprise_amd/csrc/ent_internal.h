@@ -70,7 +70,8 @@ struct ent_graph {
   int hub_min = 0;          // smallest degree in the table
   int lists_hub = -1, lists_hub_tw = -1;
   int *depth = nullptr;
-  void *aux = nullptr;     // 256 bytes of device scratch for host-side calls (counters)
+  void *aux = nullptr;     // kAuxBytes of device scratch for host-side calls (counters), then the parent counters
+  unsigned *h_bad = nullptr, *h_bad_dev = nullptr;  // pinned: vertices ent_bfs_parents_device found no parent for
   unsigned long long *hashbuf = nullptr;  // kHashRows row checksums (ent_device_row_hash)
   int *parent = nullptr;   // parent array of ent_bfs_parents (allocated on first use)
   int trace_launches = 0;  // launches recorded by the last counting search
@@ -120,6 +121,8 @@ namespace ent {
 
 // Rows one ent_device_row_hash launch sums (its per-handle buffer's length).
 constexpr int kHashRows = 512;
+// Bytes of ent_graph::aux, and of the parent counters behind them.
+constexpr size_t kAuxBytes = 256, kParentCountBytes = 16;
 
 // Frees the idle construction context of `device` (csr_build.hip).
 void build_give_back(int device);

@@ -67,3 +67,54 @@ def test_parents_reject_foreign_depths():
             dg.parents_device(a, buf, buf + 4 * g.n)  # and are one from a
         finally:
             dg.device_free(buf)
+
+
+def _first_parents(beg, adj, depth, root):
+    """The first neighbour one level closer of every reached vertex."""
+    rows = np.repeat(np.arange(beg.size - 1), np.diff(beg))
+    pos = np.where(depth[adj] == depth[rows] - 1, np.arange(adj.size), adj.size)
+    first = np.full(beg.size - 1, adj.size, np.int64)
+    np.minimum.at(first, rows, pos)
+    par = np.full(beg.size - 1, -1, np.int64)
+    hit = (first < adj.size) & (depth > 0)
+    par[hit] = adj[first[hit]]
+    par[root] = root
+    return par
+
+
+@pytest.mark.parametrize("pos", [0, 15, 16, 1039, 1040, 1041, 2063, 2064, 9000, 39997])
+def test_parents_long_rows(oracle, pos):
+    """Three hubs of 40,000 neighbours whose parent sits at row position pos
+    (and again two entries later), at the edges of the lane probe, the
+    wavefront's share and the pieces of the long-row kernel."""
+    hubs, leaves = 3, 39998
+    p1, p2, root = hubs, hubs + 1, hubs + 2
+    first_leaf = root + 1
+    n = first_leaf + hubs * leaves
+    rows = [[] for _ in range(n)]
+    for h in range(hubs):
+        mine = list(range(first_leaf + h * leaves, first_leaf + (h + 1) * leaves))
+        for v in mine:
+            rows[v] = [h]
+        q = min(pos + h, leaves)
+        rows[h] = mine[:q] + [p1] + mine[q:q + 1] + [p2] + mine[q + 1:]
+    rows[p1] = rows[p2] = list(range(hubs)) + [root]
+    rows[root] = [p1, p2]
+    beg = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64)
+    adj = np.concatenate([np.array(r, np.int32) for r in rows])
+    with DeviceGraph(beg_pos=beg, adj=adj, keep_order=True) as dg:
+        for r in (root, first_leaf):
+            print(f"[gpu] parents long rows pos={pos} root={r}", flush=True)
+            d, p, _ = dg.bfs_parents(r)
+            assert np.array_equal(d, oracle.bfs(beg, adj, r))
+            assert np.array_equal(p, _first_parents(beg, adj, d, r))
+        # A hub without a neighbour one level closer is counted and marked.
+        buf = dg.device_alloc(8 * n)
+        try:
+            dg.bfs_device(root, buf)
+            with pytest.raises(L.EntError) as e:
+                dg.parents_device(first_leaf, buf, buf + 4 * n)
+            assert e.value.code == L.ENT_EINVAL
+            dg.parents_device(root, buf, buf + 4 * n)
+        finally:
+            dg.device_free(buf)
