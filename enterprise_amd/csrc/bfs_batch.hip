@@ -1309,25 +1309,60 @@ __global__ void k_binit_src(BArgs a, const int *roots, BInit in) {
 }
 
 // Position-keyed checksum of each row (sum over i of mix(i, value), mod
-// 2^64). Block (r, c) sums chunk c of row r and adds it to out[r].
-__global__ void k_row_hash(const int *dev, long long cols, long long chunk, unsigned long long *out) {
-  const long long r = blockIdx.y;
+// 2^64). Block (c, r) sums chunk c of row r and adds it to out[r]. Four values
+// per lane and step, in one 16-byte load where the rows allow it (VEC: the
+// first row 16-byte aligned and cols a multiple of four). Bound: the two
+// 64-bit products a value takes (about 60 us for 64 rows of 2^20), as much as
+// the 268 MB of loads; XXX.
+__device__ __forceinline__ unsigned long long hash_mix(long long i, int value) {
+  unsigned long long z = ((unsigned long long)i << 32) ^ (unsigned int)value;
+  z += 0x9E3779B97F4A7C15ull;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void k_row_hash(const int *dev, long long cols, long long chunk,
+                                                  unsigned long long *out) {
+  const int *row = dev + (long long)blockIdx.y * cols;
   const long long c0 = (long long)blockIdx.x * chunk;
   const long long c1 = min(cols, c0 + chunk);
   unsigned long long h = 0;
-  for (long long i = c0 + threadIdx.x; i < c1; i += blockDim.x) {
-    unsigned long long z = ((unsigned long long)i << 32) ^ (unsigned int)dev[r * cols + i];
-    z += 0x9E3779B97F4A7C15ull;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    h += z ^ (z >> 31);
+  if (VEC) {
+    for (long long i = c0 + 4 * threadIdx.x; i < c1; i += 1024) {
+      const int4 x = *reinterpret_cast<const int4 *>(row + i);
+      h += hash_mix(i, x.x) + hash_mix(i + 1, x.y) + hash_mix(i + 2, x.z) + hash_mix(i + 3, x.w);
+    }
+  } else {
+    long long i = c0 + threadIdx.x;
+    for (; i + 768 < c1; i += 1024) {
+      const int x0 = row[i], x1 = row[i + 256], x2 = row[i + 512], x3 = row[i + 768];
+      h += hash_mix(i, x0) + hash_mix(i + 256, x1) + hash_mix(i + 512, x2) + hash_mix(i + 768, x3);
+    }
+    for (; i < c1; i += 256) h += hash_mix(i, row[i]);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
   __shared__ unsigned long long red[4];
   if (lane_id() == 0) red[threadIdx.x / kWave] = h;
   __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(&out[r], red[0] + red[1] + red[2] + red[3]);
+  if (threadIdx.x == 0) atomicAdd(&out[blockIdx.y], red[0] + red[1] + red[2] + red[3]);
+}
+
+constexpr long long kHashChunk = 1 << 14;  // values per block
+
+// Queues the checksums of `rows` rows (at most 65,535) into out, which is
+// zero.
+hipError_t queue_row_hash(const int *dev, long long rows, long long cols, unsigned long long *out, hipStream_t s) {
+  // Rows too long for the grid's first dimension take longer chunks.
+  long long chunk = kHashChunk;
+  while ((cols + chunk - 1) / chunk > (1 << 20)) chunk *= 2;
+  const dim3 grid(unsigned((cols + chunk - 1) / chunk), unsigned(rows));
+  const bool vec = (reinterpret_cast<uintptr_t>(dev) & 15) == 0 && (cols & 3) == 0;
+  if (vec) hipLaunchKernelGGL(k_row_hash<true>, grid, dim3(256), 0, s, dev, cols, chunk, out);
+  else hipLaunchKernelGGL(k_row_hash<false>, grid, dim3(256), 0, s, dev, cols, chunk, out);
+  return hipGetLastError();
 }
 
 // Scratch of ent_device_row_hash_noalloc: one checksum accumulator per row,
@@ -1825,15 +1860,11 @@ int ent_device_row_hash(ent_graph *g, const int32_t *dev, int64_t rows, int64_t 
   // The handle's own checksum buffer, kHashRows rows per launch: no
   // allocation, so calls on other handles' streams keep running meanwhile.
   unsigned long long *d = g->hashbuf;
-  long long chunk = 1 << 16;
-  const long long nchunks = (cols + chunk - 1) / chunk;
   for (int64_t r0 = 0; r0 < rows; r0 += kHashRows) {
     const int64_t nr = std::min<int64_t>(kHashRows, rows - r0);
     const int32_t *base = dev + r0 * cols;
-    void *args[] = {const_cast<int32_t **>(&base), &cols, &chunk, &d};
     HIP_TRY(hipMemsetAsync(d, 0, sizeof(unsigned long long) * size_t(nr), g->stream));
-    HIP_TRY(hipLaunchKernel(reinterpret_cast<const void *>(&k_row_hash), dim3(unsigned(nchunks), unsigned(nr)),
-                            dim3(256), args, 0, g->stream));
+    HIP_TRY(queue_row_hash(base, nr, cols, d, g->stream));
     HIP_TRY(hipMemcpyAsync(hashes_host + r0, d, sizeof(unsigned long long) * size_t(nr), hipMemcpyDeviceToHost,
                            g->stream));
     HIP_TRY(hipStreamSynchronize(g->stream));
@@ -1891,12 +1922,7 @@ extern "C" int ent_device_row_hash_noalloc(int32_t device, const int32_t *dev, i
   const long long nr = rows;
   hipLaunchKernelGGL(k_zero_u64, dim3(unsigned((nr + 255) / 256)), dim3(256), 0, 0, acc, nr);
   HIP_TRY(hipGetLastError());
-  long long chunk = 1 << 16;
-  const long long nchunks = (cols + chunk - 1) / chunk;
-  long long ncols = cols;
-  void *args[] = {const_cast<int32_t **>(&dev), &ncols, &chunk, &acc};
-  HIP_TRY(hipLaunchKernel(reinterpret_cast<const void *>(&k_row_hash), dim3(unsigned(nchunks), unsigned(nr)),
-                          dim3(256), args, 0, nullptr));
+  HIP_TRY(queue_row_hash(dev, nr, cols, acc, nullptr));
   HIP_TRY(hipMemcpy(hashes_host, acc, sizeof(unsigned long long) * size_t(nr), hipMemcpyDeviceToHost));
   return ENT_OK;
 }

@@ -475,3 +475,31 @@ def test_batch_root_order(oracle, rmat16):
             assert np.array_equal(ref[0], oracle.bfs(g.beg_pos, g.adj, int(roots[0])))
     finally:
         dg.set_config(base)
+
+
+@pytest.mark.parametrize("cols", [1, 3, 4, 5, 255, 256, 1023, 1024, 1028, 16383, 16384, 16385, 16388, 70001])
+def test_row_hash_widths(cols):
+    """Row checksums at the edges of a lane's step and a block's chunk, from
+    16-byte aligned rows and from ones that are not, with a graph handle and
+    without."""
+    from enterprise_amd import _lib
+    rows = 5
+    host = np.random.default_rng(cols).integers(-1, 1 << 30, rows * cols + 1).astype(np.int32)
+    g, _ = graphs.path(5)
+    with DeviceGraph(g) as dg:
+        ptr = dg.device_alloc(host.nbytes + 16)
+        try:
+            import ctypes as C
+            hip = C.CDLL("libamdhip64.so")
+            hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+            assert hip.hipMemcpy(ptr, host.ctypes.data, host.nbytes, 1) == 0
+            for off in (0, 1):
+                _say(f"[gpu] row hash cols={cols} offset={off}")
+                want = row_hash_host(host[off:off + rows * cols].reshape(rows, cols))
+                assert np.array_equal(dg.row_hash(ptr + 4 * off, rows, cols), want)
+                out = np.empty(rows, np.uint64)
+                _lib.check(_lib.lib().ent_device_row_hash_noalloc(0, C.c_void_p(ptr + 4 * off), rows, cols,
+                                                                  out.ctypes.data_as(C.POINTER(C.c_uint64))))
+                assert np.array_equal(out, want)
+        finally:
+            dg.device_free(ptr)
