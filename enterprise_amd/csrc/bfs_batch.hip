@@ -37,13 +37,14 @@
 //   OUTPUT replays the kept levels per 64-vertex segment in LDS and writes
 //          all k depth rows with 16-byte streaming stores (a flush: the same
 //          for the levels kept so far, in the middle of the search).
-// The pull runs in its own kernel, launched beside the others for the same
-// launch index, so its mask registers do not cap their occupancy; with
-// ENT_LAUNCH_PERSISTENT the whole search is one cooperative launch instead.
+// With eight words the pull runs in its own kernel, launched beside the others
+// for the same launch index, so its mask registers do not cap their occupancy;
+// with ENT_LAUNCH_PERSISTENT the whole search is one cooperative launch instead.
 #include <hip/hip_runtime.h>
 
 #include <chrono>
 #include <cstring>
+#include <thread>
 #include <vector>
 
 #include "ent_batch.h"
@@ -107,9 +108,15 @@ struct BState {
   // counted (a fused level does not sweep the vertices; the sum only falls,
   // so the last count bounds it from above).
   unsigned long long munf_last;
-  int pulled;  // some level of this search pulled
+  int search;  // the host's search number, carried from launch to launch
   int pad;
 };
+// The host mirror of a state: two slots (launch parity) of its words, each in
+// the low half of a 64-bit word whose high half is the tag of the launch that
+// wrote it, phases + search * kBTagMul. The host takes a slot only when all
+// its tags agree (the stores arrive in no fixed order).
+constexpr int kBStateWords = int(sizeof(BState) / 4);
+constexpr unsigned kBTagMul = 0x9E3779B1u;
 
 struct BControl {
   BState st[2];
@@ -149,6 +156,8 @@ struct BArgs {
   // W <= 4 only). When nonzero, every level also empties the ring slot two
   // levels ahead (see prep_word).
   long long fused;
+  unsigned long long *hmir;  // host mirror of the states
+  int search;
 };
 
 template <int W>
@@ -214,7 +223,10 @@ struct BSmem {
     } td;                              // top-down frontier staging
     int rows[ENT_BATCH_MAX_SOURCES];   // output: row of the source at each mask bit
   };
-  unsigned char d8[NW][kWave * 68];  // output staging: 64 lanes x 64 sources (+4 pad)
+  union {
+    unsigned char d8[NW][kWave * 68];           // output staging: 64 lanes x 64 sources (+4 pad)
+    unsigned long long part[BS / 32][32];       // prologue: partial counter sums
+  };
   unsigned long long c[C_COUNT];
   long long seg;  // output: the segment the block claimed
   BState S;
@@ -303,121 +315,142 @@ __device__ __forceinline__ void block_counts_flush(const BArgs &a, BSmem<BS> &sm
 
 // -- state -------------------------------------------------------------------
 
-__device__ BState next_bstate(const BArgs &a, const BState &p, const unsigned long long *tot, int W) {
-  BState s = p;
-  if (p.done) return s;
-  s.phases = p.phases + 1;
-  if (p.phase == BPH_TD) {  // pushed words settle in the pull phase, if any, else in APPLY
-    s.phase = p.pull_words ? BPH_BU : BPH_APPLY;
-    return s;
+// Updates s (the state after launch i - 1, in LDS) in place to the state of
+// launch i. tot holds the summed counts of launch i - 1.
+__device__ __forceinline__ void next_bstate(const BArgs &a, BState &s, const unsigned long long *tot, int W) {
+  if (s.done) return;
+  s.phases += 1;
+  const int phase = s.phase;
+  if (phase == BPH_TD) {  // pushed words settle in the pull phase, if any, else in APPLY
+    s.phase = s.pull_words ? BPH_BU : BPH_APPLY;
+    return;
   }
-  if (p.phase == BPH_OUTPUT) {
-    if (p.flush) {  // levels base .. flush_end - 1 are in the rows: resume
+  if (phase == BPH_OUTPUT) {
+    if (s.flush) {  // levels base .. flush_end - 1 are in the rows: resume
       s.flush = 0;
-      s.base = p.flush_end;
-      s.phase = p.resume;
-      return s;
+      s.base = s.flush_end;
+      s.phase = s.resume;
+      return;
     }
     s.total_edges = tot[C_EDGES];
     s.total_vertices = tot[C_VERTS];
     s.alg_bytes += 4ull * 64ull * (unsigned long long)W * (unsigned long long)a.n;
     s.done = 1;
-    return s;
+    return;
   }
-  const int L = p.level;  // -1 before level 0
-  if (L >= 0 && p.pull_words && L < 64) s.bu_mask |= 1ull << L;
-  if (L >= 0 && p.push_words && L < 64) s.td_mask |= 1ull << L;
+  const int L = s.level;  // -1 before level 0
+  const unsigned pulled = s.pull_words;
+  if (L >= 0 && pulled && L < 64) s.bu_mask |= 1ull << L;
+  if (L >= 0 && s.push_words && L < 64) s.td_mask |= 1ull << L;
   s.alg_bytes += tot[C_ALG];
   if (tot[C_JWORDS] == 0) {
     s.levels = L + 1;
     s.phase = BPH_OUTPUT;
-    return s;
+    return;
   }
-  for (int w = 0; w < 8; ++w) s.active[w] = w < W ? tot[C_ACTIVE + w] : 0ull;
   // A fused level counts no unfinished vertices: its successor steers with
   // the last count.
-  const unsigned long long mf = tot[C_MF], munf = p.phase == BPH_TDF ? p.munf_last : tot[C_MUNF];
+  const unsigned long long mf = tot[C_MF], munf = phase == BPH_TDF ? s.munf_last : tot[C_MUNF];
   s.munf_last = munf;
   // Direction per 64-source word: a word whose new frontier is large is
   // pulled, a word that lags is pushed, so a pull can stop once the large
   // words are covered instead of scanning every row for the lagging ones.
   unsigned pull = 0, live = 0;
-  for (int w = 0; w < W; ++w) {
-    if (!s.active[w]) continue;
+  for (int w = 0; w < 8; ++w) {
+    const unsigned long long act = w < W ? tot[C_ACTIVE + w] : 0ull;
+    s.active[w] = act;
+    if (!act) continue;
     live |= 1u << w;
     bool bu;
     switch (a.mode) {
       case ENT_DIR_TOPDOWN: bu = false; break;
       case ENT_DIR_BOTTOMUP: bu = true; break;
       case ENT_DIR_REFERENCE:  // the reference's one-way switch, for every word at once
-        bu = p.pull_words != 0 || (L + 1 >= 1 && 10ull * mf >= 3ull * (unsigned long long)a.m);
+        bu = pulled != 0 || (L + 1 >= 1 && 10ull * mf >= 3ull * (unsigned long long)a.m);
         break;
       default: bu = tot[C_MFW + w] * (unsigned long long)a.alpha > munf;
     }
     if (bu) pull |= 1u << w;
   }
+  const int slot = s.slot + 1;
   s.level = L + 1;
-  s.slot = p.slot + 1 == a.ring ? 0 : p.slot + 1;
+  s.slot = slot == a.ring ? 0 : slot;
   s.pull_words = pull;
   s.push_words = live & ~pull;
-  if (pull) s.pulled = 1;
-  s.phase = s.push_words ? BPH_TD : BPH_BU;
+  int next = (live & ~pull) ? BPH_TD : BPH_BU;
   // A small all-push frontier is pushed and settled in one launch.
-  if (pull == 0 && a.fused > 0 && mf <= (unsigned long long)a.fused) s.phase = BPH_TDF;
+  if (pull == 0 && a.fused > 0 && mf <= (unsigned long long)a.fused) next = BPH_TDF;
+  s.phase = next;
   // Level L' = s.level uses the slots of L' (its frontier), L' + 1 (its new
   // bits) and L' + 2 (cleared for the next push). The ring holds them beside
   // the levels base .. L' - 1 not yet in the rows while L' - base <= lcap;
   // beyond that, levels base .. L' (L' complete: it is the new frontier) are
   // flushed to the rows first.
-  if (s.level - s.base > a.lcap) {
-    s.resume = s.phase;
+  if (L + 1 - s.base > a.lcap) {
+    s.resume = next;
     s.phase = BPH_OUTPUT;
     s.flush = 1;
     s.flushes += 1;
-    s.flush_end = s.level + 1;
+    s.flush_end = L + 2;
   }
-  return s;
 }
 
+// Launch prologue: every thread sums (or ORs) one counter over a share of the
+// 64 stripes while the second wavefront fetches the previous state, thread 0
+// derives this launch's state from both in LDS; block 0 publishes it and
+// clears the counter slot of launch i + 1.
 template <int BS, int W>
 __device__ __forceinline__ void begin_blaunch(const BArgs &a, BSmem<BS> &sm, long long i, bool coherent = false) {
-  if (threadIdx.x < kWave) {
-    BControl *c = a.ctl;
-    const int lane = threadIdx.x;
-    const BCounters &pc = c->cnt[(i + 2) % 3];
-    // Totals of the 64 stripes: lane j sums (or ORs) counter j over the
-    // stripes with independent loads, so no cross-lane steps are needed.
-    __shared__ unsigned long long t[C_COUNT];
-    if (lane < C_COUNT) {
-      const bool is_or = lane >= C_ACTIVE && lane < C_ACTIVE + 8;
-      unsigned long long acc = 0;
-#pragma unroll 16
-      for (int st = 0; st < kBStripes; ++st) {
-        const unsigned long long *q = &pc.v[st * kBStripeU64 + lane];
-        const unsigned long long x = coherent ? ld_agent(q) : *q;
+  constexpr int kGroups = BS / 32, kEach = kBStripes / kGroups;
+  static_assert(C_COUNT <= 32 && kGroups * kEach == kBStripes, "a counter per thread of a group of 32");
+  constexpr int kWords = kBStateWords;
+  static_assert(kWords <= kWave && BS >= 2 * kWave, "one state word per lane");
+  __shared__ unsigned long long t[C_COUNT];
+  BControl *c = a.ctl;
+  const int col = threadIdx.x & 31, grp = threadIdx.x >> 5;
+  const bool is_or = col >= C_ACTIVE && col < C_ACTIVE + 8;
+  {
+    const unsigned long long *src = c->cnt[(i + 2) % 3].v + (long long)grp * kEach * kBStripeU64 + col;
+    unsigned long long acc = 0;
+    if (col < C_COUNT) {
+#pragma unroll
+      for (int st = 0; st < kEach; ++st) {
+        const unsigned long long x = coherent ? ld_agent(src + st * kBStripeU64) : src[st * kBStripeU64];
         acc = is_or ? (acc | x) : (acc + x);
       }
+    }
+    if (threadIdx.x >= kWave && threadIdx.x < kWave + kWords) {
+      const unsigned *s32 = reinterpret_cast<const unsigned *>(&c->st[(i + 1) & 1]) + (threadIdx.x - kWave);
+      reinterpret_cast<unsigned *>(&sm.S)[threadIdx.x - kWave] = coherent ? ld_agent(s32) : *s32;
+    }
+    sm.part[grp][col] = acc;
+  }
+  __syncthreads();
+  if (threadIdx.x < kWave) {
+    const int lane = threadIdx.x;
+    if (lane < C_COUNT) {
+      unsigned long long acc = 0;
+#pragma unroll
+      for (int k = 0; k < kGroups; ++k) acc = is_or ? (acc | sm.part[k][lane]) : (acc + sm.part[k][lane]);
       t[lane] = acc;
     }
     wave_sync();
-    if (lane == 0) {
-      BState prev;
-      if (coherent) {
-        const unsigned *s32 = reinterpret_cast<const unsigned *>(&c->st[(i + 1) & 1]);
-        unsigned *d32 = reinterpret_cast<unsigned *>(&prev);
-        for (int w = 0; w < int(sizeof(BState) / 4); ++w) d32[w] = ld_agent(s32 + w);
-      } else {
-        prev = c->st[(i + 1) & 1];
+    if (lane == 0) next_bstate(a, sm.S, t, W);
+    wave_sync();
+    if (blockIdx.x == 0) {
+      if (lane < kWords) {
+        const unsigned word = reinterpret_cast<const unsigned *>(&sm.S)[lane];
+        reinterpret_cast<unsigned *>(&c->st[i & 1])[lane] = word;
+        const unsigned tag = unsigned(sm.S.phases) + unsigned(sm.S.search) * kBTagMul;
+        a.hmir[(i & 1) * kWords + lane] = (static_cast<unsigned long long>(tag) << 32) | word;
       }
-      const BState S = next_bstate(a, prev, t, W);
-      sm.S = S;
-      if (blockIdx.x == 0) {
-        c->st[i & 1] = S;
-        c->lphase[i & 1] = S.done ? -1 : S.phase;
-      }
+      if (lane == 0) c->lphase[i & 1] = sm.S.done ? -1 : sm.S.phase;
     }
-    if (blockIdx.x == 0 && lane < C_COUNT)
-      for (int s = 0; s < kBStripes; ++s) c->cnt[(i + 1) % 3].v[s * kBStripeU64 + lane] = 0;
+  }
+  if (blockIdx.x == 0 && col < C_COUNT) {
+    unsigned long long *z = c->cnt[(i + 1) % 3].v + (long long)grp * kEach * kBStripeU64 + col;
+#pragma unroll
+    for (int st = 0; st < kEach; ++st) z[st * kBStripeU64] = 0;
   }
   block_counts_reset(sm);
   __syncthreads();
@@ -1142,23 +1175,22 @@ __device__ void boutput_phase(const BArgs &a, BSmem<BS> &sm, int lo, int hi, boo
   wave_counts<BS, W>(sm, 0, 0, 0, 0, none, edges, verts, word_sums_zero<W>());
 }
 
-// Launch i runs as two kernels queued back to back: the bottom-up phase has
-// its own kernel (its mask registers would otherwise cap the occupancy of
-// every phase), the other phases share one. Both derive the same state for
-// launch i; the one whose phase it is does the work. When the previous
-// search on the workspace never pulled (W <= 4), the host queues k_blevel
-// alone, with pulls = 1, and a pull runs there.
+// Launch i. With eight mask words it runs as two kernels queued back to back:
+// the bottom-up phase has its own (its mask registers would otherwise cap the
+// occupancy of every phase), the other phases share one. Both derive the same
+// state for launch i; the one whose phase it is does the work. Up to four
+// words the pull costs the shared kernel no registers, and the second launch
+// (4.4 us when it is not its phase, the first 8.7 when it is) is saved:
+// R-MAT 20, 64 sources 858 -> 806 us.
 template <int BS, int W>
-__global__ __launch_bounds__(BS) void k_blevel(BArgs a, long long i, int pulls) {
+__global__ __launch_bounds__(BS) void k_blevel(BArgs a, long long i) {
   __shared__ BSmem<BS> sm;
   begin_blaunch<BS, W>(a, sm, i);
   const BState &S = sm.S;
   if (S.done) return;
   const int slot = int(i % 3);
   if (S.phase == BPH_BU) {
-    // With pulls set (W <= 4 only) the host queued no k_blevel_bu for this
-    // launch: the pull runs here, at this kernel's occupancy.
-    if (W <= 4 && pulls) {
+    if (W <= 4) {
       bbu_phase<BS, W>(a, sm, S.level);
       block_counts_flush(a, sm, slot);
     }
@@ -1275,6 +1307,7 @@ __global__ void k_binit_zero(BArgs a, const int *roots) {
     S.level = -1;
     S.slot = a.ring - 1;
     S.phase = BPH_APPLY;
+    S.search = a.search;
     a.ctl->st[0] = S;
     a.ctl->st[1] = S;
   }
@@ -1390,12 +1423,10 @@ struct BatchWorkspace {
   BControl *ctl = nullptr;
   BControl *h_ctl = nullptr;
   size_t bytes = 0;
+  unsigned long long *h_mir = nullptr, *h_mir_dev = nullptr;  // host-coherent state mirror
   int expect_launches = 16;
   int *rows = nullptr;     // device rows of ent_bfs_batch (grown on demand)
   size_t rows_bytes = 0;
-  // The last search pulled at some level: queue k_blevel_bu beside every
-  // launch (otherwise, with W <= 4, k_blevel runs a pull itself).
-  bool pulled_last = true;
   // Every nonzero mask in the lv ring belongs to a vertex in its slot's
   // bitmap (what fused levels rely on). Holds after the rings are zeroed and
   // after a search that completed with fused levels allowed; a search that
@@ -1451,6 +1482,13 @@ int reserve(ent_graph *g, int k, int lcap) {
     batch_release(g);
     return set_error(ENT_ENOMEM, "pinned host memory");
   }
+  const size_t mir_bytes = sizeof(unsigned long long) * 2 * kBStateWords;
+  if (hipHostMalloc(reinterpret_cast<void **>(&b->h_mir), mir_bytes, hipHostMallocCoherent) != hipSuccess ||
+      hipHostGetDevicePointer(reinterpret_cast<void **>(&b->h_mir_dev), b->h_mir, 0) != hipSuccess) {
+    batch_release(g);
+    return set_error(ENT_ENOMEM, "pinned host memory");
+  }
+  std::memset(b->h_mir, 0, mir_bytes);  // search 0, which no search uses
   b->bytes = ws_bytes(g->n, W, lcap);
   return ENT_OK;
 }
@@ -1461,8 +1499,9 @@ struct BKernels {
 
 template <int W>
 BKernels blevel_kernels() {
-  return {reinterpret_cast<const void *>(&k_blevel<kBatchBS, W>),
-          reinterpret_cast<const void *>(&k_blevel_bu<kBatchBS, W>),
+  const void *bu = nullptr;  // queued beside every launch of eight words only
+  if constexpr (W == 8) bu = reinterpret_cast<const void *>(&k_blevel_bu<kBatchBS, W>);
+  return {reinterpret_cast<const void *>(&k_blevel<kBatchBS, W>), bu,
           reinterpret_cast<const void *>(&k_bpersist<kBatchBS, W>)};
 }
 
@@ -1496,6 +1535,67 @@ std::vector<int32_t> place_sources(const ent_graph *g, const int32_t *roots, int
     placed[size_t(ENT_BATCH_MAX_SOURCES + p)] = order[size_t(p)];
   }
   return placed;
+}
+
+// Blocks per launch. By default the blocks that are resident at once (23 KB of
+// LDS each, six per CU, or fewer by registers: a part of a second round costs
+// more than it spreads; R-MAT 23, 64 sources: 3.18 ms at 6 per CU, 3.78 at 8;
+// R-MAT 22, 100 sources: 4.01 at 4, 4.21 at 8; 200 sources: 7.58 at 5, 7.69 at
+// 8; eight words keep 8: R-MAT 20, 512 sources 2.71 against 2.82 at 4), and no
+// more than a wavefront per 64 vertices: every block pays the prologue (65,536
+// vertices, 20 sources: 207 us at 256 blocks, 312 at 2,048).
+int batch_grid(const ent_graph *g, int W) {
+  const ent_bfs_config &c = g->cfg;
+  if (c.grid_blocks > 0) return c.grid_blocks;
+  if (c.blocks_per_cu > 0) return g->cus * c.blocks_per_cu;
+  const int per_cu = W == 1 ? 6 : W == 2 ? 4 : W == 4 ? 5 : 8;
+  const int64_t need = (g->nwords + kBatchBS / kWave - 1) / (kBatchBS / kWave);
+  return int(std::min<int64_t>(g->cus * per_cu, std::max<int64_t>(need, std::max(1, g->cus / 2))));
+}
+
+bool read_batch_slot(const BatchWorkspace *b, int slot, BState *out, unsigned *tag) {
+  const volatile unsigned long long *m = b->h_mir + slot * kBStateWords;
+  unsigned w[kBStateWords];
+  const unsigned t0 = unsigned(m[0] >> 32);
+  bool same = true;
+  for (int k = 0; k < kBStateWords; ++k) {
+    const unsigned long long x = m[k];
+    same = same && unsigned(x >> 32) == t0;
+    w[k] = unsigned(x);
+  }
+  std::memcpy(static_cast<void *>(out), w, sizeof w);
+  *tag = t0;
+  return same;
+}
+
+// Waits, spinning on the mirror, until this search is done (its rows are then
+// final: the launch that finds it done starts after every earlier one has
+// ended) or launch `last`, the last one queued, has published its state. The
+// stream is queried every 256 spins, so a failed launch ends the wait too.
+int wait_batch(ent_graph *g, long long last, unsigned search, BState *out) {
+  const unsigned want = unsigned(last + 1) + search * kBTagMul;
+  bool drained = false;
+  for (unsigned long spins = 0;; ++spins) {
+    BState s;
+    unsigned tag;
+    for (int sl = 0; sl < 2; ++sl) {
+      if (!read_batch_slot(g->batch, sl, &s, &tag) || unsigned(s.search) != search) continue;
+      if (s.done || tag == want) {
+        *out = s;
+        return ENT_OK;
+      }
+    }
+    if (drained) return set_error(ENT_EINTERNAL, "batch state not published");
+    if ((spins & 255) == 255) {
+      const hipError_t e = hipStreamQuery(g->stream);
+      if (e == hipSuccess) drained = true;  // the mirror is complete: one more look
+      else if (e != hipErrorNotReady) return set_error(ENT_EDEVICE, "batch failed: %s", hipGetErrorString(e));
+    }
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+    if (spins >= (1ul << 14)) std::this_thread::yield();
+  }
 }
 
 int run_batch(ent_graph *g, const int32_t *roots, int k, int *out, BState *fin) {
@@ -1537,6 +1637,9 @@ int run_batch(ent_graph *g, const int32_t *roots, int k, int *out, BState *fin) 
   a.fused = (W <= 4 && c.batch_fused > 0) ? std::max<long long>(1, (long long)g->n / c.batch_fused) : 0;
   const std::vector<int32_t> placed = place_sources(g, roots, k);
   a.rowmap = b->roots + ENT_BATCH_MAX_SOURCES;
+  a.hmir = b->h_mir_dev;
+  if (++g->search_seq == 0) g->search_seq = 1;
+  a.search = int(g->search_seq);
   // Level-0 counts on the host: distinct (vertex, word) pairs of the roots.
   std::vector<std::pair<int32_t, int>> vw;
   std::vector<int32_t> vs;
@@ -1578,6 +1681,11 @@ int run_batch(ent_graph *g, const int32_t *roots, int k, int *out, BState *fin) 
                             g->stream));
   }
   const BKernels kl = blevel_for(W);
+  const int lgrid = batch_grid(g, W);
+  // On small graphs a wavefront's top-down chunk shrinks until every
+  // wavefront has one (65,536 vertices, 20 sources: 151 against 159 us).
+  const int64_t share = (g->nwords + lgrid * (kBatchBS / kWave) - 1) / (lgrid * (kBatchBS / kWave));
+  if (c.launch != ENT_LAUNCH_PERSISTENT) a.chunk_words = int(std::min<int64_t>(a.chunk_words, std::max<int64_t>(share, 1)));
   if (c.launch == ENT_LAUNCH_PERSISTENT) {
     // Every block must be resident: no more wavefronts per CU than the
     // kernel's register budget guarantees (4 SIMDs x bpersist_waves_per_simd
@@ -1600,35 +1708,32 @@ int run_batch(ent_graph *g, const int32_t *roots, int k, int *out, BState *fin) 
     fin->error |= (s0.error | s1.error) & BERR_TIMEOUT;
     g->last_grid = pgrid;
     b->rings_clean = a.fused > 0 && fin->done && !fin->error;
+    HIP_TRY(hipEventRecord(g->ev1, g->stream));
     return ENT_OK;
   }
-  const int lgrid = c.grid_blocks > 0 ? c.grid_blocks : g->cus * std::max(1, c.blocks_per_cu > 0 ? c.blocks_per_cu : 8);
   long long i = 0;
-  int kk = std::max(2, b->expect_launches);
-  // A search like the last one that never pulled queues one kernel per
-  // launch; a pull it does meet runs in k_blevel (W <= 4). W = 8 always
-  // queues the pull kernel, whose registers k_blevel lacks.
-  const bool pull_kernel = W > 4 || b->pulled_last;
-  int pulls = pull_kernel ? 0 : 1;
+  // As many launches as the last search on the workspace needed, then 1, 2,
+  // 4 ... more, each batch queued once the last launch of the one before has
+  // started.
+  int kk = std::max(2, b->expect_launches), follow = 1;
   // At most two launches per level (top-down, then pull or apply), one flush
   // per lcap + 1 levels and the output; levels <= n.
   const long long max_launches = 4LL * ((long long)g->n + 4);
   for (;;) {
     for (int j = 0; j < kk; ++j, ++i) {
-      void *gargs[] = {&a, &i, &pulls};
       void *args[] = {&a, &i};
-      HIP_TRY(hipLaunchKernel(kl.gen, dim3(lgrid), dim3(kBatchBS), gargs, 0, g->stream));
-      if (pull_kernel) HIP_TRY(hipLaunchKernel(kl.bu, dim3(lgrid), dim3(kBatchBS), args, 0, g->stream));
+      HIP_TRY(hipLaunchKernel(kl.gen, dim3(lgrid), dim3(kBatchBS), args, 0, g->stream));
+      if (kl.bu) HIP_TRY(hipLaunchKernel(kl.bu, dim3(lgrid), dim3(kBatchBS), args, 0, g->stream));
     }
-    HIP_TRY(hipMemcpyAsync(b->h_ctl, b->ctl, sizeof(BState) * 2, hipMemcpyDeviceToHost, g->stream));
-    HIP_TRY(hipStreamSynchronize(g->stream));
-    *fin = b->h_ctl->st[(i - 1) & 1];
+    HIP_TRY(hipEventRecord(g->ev1, g->stream));  // end of the search once it is done
+    const int rc = wait_batch(g, i - 1, unsigned(a.search), fin);
+    if (rc) return rc;
     if (fin->done) break;
     if (i > max_launches) return set_error(ENT_EINTERNAL, "batch did not finish in %lld launches", i);
-    kk = std::min(2 * kk, 512);
+    kk = follow;
+    follow = std::min(2 * follow, 512);
   }
-  b->expect_launches = std::min(fin->phases + 1, 512);
-  b->pulled_last = fin->pulled != 0;
+  b->expect_launches = std::min(fin->phases, 512);
   g->last_grid = lgrid;
   b->rings_clean = a.fused > 0 && !fin->error;
   return ENT_OK;
@@ -1648,6 +1753,7 @@ void batch_release(ent_graph *g) {
   dev_free(g, b->ctl, sizeof(BControl));
   dev_free(g, b->rows, b->rows_bytes);
   if (b->h_ctl) ignore(hipHostFree(b->h_ctl));
+  if (b->h_mir) ignore(hipHostFree(b->h_mir));
   delete b;
   g->batch = nullptr;
 }
@@ -1739,8 +1845,9 @@ int batch_locked(ent_graph *g, const int32_t *roots, int k, int32_t *depths_dev,
     return set_error(ENT_EINTERNAL, "device reported error flags 0x%x", fin.error);
   }
   const unsigned long long edges = fin.total_edges, verts = fin.total_vertices, alg = fin.alg_bytes;
-  HIP_TRY(hipEventRecord(g->ev1, g->stream));
-  HIP_TRY(hipEventSynchronize(g->ev1));
+  // The search recorded ev1 behind its last launch: with statistics wanted,
+  // the launches that exit at once behind the end are waited for too.
+  if (st) HIP_TRY(hipEventSynchronize(g->ev1));
   const auto t1 = std::chrono::steady_clock::now();
   if (st) {
     std::memset(st, 0, sizeof *st);
