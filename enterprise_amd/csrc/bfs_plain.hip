@@ -1317,6 +1317,47 @@ int check_config(const ent_bfs_config *c) {
   return ENT_OK;
 }
 
+// Blocks per level launch, and the bitmap words of a wavefront's chunk.
+// Chunks go to consecutive wavefronts of one XCD before the next
+// (xcd_wave_id), so a sweep that leaves wavefronts without a chunk leaves whole
+// XCDs idle, and one that needs a little more than a whole number of rounds
+// runs a nearly empty last one. By default the sweep is therefore cut to fit:
+//  - from 2^21 vertices on the full grid (8,192 wavefronts), chunks of the
+//    words that make a whole number of rounds, as near bu_chunk_words as that
+//    allows (R-MAT 5,000,000: 190 us with one round of 10 words, 219 with 8
+//    words and a second round a fifth full; uniform 3,000,017: 266 with 6
+//    words, 286 with 8, which leave the last two XCDs idle);
+//  - below, a smaller grid whose wavefronts all have one chunk of 4 (from 2^20
+//    vertices on) or 2 words: every block of a launch pays the prologue
+//    (R-MAT 20: 102 us with 1,024 blocks and 4 words, 107 with 2,048 and 2, 134
+//    with 2,048 and 8, on two XCDs; R-MAT 18: 75.6 against 98).
+// bu_chunk_words bounds the chunk of small graphs from above; grid_blocks and
+// blocks_per_cu, when set, are taken as they are.
+struct LevelShape {
+  int grid, chunk;
+};
+
+LevelShape level_shape(const ent_graph *g) {
+  const ent_bfs_config &c = g->cfg;
+  const int per_block = c.block_size / kWave;
+  const int full = g->cus * std::max(1, 2048 / c.block_size);
+  LevelShape s{full, c.bu_chunk_words};
+  if (c.grid_blocks > 0) s.grid = c.grid_blocks;
+  else if (c.blocks_per_cu > 0) s.grid = g->cus * c.blocks_per_cu;
+  else if (g->nwords < 4ll * full * per_block) {
+    const int64_t words = g->nwords >= 2ll * full * per_block ? 4 : 2;
+    const int64_t waves = (g->nwords + words - 1) / words;
+    const int64_t need = ((waves + per_block - 1) / per_block + 7) / 8 * 8;
+    s.grid = int(std::min<int64_t>(full, std::max<int64_t>(need, std::max(8, g->cus / 2))));
+  }
+  const int64_t waves = int64_t(s.grid) * per_block;
+  const int64_t one = waves * c.bu_chunk_words;  // words of a round at the configured chunk
+  const int64_t rounds = std::max<int64_t>(1, (g->nwords + one / 2) / one);
+  const int64_t even = std::max<int64_t>(1, (g->nwords + rounds * waves - 1) / (rounds * waves));
+  s.chunk = int(std::min<int64_t>(even, kWave));
+  return s;
+}
+
 Args make_args(ent_graph *g, int *depth) {
   Args a{};
   a.off = g->off;
@@ -1353,7 +1394,7 @@ Args make_args(ent_graph *g, int *depth) {
   a.alpha = c.alpha;
   a.beta = c.beta;
   a.bu_probe = c.bu_probe;
-  a.chunk_words = c.bu_chunk_words;
+  a.chunk_words = c.launch == ENT_LAUNCH_PERSISTENT ? c.bu_chunk_words : level_shape(g).chunk;
   a.hub_slot = g->hub_slot;
   a.hub_tag = g->hub_tag;
   a.hub_mask = g->hub_slots > 0 ? g->hub_slots - 1 : -1;
@@ -1391,11 +1432,7 @@ KernelSet kernels_for(int bs, bool hub, bool count) {
   }
 }
 
-int level_grid(ent_graph *g) {
-  if (g->cfg.grid_blocks > 0) return g->cfg.grid_blocks;
-  const int bpc = g->cfg.blocks_per_cu > 0 ? g->cfg.blocks_per_cu : std::max(1, 2048 / g->cfg.block_size);
-  return g->cus * bpc;
-}
+int level_grid(ent_graph *g) { return level_shape(g).grid; }
 
 // Blocks per CU for the cooperative kernel. Every block must be resident at
 // once, and the runtime's occupancy query does not see every register limit,
