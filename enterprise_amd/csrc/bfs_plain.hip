@@ -1062,6 +1062,161 @@ __global__ __launch_bounds__(BS) void k_level(Args a, long long i) {
   run_phase<BS, HUB, COUNT>(a, sm, i);
 }
 
+// Whole search of a small graph in one block: visited bits and frontier
+// queues in LDS, the frontier's edges spread over all threads.
+//
+// A launch per level costs about 8 us of launch, prologue and dependent round
+// trips whatever the graph's size, and a hub's row goes to one wavefront. Here
+// eight lanes take two frontier vertices' rows at a time, the whole block a row
+// of kTinyHub edges or more, and a neighbour is claimed with an atomic OR
+// in LDS and queued there: two round trips to L2 and a few block barriers a
+// level. Bound: one CU's instruction issue, about 2 edges a nanosecond, so the
+// rule stops at kTinyEdges. Against a launch per level: R-MAT 1,024 vertices 91
+// -> 34.5 us, 2,000 with 60,000 edges 75 -> 40, 10,000 with 93,000 edges 79 ->
+// 70 (and with 220,000 edges 59 -> 124, hence the rule), uniform 2,000 90 ->
+// 28, a 30 x 40 grid 183 -> 55. More rows in flight per group, sixteen lanes
+// a row, and a queue rebuilt from the new bits were all slower.
+//
+// The first wavefront publishes the finished state to the host mirror itself:
+// every wavefront's stores are complete at the barrier before it, and its
+// system-scope release writes them back first.
+constexpr int kTinyThreads = 1024;
+constexpr int kTinyVertices = 1 << 14;  // 16-bit queue entries, 64 KiB for both queues
+constexpr int kTinyLanes = 8;
+constexpr int kTinyRows = 2;            // rows a group of lanes has in flight
+constexpr unsigned kTinyHub = 256;
+constexpr int64_t kTinyEdges = 3 << 15;
+constexpr int kTinyHubs = kTinyEdges / kTinyHub;  // there are no more rows of that length
+struct TinySmem {
+  unsigned vis[kTinyVertices / 32];
+  unsigned short q[2][kTinyVertices];
+  unsigned hub_s[kTinyHubs], hub_d[kTinyHubs];
+  unsigned qn[2], nhub[2];
+  unsigned long long mf;
+  State S;
+};
+
+__global__ __launch_bounds__(kTinyThreads) void k_tiny(const long long *off, const int *adj, int *depth, int n,
+                                                       int root, int search, unsigned long long *hmir) {
+  __shared__ TinySmem sm;
+  const int t = threadIdx.x, lane = lane_id();
+  const unsigned long long t_begin = rt_clock();
+  for (int k = t; k < kTinyVertices / 32; k += kTinyThreads) sm.vis[k] = k == (root >> 5) ? 1u << (root & 31) : 0u;
+  for (int v = t; v < n; v += kTinyThreads) depth[v] = v == root ? 0 : -1;
+  if (t == 0) {
+    sm.q[0][0] = (unsigned short)root;
+    sm.qn[0] = 1;
+    sm.nhub[0] = sm.nhub[1] = 0;
+    sm.mf = 0;
+  }
+  __syncthreads();
+  unsigned long long mf = 0;
+  unsigned total_nf = 0;
+  int L = 0;
+  for (;; ++L) {
+    const unsigned short *qin = sm.q[L & 1];
+    unsigned short *qout = sm.q[(L + 1) & 1];
+    unsigned *qcnt = &sm.qn[(L + 1) & 1], *nhub = &sm.nhub[L & 1];
+    const unsigned cnt = sm.qn[L & 1];
+    total_nf += cnt;
+    if (cnt == 0) break;  // the whole block
+    if (t == 0) {
+      *qcnt = 0;
+      sm.nhub[(L + 1) & 1] = 0;
+    }
+    __syncthreads();
+    // Claims u and queues it if it was unvisited (-1: no neighbour).
+    auto claim = [&](int u) {
+      if (u < 0) return;
+      const unsigned bit = 1u << (u & 31);
+      // A plain look first: most edges lead back.
+      if ((sm.vis[u >> 5] & bit) || (atomicOr(&sm.vis[u >> 5], bit) & bit)) return;
+      qout[atomicAdd(qcnt, 1u)] = (unsigned short)u;
+      depth[u] = L + 1;
+    };
+    // Neighbours i, i + stride, i + 2 stride, i + 3 stride of the row [s, s + d).
+    auto visit = [&](unsigned s, unsigned d, unsigned i, unsigned stride) {
+      int u[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j] = i + j * stride < d ? adj[s + i + j * stride] : -1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) claim(u[j]);
+    };
+    constexpr unsigned kGroups = kTinyThreads / kTinyLanes;
+    const unsigned gl = unsigned(t) % kTinyLanes;
+    for (unsigned k0 = unsigned(t) / kTinyLanes; k0 < cnt; k0 += kTinyRows * kGroups) {
+      unsigned s[kTinyRows], d[kTinyRows];
+#pragma unroll
+      for (int x = 0; x < kTinyRows; ++x) {
+        const unsigned k = k0 + x * kGroups;
+        s[x] = d[x] = 0;
+        if (k < cnt) {
+          const int v = qin[k];
+          const long long b = off[v];
+          s[x] = unsigned(b);
+          d[x] = unsigned(off[v + 1] - b);
+        }
+      }
+      int u[kTinyRows][2];
+#pragma unroll
+      for (int x = 0; x < kTinyRows; ++x) {
+        if (gl == 0) mf += d[x];
+        if (d[x] >= kTinyHub) {
+          if (gl == 0) {
+            const unsigned h = atomicAdd(nhub, 1u);
+            sm.hub_s[h] = s[x];
+            sm.hub_d[h] = d[x];
+          }
+          d[x] = 0;
+        }
+        u[x][0] = gl < d[x] ? adj[s[x] + gl] : -1;
+        u[x][1] = gl + kTinyLanes < d[x] ? adj[s[x] + gl + kTinyLanes] : -1;
+      }
+#pragma unroll
+      for (int x = 0; x < kTinyRows; ++x) {
+        claim(u[x][0]);
+        claim(u[x][1]);
+      }
+#pragma unroll
+      for (int x = 0; x < kTinyRows; ++x)
+        for (unsigned i = gl + 2 * kTinyLanes; i < d[x]; i += 4 * kTinyLanes) visit(s[x], d[x], i, kTinyLanes);
+    }
+    __syncthreads();
+    const unsigned nh = *nhub;
+    for (unsigned h = 0; h < nh; ++h) {
+      const unsigned s = sm.hub_s[h], d = sm.hub_d[h];
+      for (unsigned i = t; i < d; i += 4 * kTinyThreads) visit(s, d, i, kTinyThreads);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mf += __shfl_xor(mf, o);
+  if (lane == 0) atomicAdd(&sm.mf, mf);
+  __syncthreads();
+  if (t == 0) {
+    State S{};
+    S.level = L;
+    S.done = 1;
+    S.levels = L;
+    S.td_levels = L;
+    S.phases = 1;
+    S.total_nf = total_nf;
+    S.total_mf = sm.mf;
+    S.t_begin = t_begin;
+    S.t_end = rt_clock();
+    S.search = search;
+    sm.S = S;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are done
+  __syncthreads();
+  if (t < kWave) {
+    __threadfence_system();
+    const unsigned tag = 1u + unsigned(search) * kTagMul;
+    if (lane < kHostStateWords)
+      hmir[lane] = (static_cast<unsigned long long>(tag) << 32) | reinterpret_cast<const unsigned *>(&sm.S)[lane];
+  }
+}
+
 // Hands the search over to the several-levels-per-launch form (bfs_deep.hip)
 // after launch i - 1, a queue-driven level: derives the state launch i would
 // have and, if that is another queue-driven level whose frontier does not
@@ -1590,6 +1745,26 @@ int run_deep(ent_graph *g, Args &a, long long next, State *fin, int *taken) {
   return ENT_OK;
 }
 
+// Whether a search on g runs in one block (k_tiny): at most kTinyVertices
+// vertices and kTinyEdges edges, a launch form that is free to, and the same
+// configurations as above.
+bool tiny_fits(const ent_graph *g) {
+  const ent_bfs_config &c = g->cfg;
+  return g->n <= kTinyVertices && g->m <= kTinyEdges && !c.count_examined && g->hub_slots == 0 && c.queue_small >= 0 &&
+         (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN) &&
+         (c.launch == ENT_LAUNCH_STREAM || c.launch == ENT_LAUNCH_GRAPH);
+}
+
+int run_tiny(ent_graph *g, Args &a, int root, State *fin) {
+  if (++g->search_seq == 0) g->search_seq = 1;
+  int search = int(g->search_seq);
+  void *args[] = {&a.off, &a.adj, &a.depth, &a.n, &root, &search, &a.hmir};
+  HIP_TRY(launch(reinterpret_cast<const void *>(&k_tiny), 1, kTinyThreads, args, g->stream));
+  HIP_TRY(hipEventRecord(g->ev1, g->stream));
+  g->last_grid = 1;
+  return wait_state(g, 0, g->search_seq, fin);
+}
+
 // Runs one search; on success *fin holds the final state.
 int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
   const ent_bfs_config &cfg = g->cfg;
@@ -1602,6 +1777,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
     return set_error(ENT_EINVAL, "hub_cache %d with block_size %d needs %zu bytes of LDS per block (64 KiB max)",
                      cfg.hub_cache, cfg.block_size, ks.smem + hub_lds_bytes(cfg));
   Args a = make_args(g, depth_dev);
+  if (tiny_fits(g)) return run_tiny(g, a, root, fin);  // leaves the marks as they are
   const int bs = cfg.block_size;
   int first_bu = cfg.direction == ENT_DIR_BOTTOMUP ? 1 : 0;
   if (++g->search_seq == 0) g->search_seq = 1;  // 0 marks the zeroed mirror
@@ -1989,7 +2165,7 @@ static int search_locked(ent_graph *g, int root, int *depth, ent_stats *st,
   if (c.error)
     return set_error(ENT_EINTERNAL, "device reported error flags 0x%x (2 level guard, 4 barrier timeout)", c.error);
   if (!c.done) return set_error(ENT_EINTERNAL, "search ended without completion");
-  g->marks_clean = true;
+  if (!tiny_fits(g)) g->marks_clean = true;
   // The last counted launch finds the frontier empty and records nothing.
   if (g->cfg.count_examined) g->trace_launches = c.phases - 1;
   if (st) {

@@ -390,3 +390,42 @@ def test_topdown_directed_sinks(oracle, launch):
             reached = want >= 0
             assert st["reached_vertices"] == int(reached.sum())
             assert st["reached_edges"] == int(np.diff(beg)[reached].sum())
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 65, 1000, 4097, 16383, 16384, 16385])
+def test_one_block_search(oracle, n):
+    """Searches of small graphs in one block, at the edges of its vertex rule:
+    random edges, rows of 255, 256 and 257 edges (the whole block takes the
+    longer ones), isolated vertices and roots, an unaligned depth array; and
+    the other forms before and after on the same handle."""
+    rng = np.random.default_rng(n)
+    src, dst = rng.integers(0, n, 2 * n), rng.integers(0, max(1, n - n // 8), 2 * n)
+    if n > 1000:
+        hubs = [np.full(d, h) for h, d in enumerate((255, 256, 257, 900))]
+        src = np.concatenate([src, *hubs])
+        dst = np.concatenate([dst, *(rng.choice(n, h.size, replace=False) for h in hubs)])
+    g = HostGraph.from_edges(n, src, dst)
+    roots = sorted({0, n - 1, n // 2, *(int(r) for r in rng.integers(0, n, 3))})
+    with DeviceGraph(g) as dg:
+        buf = dg.device_alloc(4 * n + 4)
+        try:
+            for launch, direction in (("stream", "auto"), ("levels", "auto"), ("graph", "topdown"),
+                                      ("stream", "bottomup"), ("stream", "topdown"), ("persistent", "auto")):
+                dg.configure(launch=LAUNCHES[launch], direction=DIRS[direction])
+                for r in roots:
+                    st = _check(oracle, g, dg, r, f"one block n={n} {launch}/{direction}")
+                    assert st["td_levels"] + st["bu_levels"] == st["levels"]
+                dg.bfs_device(roots[0], buf + 4)
+                assert np.array_equal(dg.copy_depth(buf + 4, n), oracle.bfs(g.beg_pos, g.adj, roots[0]))
+        finally:
+            dg.device_free(buf)
+
+
+@pytest.mark.parametrize("tuples", [48000, 49200, 50500])
+def test_one_block_edge_rule(oracle, tuples):
+    """Edge counts around the one-block rule's 98,304."""
+    rng = np.random.default_rng(tuples)
+    g = HostGraph.from_edges(9000, rng.integers(0, 9000, tuples), rng.integers(0, 9000, tuples))
+    with DeviceGraph(g) as dg:
+        for r in g.pick_roots(3, 5):
+            _check(oracle, g, dg, int(r), f"one block m={g.m}")
