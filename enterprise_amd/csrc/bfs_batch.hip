@@ -53,6 +53,7 @@
 #include "ent_deep.h"
 #include "ent_device.h"
 #include "ent_internal.h"
+#include "ent_tiny.h"
 
 namespace ent {
 
@@ -1412,6 +1413,20 @@ __global__ void k_zero_u64(unsigned long long *p, long long n) {
     p[i] = 0ull;
 }
 
+// Small graphs: source blockIdx.x searched in one block (ent_tiny.h), what it
+// found to host memory (levels, vertices, edges).
+__global__ __launch_bounds__(kTinyThreads) void k_tiny_batch(const long long *off, const int *adj, const int *roots,
+                                                             int *rows, int n, unsigned long long *found) {
+  __shared__ TinySmem sm;
+  const int s = blockIdx.x;
+  const TinyResult r = tiny_search(sm, off, adj, rows + (long long)s * n, n, roots[s]);
+  if (threadIdx.x == 0) {
+    found[3 * s] = (unsigned long long)r.levels;
+    found[3 * s + 1] = r.reached;
+    found[3 * s + 2] = sm.mf;
+  }
+}
+
 struct BatchWorkspace {
   int words = 0;      // W (1, 2, 4 or 8)
   int lcap = 0;       // levels kept between flushes (ring of lcap + 3 slots)
@@ -1423,7 +1438,9 @@ struct BatchWorkspace {
   BControl *ctl = nullptr;
   BControl *h_ctl = nullptr;
   size_t bytes = 0;
-  unsigned long long *h_mir = nullptr, *h_mir_dev = nullptr;  // host-coherent state mirror
+  // Host-coherent: the state mirror, what k_tiny_batch found, and the joint
+  // frontiers' bytes of a batch searched side by side.
+  unsigned long long *h_mir = nullptr, *h_mir_dev = nullptr;
   int expect_launches = 16;
   int *rows = nullptr;     // device rows of ent_bfs_batch (grown on demand)
   size_t rows_bytes = 0;
@@ -1482,7 +1499,7 @@ int reserve(ent_graph *g, int k, int lcap) {
     batch_release(g);
     return set_error(ENT_ENOMEM, "pinned host memory");
   }
-  const size_t mir_bytes = sizeof(unsigned long long) * 2 * kBStateWords;
+  const size_t mir_bytes = sizeof(unsigned long long) * (2 * kBStateWords + 3 * ENT_BATCH_MAX_SOURCES + 1);
   if (hipHostMalloc(reinterpret_cast<void **>(&b->h_mir), mir_bytes, hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer(reinterpret_cast<void **>(&b->h_mir_dev), b->h_mir, 0) != hipSuccess) {
     batch_release(g);
@@ -1778,18 +1795,67 @@ bool deep_batch_fits(const ent_graph *g, int k) {
          (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN);
 }
 
+// Roots by row and rows by 64-source group, to b->roots.
+int upload_sources(ent_graph *g, const int32_t *roots, int k) {
+  std::vector<int32_t> placed = place_sources(g, roots, k);
+  std::copy(roots, roots + k, placed.begin());
+  HIP_TRY(hipMemcpyAsync(g->batch->roots, placed.data(), sizeof(int32_t) * placed.size(), hipMemcpyHostToDevice,
+                         g->stream));
+  return ENT_OK;
+}
+
+// Ends a batch whose sources were searched side by side: queues the byte
+// count where it is wanted, waits, and fills in what the searches did not (the
+// caller adds levels, vertices and edges before or after).
+int drain_side_by_side(ent_graph *g, int k, const int *out, bool want_bytes, BState *fin) {
+  unsigned long long *joint = g->batch->h_mir + 2 * kBStateWords + 3 * ENT_BATCH_MAX_SOURCES;
+  if (want_bytes) {
+    const int rc = deep_queue_joint_bytes(g, out, g->batch->roots + ENT_BATCH_MAX_SOURCES, k, joint);
+    if (rc) return rc;
+  }
+  HIP_TRY(hipEventRecord(g->ev1, g->stream));
+  HIP_TRY(hipEventSynchronize(g->ev1));
+  fin->done = 1;
+  if (want_bytes) fin->alg_bytes = *joint + 4ull * 64ull * (unsigned long long)words_for(k) * (unsigned long long)g->n;
+  return ENT_OK;
+}
+
+// What follows from the levels of such a batch. The level history is not
+// used; the count of times the search outgrew it follows all the same.
+void side_by_side_levels(const ent_graph *g, BState *fin) {
+  fin->td_mask = fin->levels >= 64 ? ~0ull : (1ull << fin->levels) - 1;
+  const int kept = g->batch->lcap;
+  if (fin->levels >= kept + 2) fin->flushes = 1 + (fin->levels - 2 - kept) / (kept + 2);
+}
+
+// A batch on a small graph: one block per source, all in one launch.
+int run_tiny_batch(ent_graph *g, const int32_t *roots, int k, int *out, bool want_bytes, BState *fin) {
+  int rc = upload_sources(g, roots, k);
+  if (rc) return rc;
+  const BatchWorkspace *b = g->batch;
+  hipLaunchKernelGGL(k_tiny_batch, dim3(unsigned(k)), dim3(kTinyThreads), 0, g->stream, g->off, g->adj, b->roots, out,
+                     int(g->n), b->h_mir_dev + 2 * kBStateWords);
+  HIP_TRY(hipGetLastError());
+  if ((rc = drain_side_by_side(g, k, out, want_bytes, fin))) return rc;
+  const unsigned long long *f = b->h_mir + 2 * kBStateWords;
+  for (int s = 0; s < k; ++s) {
+    fin->levels = std::max(fin->levels, int(f[3 * s]));
+    fin->total_vertices += f[3 * s + 1];
+    fin->total_edges += f[3 * s + 2];
+  }
+  fin->phases = 1;
+  side_by_side_levels(g, fin);
+  return ENT_OK;
+}
+
 // *ran stays false when a frontier outgrew the queues (the rows are then
 // written again by the joint search).
 int run_deep_batch(ent_graph *g, const int32_t *roots, int k, int *out, bool want_bytes, BState *fin, bool *ran) {
   int rc = deep_reserve(g, k, kDeepQueue);
   if (rc) return rc;
-  // The roots by row, and the rows by 64-source group for the byte count.
-  int *droots = g->batch->roots;
-  std::vector<int32_t> placed = place_sources(g, roots, k);
-  std::copy(roots, roots + k, placed.begin());
-  HIP_TRY(hipMemcpyAsync(droots, placed.data(), sizeof(int32_t) * placed.size(), hipMemcpyHostToDevice, g->stream));
+  if ((rc = upload_sources(g, roots, k))) return rc;
   std::vector<DeepState> st(static_cast<size_t>(k));
-  if ((rc = deep_batch(g, droots, k, out, st.data()))) return rc;
+  if ((rc = deep_batch(g, g->batch->roots, k, out, st.data()))) return rc;
   for (const DeepState &s : st)
     if (s.error) {
       HIP_TRY(hipStreamSynchronize(g->stream));
@@ -1801,17 +1867,8 @@ int run_deep_batch(ent_graph *g, const int32_t *roots, int k, int *out, bool wan
     fin->total_vertices += s.total_nf;
     fin->total_edges += s.total_mf;
   }
-  fin->td_mask = fin->levels >= 64 ? ~0ull : (1ull << fin->levels) - 1;
-  fin->done = 1;
-  if (want_bytes) {
-    unsigned long long joint = 0;
-    if ((rc = deep_joint_bytes(g, out, droots + ENT_BATCH_MAX_SOURCES, k, &joint))) return rc;
-    fin->alg_bytes = joint + 4ull * 64ull * (unsigned long long)words_for(k) * (unsigned long long)g->n;
-  }
-  // The level history is not used; the count of times the search outgrew it
-  // follows from the levels all the same.
-  const int kept = g->batch->lcap;
-  if (fin->levels >= kept + 2) fin->flushes = 1 + (fin->levels - 2 - kept) / (kept + 2);
+  side_by_side_levels(g, fin);
+  if ((rc = drain_side_by_side(g, k, out, want_bytes, fin))) return rc;
   *ran = true;
   return ENT_OK;
 }
@@ -1827,7 +1884,10 @@ int batch_locked(ent_graph *g, const int32_t *roots, int k, int32_t *depths_dev,
   HIP_TRY(hipEventRecord(g->ev0, g->stream));
   BState fin{};
   bool ran = false;
-  if (deep_batch_fits(g, k)) {
+  if (tiny_fits(g) && g->cfg.batch_fused > 0) {
+    rc = run_tiny_batch(g, roots, k, depths_dev, st != nullptr, &fin);
+    ran = true;
+  } else if (deep_batch_fits(g, k)) {
     rc = run_deep_batch(g, roots, k, depths_dev, st != nullptr, &fin, &ran);
     if (!rc && !ran) g->deep_batch_off = true;
   }

@@ -609,15 +609,15 @@ int deep_batch(ent_graph *g, const int32_t *roots, int k, int *rows, DeepState *
   return deep_run(g, a, width, k, blocks, search, fin);
 }
 
-int deep_joint_bytes(ent_graph *g, const int *rows, const int *order_dev, int k, unsigned long long *bytes) {
+int deep_queue_joint_bytes(ent_graph *g, const int *rows, const int *order_dev, int k, unsigned long long *host) {
   unsigned long long *d = static_cast<unsigned long long *>(g->aux);
   HIP_TRY(hipMemsetAsync(d, 0, sizeof *d, g->stream));
-  const dim3 grid(unsigned(g->cus) * 8, unsigned((k + 63) / 64));
+  const unsigned blocks = unsigned(std::min<int64_t>(g->cus * 8, (g->n + 255) / 256));
+  const dim3 grid(blocks, unsigned((k + 63) / 64));
   auto kernel = k <= 16 ? &k_deep_joint<16> : k <= 32 ? &k_deep_joint<32> : &k_deep_joint<64>;
   hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g->stream, g->off, rows, order_dev, int(g->n), k, d);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(bytes, d, sizeof *bytes, hipMemcpyDeviceToHost, g->stream));
-  HIP_TRY(hipStreamSynchronize(g->stream));
+  HIP_TRY(hipMemcpyAsync(host, d, sizeof *host, hipMemcpyDeviceToHost, g->stream));
   return ENT_OK;
 }
 

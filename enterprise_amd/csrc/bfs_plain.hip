@@ -61,6 +61,7 @@
 #include "ent_common.h"
 #include "ent_deep.h"
 #include "ent_device.h"
+#include "ent_tiny.h"
 
 namespace ent {
 
@@ -1062,158 +1063,38 @@ __global__ __launch_bounds__(BS) void k_level(Args a, long long i) {
   run_phase<BS, HUB, COUNT>(a, sm, i);
 }
 
-// Whole search of a small graph in one block: visited bits and frontier
-// queues in LDS, the frontier's edges spread over all threads.
-//
-// A launch per level costs about 8 us of launch, prologue and dependent round
-// trips whatever the graph's size, and a hub's row goes to one wavefront. Here
-// eight lanes take two frontier vertices' rows at a time, the whole block a row
-// of kTinyHub edges or more, and a neighbour is claimed with an atomic OR
-// in LDS and queued there: two round trips to L2 and a few block barriers a
-// level. Bound: one CU's instruction issue, about 2 edges a nanosecond, so the
-// rule stops at kTinyEdges. Against a launch per level: R-MAT 1,024 vertices 91
-// -> 34.5 us, 2,000 with 60,000 edges 75 -> 40, 10,000 with 93,000 edges 79 ->
-// 70 (and with 220,000 edges 59 -> 124, hence the rule), uniform 2,000 90 ->
-// 28, a 30 x 40 grid 183 -> 55. More rows in flight per group, sixteen lanes
-// a row, and a queue rebuilt from the new bits were all slower.
-//
-// The first wavefront publishes the finished state to the host mirror itself:
-// every wavefront's stores are complete at the barrier before it, and its
-// system-scope release writes them back first.
-constexpr int kTinyThreads = 1024;
-constexpr int kTinyVertices = 1 << 14;  // 16-bit queue entries, 64 KiB for both queues
-constexpr int kTinyLanes = 8;
-constexpr int kTinyRows = 2;            // rows a group of lanes has in flight
-constexpr unsigned kTinyHub = 256;
-constexpr int64_t kTinyEdges = 3 << 15;
-constexpr int kTinyHubs = kTinyEdges / kTinyHub;  // there are no more rows of that length
-struct TinySmem {
-  unsigned vis[kTinyVertices / 32];
-  unsigned short q[2][kTinyVertices];
-  unsigned hub_s[kTinyHubs], hub_d[kTinyHubs];
-  unsigned qn[2], nhub[2];
-  unsigned long long mf;
-  State S;
-};
-
+// A small graph's search in one block (ent_tiny.h). The first wavefront
+// publishes the finished state to the host mirror itself: every wavefront's
+// stores are complete at the barrier before it, and its system-scope release
+// writes them back first.
 __global__ __launch_bounds__(kTinyThreads) void k_tiny(const long long *off, const int *adj, int *depth, int n,
                                                        int root, int search, unsigned long long *hmir) {
   __shared__ TinySmem sm;
-  const int t = threadIdx.x, lane = lane_id();
+  __shared__ State S;
   const unsigned long long t_begin = rt_clock();
-  for (int k = t; k < kTinyVertices / 32; k += kTinyThreads) sm.vis[k] = k == (root >> 5) ? 1u << (root & 31) : 0u;
-  for (int v = t; v < n; v += kTinyThreads) depth[v] = v == root ? 0 : -1;
-  if (t == 0) {
-    sm.q[0][0] = (unsigned short)root;
-    sm.qn[0] = 1;
-    sm.nhub[0] = sm.nhub[1] = 0;
-    sm.mf = 0;
-  }
-  __syncthreads();
-  unsigned long long mf = 0;
-  unsigned total_nf = 0;
-  int L = 0;
-  for (;; ++L) {
-    const unsigned short *qin = sm.q[L & 1];
-    unsigned short *qout = sm.q[(L + 1) & 1];
-    unsigned *qcnt = &sm.qn[(L + 1) & 1], *nhub = &sm.nhub[L & 1];
-    const unsigned cnt = sm.qn[L & 1];
-    total_nf += cnt;
-    if (cnt == 0) break;  // the whole block
-    if (t == 0) {
-      *qcnt = 0;
-      sm.nhub[(L + 1) & 1] = 0;
-    }
-    __syncthreads();
-    // Claims u and queues it if it was unvisited (-1: no neighbour).
-    auto claim = [&](int u) {
-      if (u < 0) return;
-      const unsigned bit = 1u << (u & 31);
-      // A plain look first: most edges lead back.
-      if ((sm.vis[u >> 5] & bit) || (atomicOr(&sm.vis[u >> 5], bit) & bit)) return;
-      qout[atomicAdd(qcnt, 1u)] = (unsigned short)u;
-      depth[u] = L + 1;
-    };
-    // Neighbours i, i + stride, i + 2 stride, i + 3 stride of the row [s, s + d).
-    auto visit = [&](unsigned s, unsigned d, unsigned i, unsigned stride) {
-      int u[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) u[j] = i + j * stride < d ? adj[s + i + j * stride] : -1;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) claim(u[j]);
-    };
-    constexpr unsigned kGroups = kTinyThreads / kTinyLanes;
-    const unsigned gl = unsigned(t) % kTinyLanes;
-    for (unsigned k0 = unsigned(t) / kTinyLanes; k0 < cnt; k0 += kTinyRows * kGroups) {
-      unsigned s[kTinyRows], d[kTinyRows];
-#pragma unroll
-      for (int x = 0; x < kTinyRows; ++x) {
-        const unsigned k = k0 + x * kGroups;
-        s[x] = d[x] = 0;
-        if (k < cnt) {
-          const int v = qin[k];
-          const long long b = off[v];
-          s[x] = unsigned(b);
-          d[x] = unsigned(off[v + 1] - b);
-        }
-      }
-      int u[kTinyRows][2];
-#pragma unroll
-      for (int x = 0; x < kTinyRows; ++x) {
-        if (gl == 0) mf += d[x];
-        if (d[x] >= kTinyHub) {
-          if (gl == 0) {
-            const unsigned h = atomicAdd(nhub, 1u);
-            sm.hub_s[h] = s[x];
-            sm.hub_d[h] = d[x];
-          }
-          d[x] = 0;
-        }
-        u[x][0] = gl < d[x] ? adj[s[x] + gl] : -1;
-        u[x][1] = gl + kTinyLanes < d[x] ? adj[s[x] + gl + kTinyLanes] : -1;
-      }
-#pragma unroll
-      for (int x = 0; x < kTinyRows; ++x) {
-        claim(u[x][0]);
-        claim(u[x][1]);
-      }
-#pragma unroll
-      for (int x = 0; x < kTinyRows; ++x)
-        for (unsigned i = gl + 2 * kTinyLanes; i < d[x]; i += 4 * kTinyLanes) visit(s[x], d[x], i, kTinyLanes);
-    }
-    __syncthreads();
-    const unsigned nh = *nhub;
-    for (unsigned h = 0; h < nh; ++h) {
-      const unsigned s = sm.hub_s[h], d = sm.hub_d[h];
-      for (unsigned i = t; i < d; i += 4 * kTinyThreads) visit(s, d, i, kTinyThreads);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mf += __shfl_xor(mf, o);
-  if (lane == 0) atomicAdd(&sm.mf, mf);
-  __syncthreads();
-  if (t == 0) {
-    State S{};
-    S.level = L;
-    S.done = 1;
-    S.levels = L;
-    S.td_levels = L;
-    S.phases = 1;
-    S.total_nf = total_nf;
-    S.total_mf = sm.mf;
-    S.t_begin = t_begin;
-    S.t_end = rt_clock();
-    S.search = search;
-    sm.S = S;
+  const TinyResult r = tiny_search(sm, off, adj, depth, n, root);
+  if (threadIdx.x == 0) {
+    State s{};
+    s.level = r.levels;
+    s.done = 1;
+    s.levels = r.levels;
+    s.td_levels = r.levels;
+    s.phases = 1;
+    s.total_nf = r.reached;
+    s.total_mf = sm.mf;
+    s.t_begin = t_begin;
+    s.t_end = rt_clock();
+    s.search = search;
+    S = s;
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are done
   __syncthreads();
-  if (t < kWave) {
+  if (threadIdx.x < kWave) {
+    const int lane = threadIdx.x;
     __threadfence_system();
     const unsigned tag = 1u + unsigned(search) * kTagMul;
     if (lane < kHostStateWords)
-      hmir[lane] = (static_cast<unsigned long long>(tag) << 32) | reinterpret_cast<const unsigned *>(&sm.S)[lane];
+      hmir[lane] = (static_cast<unsigned long long>(tag) << 32) | reinterpret_cast<const unsigned *>(&S)[lane];
   }
 }
 
@@ -1743,16 +1624,6 @@ int run_deep(ent_graph *g, Args &a, long long next, State *fin, int *taken) {
   fin->phases += D.launches;
   fin->t_end = D.t_end;
   return ENT_OK;
-}
-
-// Whether a search on g runs in one block (k_tiny): at most kTinyVertices
-// vertices and kTinyEdges edges, a launch form that is free to, and the same
-// configurations as above.
-bool tiny_fits(const ent_graph *g) {
-  const ent_bfs_config &c = g->cfg;
-  return g->n <= kTinyVertices && g->m <= kTinyEdges && !c.count_examined && g->hub_slots == 0 && c.queue_small >= 0 &&
-         (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN) &&
-         (c.launch == ENT_LAUNCH_STREAM || c.launch == ENT_LAUNCH_GRAPH);
 }
 
 int run_tiny(ent_graph *g, Args &a, int root, State *fin) {

@@ -87,8 +87,9 @@ int deep_run(ent_graph *g, const DeepArgs &a, int width, int k, int blocks, unsi
 // entries.
 int deep_batch(ent_graph *g, const int32_t *roots, int k, int *rows, DeepState *fin);
 
-// Algorithmic bytes of the joint frontiers: 8 + 12 deg(v) for each distinct
-// (vertex, depth) pair of each 64-source group (rows order[64 g] on).
-int deep_joint_bytes(ent_graph *g, const int *rows, const int *order_dev, int k, unsigned long long *bytes);
+// Queues the algorithmic bytes of the joint frontiers, 8 + 12 deg(v) for each
+// distinct (vertex, depth) pair of each 64-source group (rows order[64 g] on),
+// and their copy to *host (pinned).
+int deep_queue_joint_bytes(ent_graph *g, const int *rows, const int *order_dev, int k, unsigned long long *host);
 
 }  // namespace ent

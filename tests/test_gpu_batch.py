@@ -503,3 +503,25 @@ def test_row_hash_widths(cols):
                 assert np.array_equal(out, want)
         finally:
             dg.device_free(ptr)
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (40, 3), (1000, 64), (3000, 65), (6000, 200), (16384, 16), (5000, 512)])
+def test_batch_one_block_per_source(oracle, n, k):
+    """Batches on small graphs, one block per source: every row equals the
+    oracle's, and the counts equal the joint search's on the same roots."""
+    rng = np.random.default_rng(n)
+    g = HostGraph.from_edges(n, rng.integers(0, n, 3 * n), rng.integers(0, max(1, n - n // 10), 3 * n))
+    roots = rng.integers(0, n, k).astype(np.int32)
+    with DeviceGraph(g) as dg:
+        dg.batch_reserve(k, 5)
+        _say(f"[gpu] batch, one block per source n={n} k={k}")
+        out, st = dg.bfs_batch(roots)
+        dg.configure(batch_fused=0)
+        joint, sj = dg.bfs_batch(roots)
+        for i, r in enumerate(roots):
+            if i < 20 or i % 37 == 0:
+                assert np.array_equal(out[i], oracle.bfs(g.beg_pos, g.adj, int(r))), i
+        assert np.array_equal(out, joint)
+        for key in ("levels", "reached_vertices", "reached_edges", "alg_bytes", "words", "k", "flushes"):
+            assert st[key] == sj[key], (key, st, sj)
+        assert st["phases"] == 1
