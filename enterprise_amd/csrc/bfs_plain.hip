@@ -164,6 +164,7 @@ struct Args {
   const long long *off;
   const int *adj;
   const unsigned long long *nzmask;
+  const int *head;        // first neighbour of each row (k_heads), or null
   const int *hub_block;   // static block-class list
   const int *piece_v;     // static grid-class pieces: vertex
   const int *piece_k;     // piece index within the vertex
@@ -496,7 +497,24 @@ __device__ void inspect_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tall
 // bu_probe neighbours, hands longer unresolved lists to the whole wavefront
 // (ballot early exit), then writes its words of the next frontier and of the
 // visited bitmap without atomics, the depths, and the counts.
-template <int BS, bool HUB, bool COUNT>
+//
+// HEAD: a chunk with at least kBuDense undiscovered vertices per word first
+// tries every one of them against its first neighbour, read from the dense
+// array `head` (k_heads): 4 coalesced bytes per vertex instead of two offsets
+// and a line of the row. Rows hold their highest-degree neighbours first, so on
+// a skewed graph that one test finds 97-99% of what a dense level finds, and bit
+// 31 drops the rows that have nothing else to try; the rest go through the row
+// scan above from their second neighbour on. Lanes take kBuWords words at a
+// time, so that many head loads, then frontier loads, are in flight. The scan
+// alone is bound by those scattered row reads: R-MAT searches, edge factor 16,
+// without and with heads, 2^20 vertices 102 and 97 us, 2^22 157 and 138, 2^23
+// 610 and 438, 2^24 568 and 488. kBuDense 8, 16 and 32 give 507, 509 and 614 us
+// at 2^23 (two neighbours per head); kBuWords 2, 4 and 8 give 436, 434 and 508;
+// heads of one, two and four neighbours 434, 509 and 605, since the array is
+// then no longer the smaller read.
+constexpr int kBuDense = 16;
+constexpr int kBuWords = 4;
+template <int BS, bool HUB, bool COUNT, bool HEAD>
 __device__ void bu_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COUNT> &tl) {
   const unsigned long long *fr = a.front[L & 1];
   const int hm = a.hub_mask;
@@ -521,7 +539,50 @@ __device__ void bu_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COU
     const unsigned long long vis = own ? a.visited[w] : ~0ull;
     if (own) tl.s(8);
     wf[lane] = 0;
-    const int total = wave_compact_setup(~vis, wc, we);
+    int total = wave_compact_setup(~vis, wc, we);
+    int skip = 0;
+    if (HEAD && total >= CW * kBuDense) {
+      skip = 1;
+      for (int j0 = 0; j0 < CW; j0 += kBuWords) {
+        unsigned long long cw[kBuWords];
+        int h[kBuWords];  // bit 31: nothing else to try
+        unsigned bit[kBuWords];
+#pragma unroll
+        for (int x = 0; x < kBuWords; ++x) {
+          cw[x] = j0 + x < CW ? wc[j0 + x] : 0ull;
+          const long long hv = (w0 + j0 + x) * 64 + lane;
+          h[x] = ((cw[x] >> lane) & 1) ? a.head[hv] : INT32_MAX;
+        }
+#pragma unroll
+        for (int x = 0; x < kBuWords; ++x) {
+          bit[x] = 0;
+          if ((cw[x] >> lane) & 1) {
+            const int u = h[x] & INT32_MAX;
+            bit[x] = (reinterpret_cast<const unsigned *>(fr)[u >> 5] >> (u & 31)) & 1u;
+          }
+        }
+#pragma unroll
+        for (int x = 0; x < kBuWords; ++x) {
+          const unsigned long long hits = __ballot(bit[x] != 0);
+          const unsigned long long left = cw[x] & ~hits & ~__ballot(h[x] < 0);
+          if (lane == 0) {
+            wf[j0 + x] = hits;
+            wc[j0 + x] = left;
+          }
+          if (bit[x]) {
+            const int hv = int((w0 + j0 + x) * 64) + lane;
+            const long long d = a.off[hv + 1] - a.off[hv];
+            a.depth[hv] = L + 1;
+            nf += 1;
+            mf += (unsigned long long)d;
+            md = deg_max(md, d);
+            stage_push(sm, hv);
+          }
+        }
+      }
+      wave_sync();
+      total = wave_compact_setup(lane < CW ? wc[lane] : 0ull, wc, we);
+    }
     for (int b0 = 0; b0 < total; b0 += kWave) {
       const int k = b0 + lane;
       int v = 0, j = 0;
@@ -539,7 +600,7 @@ __device__ void bu_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COU
         const long long pe = min(e, s + a.bu_probe);
         // Four neighbours per step: their loads overlap; the step stops the
         // scan if any of them is in the frontier.
-        for (p = s; p + 3 < pe; p += 4) {
+        for (p = s + skip; p + 3 < pe; p += 4) {
           const int u0 = a.adj[p], u1 = a.adj[p + 1], u2 = a.adj[p + 2], u3 = a.adj[p + 3];
           tl.e(4);
           // A frontier hub among the four ends the scan from LDS.
@@ -1023,7 +1084,7 @@ __global__ __launch_bounds__(BS) void k_init(Args a, int root, int first_bu, int
   }
 }
 
-template <int BS, bool HUB, bool COUNT>
+template <int BS, bool HUB, bool COUNT, bool HEAD = false>
 __device__ __forceinline__ void run_phase(const Args &a, Smem<BS> &sm, long long i) {
   const int L = sm.S.level;
   const int slot = int(i % 3);
@@ -1033,7 +1094,7 @@ __device__ __forceinline__ void run_phase(const Args &a, Smem<BS> &sm, long long
       if (HUB && a.hub_td) td_phase<BS, HUB, COUNT>(a, sm, L, tl);
       else td_phase<BS, false, COUNT>(a, sm, L, tl);
       break;
-    case PH_BU: bu_phase<BS, HUB, COUNT>(a, sm, L, slot, tl); break;
+    case PH_BU: bu_phase<BS, HUB, COUNT, HEAD>(a, sm, L, slot, tl); break;
     case PH_INSPECT: inspect_phase<BS, HUB, COUNT>(a, sm, L, slot, tl); break;
     case PH_TDQ: tdq_phase<BS, COUNT>(a, sm, L, slot, tl); break;
     default: rebuild_phase<BS, HUB, COUNT>(a, sm, L, tl); break;
@@ -1061,6 +1122,18 @@ __global__ __launch_bounds__(BS) void k_level(Args a, long long i) {
   begin_launch<BS, COUNT>(a, sm, i, false);
   if (sm.S.done) return;
   run_phase<BS, HUB, COUNT>(a, sm, i);
+}
+
+// The same with heads in its bottom-up phase, for graphs that have them. That
+// phase wants 68 VGPRs and 88 SGPRs, which leaves 7 wavefronts per SIMD and a
+// grid of 8 blocks per CU with a last wave of its own (a search of 2^22 vertices
+// then takes 174 us); held to 8, at 7 spilled SGPRs, it is 138.
+template <int BS>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_level_heads(Args a, long long i) {
+  __shared__ Smem<BS> sm;
+  begin_launch<BS, false>(a, sm, i, false);
+  if (sm.S.done) return;
+  run_phase<BS, false, false, true>(a, sm, i);
 }
 
 // A small graph's search in one block (ent_tiny.h). The first wavefront
@@ -1150,6 +1223,15 @@ __global__ __launch_bounds__(kWave) void k_deep_take(Args a, long long i, DeepCt
   }
   static_assert(kDeepStripes == kStripes && kStripes == kWave, "one queue stripe per lane");
   d->st[1].qn[lane] = unsigned(min(qn, (unsigned long long)a.qcap_s));
+}
+
+// First neighbour of every row in device order (vertex 0 for rows without
+// edges, which no bottom-up level probes); bit 31 says that the row has no more.
+__global__ __launch_bounds__(256) void k_heads(const long long *off, const int *adj, long long n, int *head) {
+  for (long long v = (long long)blockIdx.x * 256 + threadIdx.x; v < n; v += (long long)gridDim.x * 256) {
+    const long long s = off[v], d = off[v + 1] - s;
+    head[v] = (d > 0 ? adj[s] : 0) | (d <= 1 ? INT32_MIN : 0);
+  }
 }
 
 // Whole search in one cooperative launch: launches 0, 1, 2, ... separated by
@@ -1399,6 +1481,7 @@ Args make_args(ent_graph *g, int *depth) {
   a.off = g->off;
   a.adj = g->adj;
   a.nzmask = g->nzmask;
+  a.head = g->store->head;
   a.hub_block = g->hub_block;
   a.piece_v = g->piece_v;
   a.piece_k = g->piece_k;
@@ -1453,18 +1536,21 @@ KernelSet kernel_set_of() {
 }
 
 template <int BS>
-KernelSet kernel_set(bool hub, bool count) {
+KernelSet kernel_set(bool hub, bool count, bool head) {
   if (count) return hub ? kernel_set_of<BS, true, true>() : kernel_set_of<BS, false, true>();
-  return hub ? kernel_set_of<BS, true, false>() : kernel_set_of<BS, false, false>();
+  if (hub) return kernel_set_of<BS, true, false>();
+  KernelSet ks = kernel_set_of<BS, false, false>();
+  if (head) ks.level = reinterpret_cast<const void *>(&k_level_heads<BS>);
+  return ks;
 }
 
-KernelSet kernels_for(int bs, bool hub, bool count) {
+KernelSet kernels_for(int bs, bool hub, bool count, bool head) {
   switch (bs) {
-    case 64: return kernel_set<64>(hub, count);
-    case 128: return kernel_set<128>(hub, count);
-    case 512: return kernel_set<512>(hub, count);
-    case 1024: return kernel_set<1024>(hub, count);
-    default: return kernel_set<256>(hub, count);
+    case 64: return kernel_set<64>(hub, count, head);
+    case 128: return kernel_set<128>(hub, count, head);
+    case 512: return kernel_set<512>(hub, count, head);
+    case 1024: return kernel_set<1024>(hub, count, head);
+    default: return kernel_set<256>(hub, count, head);
   }
 }
 
@@ -1642,7 +1728,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
   int rc = build_lists(g);
   if (rc) return rc;
   const bool count = cfg.count_examined != 0;
-  const KernelSet ks = kernels_for(cfg.block_size, g->hub_slots > 0, count);
+  const KernelSet ks = kernels_for(cfg.block_size, g->hub_slots > 0, count, g->store->head != nullptr);
   if (count) HIP_TRY(hipMemsetAsync(g->ctl->exam, 0, sizeof(g->ctl->exam), g->stream));
   if (ks.smem + hub_lds_bytes(cfg) > 65536)
     return set_error(ENT_EINVAL, "hub_cache %d with block_size %d needs %zu bytes of LDS per block (64 KiB max)",
@@ -1878,6 +1964,17 @@ int ent_graph_upload_ex(const int64_t *beg_pos, const int32_t *adj, int64_t n, i
 
 namespace ent {
 
+// Graphs that get heads (bu_phase): only skewed ones, whose first neighbours are
+// hubs. Uniform random graphs of edge factor 8 have a largest degree of 2-3
+// times the mean and lose by them (200,000 vertices 132 us without, 136 with);
+// R-MAT ones have 30 times and more at every size. Below 2^19 vertices a level
+// is launch-bound (2^18: 74.5 us without, 75.2 with; 2^19 91.8 and 90.2).
+// Rows in the caller's order find less with their first neighbour: 2^21
+// vertices 131 and 133 us, 2^22 160 and 152, 2^23 559 and 419.
+constexpr int kHeadSkew = 16;
+constexpr int64_t kHeadVertices = 1 << 19;
+constexpr int64_t kHeadVerticesKept = 1 << 22;
+
 int upload_graph(const int64_t *beg_pos, const int32_t *adj, bool adj_on_device, int64_t n, int64_t m, int device,
                  int32_t flags, ent_graph **out) {
   if (flags & ~int32_t(ENT_UPLOAD_KEEP_ORDER)) return set_error(ENT_EINVAL, "unknown upload flags 0x%x", flags);
@@ -1962,6 +2059,19 @@ int upload_graph(const int64_t *beg_pos, const int32_t *adj, bool adj_on_device,
   UP_TRY(hipMemcpy(g->nzmask, nz.data(), sizeof(unsigned long long) * size_t(g->nwords), hipMemcpyHostToDevice));
   rc = alloc_workspace(g);
   if (!rc && !(flags & ENT_UPLOAD_KEEP_ORDER)) rc = order_rows_by_degree(g);
+  const bool heads = n >= (flags & ENT_UPLOAD_KEEP_ORDER ? kHeadVerticesKept : kHeadVertices) &&
+                     g->store->max_deg / kHeadSkew >= m / n;
+  if (!rc && heads && device_malloc(device, reinterpret_cast<void **>(&g->store->head), sizeof(int) * size_t(n)) != hipSuccess) {
+    g->store->head = nullptr;  // no room: the levels scan the rows alone
+    ignore(hipGetLastError());
+  }
+  if (!rc && g->store->head) {
+    g->dev_bytes += sizeof(int) * size_t(n);
+    hipLaunchKernelGGL(k_heads, dim3(unsigned(g->cus) * 8), dim3(256), 0, g->stream, g->off, g->adj, (long long)n,
+                       g->store->head);
+    UP_TRY(hipGetLastError());
+    UP_TRY(hipStreamSynchronize(g->stream));
+  }
   if (rc) {
     release(g);
     return rc;

@@ -31,6 +31,7 @@ struct GraphStore {
   unsigned long long *nzmask = nullptr;  // bit v: degree(v) > 0
   std::vector<int32_t> h_deg;            // host copy of degrees (for the static lists)
   int32_t max_deg = 0;
+  int *head = nullptr;                   // first neighbour of each row, or null (bfs_plain.hip)
   std::mutex rows_mu;                    // guards rows, rows_width (ent_deep.h)
   int *rows = nullptr;
   int rows_width = -1;                   // -1: not built yet
@@ -40,6 +41,7 @@ struct GraphStore {
     ignore(hipFree(adj));
     ignore(hipFree(nzmask));
     ignore(hipFree(rows));
+    ignore(hipFree(head));
   }
 };
 // Reorders every adjacency row by descending floor(log2(neighbour degree)),

@@ -429,3 +429,26 @@ def test_one_block_edge_rule(oracle, tuples):
     with DeviceGraph(g) as dg:
         for r in g.pick_roots(3, 5):
             _check(oracle, g, dg, int(r), f"one block m={g.m}")
+
+
+@pytest.mark.parametrize("n,per,keep", [(1 << 19, 2, False), ((1 << 19) + 33, 12, False), ((1 << 22) + 1, 3, True)])
+def test_first_neighbour_heads(oracle, n, per, keep):
+    """Skewed graphs from the size at which bottom-up levels try each vertex's
+    first neighbour before its row: rows of no, one, two and many neighbours,
+    whole and ragged last words, rows in degree and in the caller's order."""
+    rng = np.random.default_rng(n + per)
+    src = rng.integers(0, n, per * n)
+    dst = (n * rng.random(per * n) ** 4).astype(np.int64)
+    g = HostGraph.from_edges(n, src, dst)
+    deg = np.diff(g.beg_pos)
+    assert deg.max() >= 16 * (g.m // n + 1)
+    with DeviceGraph(g, keep_order=keep) as dg:
+        for dname in ("auto", "reference", "bottomup"):
+            for launch in ("stream", "graph", "persistent"):
+                dg.configure(direction=DIRS[dname], launch=LAUNCHES[launch])
+                for r in g.pick_roots(2, 9):
+                    _check(oracle, g, dg, int(r), f"heads n={n}/{dname}/{launch}")
+        dg.configure(direction=L.DIR_BOTTOMUP, launch=L.LAUNCH_STREAM)
+        for bs, cw in ((64, 64), (512, 3), (1024, 1)):
+            dg.configure(block_size=bs, bu_chunk_words=cw)
+            _check(oracle, g, dg, int(np.argmin(np.where(deg > 0, deg, n))), f"heads n={n}/bs{bs}/cw{cw}")
