@@ -694,7 +694,10 @@ __device__ void bu_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COU
 // graph, each a short latency chain) skip it, and once one has, the clearing
 // stops too. Both are off with the LDS hub table, whose frontier hubs the
 // rebuild records.
-constexpr int kTdqBitmapLevels = 3;
+// Uniform graphs reach their first large level after four (edge factor 8, 3 and
+// 4 levels of bitmaps: 200,000 vertices 90 and 86 us, 3 million 213 and 207);
+// with 5, 6 and 8 nothing else gains.
+constexpr int kTdqBitmapLevels = 4;
 __device__ __forceinline__ bool tdq_writes_bitmap(const Args &a, const State &s, int L) {
   return a.hub_mask < 0 && L < kTdqBitmapLevels && ((s.fz >> ((L + 1) & 1)) & 1);
 }
@@ -715,10 +718,22 @@ __device__ __forceinline__ int queue_entry(const Args &a, const Smem<BS> &sm, co
 }
 
 // Top-down level L from the striped queue (small frontiers whose vertices all
-// have degree < queue_max_degree): one launch per level. A lane (or, for degree >=
-// t_wave, the whole wavefront) expands a frontier vertex; each unvisited
-// neighbour is claimed with an atomic OR on its visited word, and the
+// have degree < queue_max_degree): one launch per level. A group of lanes (or, for
+// degree >= t_wave, the whole wavefront) expands a frontier vertex; each
+// unvisited neighbour is claimed with an atomic OR on its visited word, and the
 // claiming lane writes its depth and stages it for the next queue.
+//
+// Such a level is one chain of memory round trips, two per four edges of a
+// lane, and with a lane per vertex a row of 17 takes ten of them. Sixteen lanes
+// per vertex, or as many as leave a lane of the grid to every entry's group,
+// take rows below t_wave in one step. It also spreads what a few hundred
+// vertices find over as many blocks: one block's found more than its stage
+// holds, and the next level was left to the three launches of the bitmap form.
+// A search with 1, 4, 8, 16 and 32 lanes per vertex: uniform, edge factor 8,
+// 200,000 vertices 130, 97, 92, 89 and 89 us; 3 million 268, 262, 250, 249 and
+// 252 (213 with this kernel's registers held to 8 wavefronts per SIMD);
+// R-MAT, 30,000 vertices 84, 79, 78, 78 and 78.
+constexpr int kTdqGroupLog = 4;
 template <int BS, bool COUNT>
 __device__ void tdq_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COUNT> &tl) {
   const int lane = lane_id();
@@ -787,8 +802,11 @@ __device__ void tdq_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<CO
   // vertices spreads over that many CUs instead of filling a few blocks.
   const long long wv = (long long)(threadIdx.x / kWave) * gridDim.x + blockIdx.x;
   const long long nt = (long long)gridDim.x * BS;
-  for (long long base = wv * kWave; base < total; base += nt) {
-    const long long k = base + lane;
+  int gs = kTdqGroupLog;
+  while (gs > 0 && ((long long)total << gs) > nt) --gs;
+  const int gl = lane & ((1 << gs) - 1);
+  for (long long base = (wv * kWave) >> gs; base < total; base += nt >> gs) {
+    const long long k = base + (lane >> gs);
     long long s = 0, e = 0;
     if (k < total) {
       int lo = 0, hi = kStripes - 1;
@@ -800,15 +818,20 @@ __device__ void tdq_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<CO
       const int v = qin[(long long)lo * a.qcap_s + (k - sm.qpre[lo])];
       s = a.off[v];
       e = a.off[v + 1];
-      tl.v(1);
-      if (e - s < a.t_wave) visit_range(s, e, 1);
+      tl.v(gl == 0 ? 1 : 0);
     }
-    unsigned long long wm = __ballot(k < total && e - s >= a.t_wave);
-    while (wm) {
+    const bool wide = e - s >= a.t_wave;
+    unsigned long long wm = __ballot(wide && gl == 0);
+    long long i0 = s + gl, i1 = wide ? s : e;
+    int stride = 1 << gs;
+    for (;;) {
+      visit_range(i0, i1, stride);
+      if (!wm) break;
       const int src = __ffsll((long long)wm) - 1;
       wm &= wm - 1;
-      const long long ss = __shfl(s, src), ee = __shfl(e, src);
-      visit_range(ss + lane, ee, kWave);
+      i0 = __shfl(s, src) + lane;
+      i1 = __shfl(e, src);
+      stride = kWave;
     }
   }
   wave_add_counts(sm, nf, mf, md);
@@ -1116,8 +1139,12 @@ __device__ __forceinline__ void run_phase(const Args &a, Smem<BS> &sm, long long
 // launch derives the next state itself.
 // HUB: the variant with the LDS hub table; COUNT: the variant that tallies
 // examined work (each only launched when configured).
+//
+// Held to 8 wavefronts per SIMD: with 7, which 82 SGPRs leave it, the grid has a
+// last wave of its own (uniform searches, 3 million vertices of edge factor 8
+// 250 us and 213, 10 million of edge factor 4 815 and 712).
 template <int BS, bool HUB, bool COUNT>
-__global__ __launch_bounds__(BS) void k_level(Args a, long long i) {
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_level(Args a, long long i) {
   __shared__ Smem<BS> sm;
   begin_launch<BS, COUNT>(a, sm, i, false);
   if (sm.S.done) return;

@@ -452,3 +452,24 @@ def test_first_neighbour_heads(oracle, n, per, keep):
         for bs, cw in ((64, 64), (512, 3), (1024, 1)):
             dg.configure(block_size=bs, bu_chunk_words=cw)
             _check(oracle, g, dg, int(np.argmin(np.where(deg > 0, deg, n))), f"heads n={n}/bs{bs}/cw{cw}")
+
+
+@pytest.mark.parametrize("fan", [1, 3, 4, 5, 16, 63, 65, 1000])
+@pytest.mark.parametrize("deg", [1, 15, 16, 31, 32, 70])
+def test_queue_level_groups(oracle, fan, deg):
+    """A root with `fan` children of degree `deg`, beside a star that keeps the
+    graph out of the one-block and low-degree forms: queue-driven levels whose
+    entries get 16, 8, ... 1 lanes, as the grid allows, and whole wavefronts."""
+    rng = np.random.default_rng(fan * 100 + deg)
+    leaves = fan * (deg - 1)
+    child = 1 + np.arange(fan)
+    hub = 1 + fan + leaves
+    n = hub + 1 + 20000
+    src = np.concatenate([np.zeros(fan, np.int64), np.repeat(child, deg - 1), np.full(20000, hub)])
+    dst = np.concatenate([child, 1 + fan + rng.permutation(leaves), hub + 1 + np.arange(20000)])
+    g = HostGraph.from_edges(n, src, dst)
+    with DeviceGraph(g) as dg:
+        for blocks in (0, 1, 5):
+            for launch in ("stream", "persistent"):
+                dg.configure(direction=L.DIR_TOPDOWN, grid_blocks=blocks, launch=LAUNCHES[launch])
+                _check(oracle, g, dg, 0, f"groups fan={fan} deg={deg} blocks={blocks}/{launch}")
