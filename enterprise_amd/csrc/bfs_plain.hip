@@ -1338,6 +1338,7 @@ void release(ent_graph *g) {
   ignore(hipFree(g->ctl));
   if (g->h_ctl) ignore(hipHostFree(g->h_ctl));
   if (g->h_mir) ignore(hipHostFree(g->h_mir));
+  if (g->narrow_flags) ignore(hipHostFree(g->narrow_flags));
   for (int b = 0; b < 2; ++b) {
     if (g->stage[b]) ignore(hipHostFree(g->stage[b]));
     if (g->stage_ev[b]) ignore(hipEventDestroy(g->stage_ev[b]));
@@ -1882,6 +1883,17 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
 
 // Per-handle search workspace: stream, events, depth, bitmaps, marks,
 // queues and control block.
+// Pinned memory of copy_depths: blocks and halves of this many vertices, for graphs
+// of kNarrowVertices to kNarrowEnd - 1. Smaller ones gain nothing (one block
+// searches them, and their copy is one short transfer); at 2^23, 32 MiB of
+// depths, C libraries hand out fresh pages for every array, and several threads
+// (copy_to_host) write those sooner than one: 12 million vertices 2,640 us
+// there, 2,770 here, but 8 million 1,430 and 900.
+constexpr int kNarrowBlock = 1 << 14;
+constexpr int64_t kNarrowHalf = 1 << 20;
+constexpr int64_t kNarrowVertices = 1 << 15;
+constexpr int64_t kNarrowEnd = 1 << 23;
+
 int alloc_workspace(ent_graph *g) {
   int rc;
   const int64_t n = g->n;
@@ -1910,6 +1922,21 @@ int alloc_workspace(ent_graph *g) {
   HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&g->h_mir), mir_bytes, hipHostMallocCoherent));
   std::memset(g->h_mir, 0, mir_bytes);
   HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void **>(&g->h_mir_dev), g->h_mir, 0));
+  if (n >= kNarrowVertices && n < kNarrowEnd) {  // pinned memory of copy_depths, which does without if there is none
+    const size_t flags = sizeof(unsigned) * size_t(2 * kNarrowHalf / kNarrowBlock);
+    const size_t bytes = size_t(std::min<int64_t>(n + 15, 2 * kNarrowHalf)) / 16 * 16;
+    void *h = nullptr, *d = nullptr;
+    if (hipHostMalloc(&h, flags + bytes, hipHostMallocCoherent) == hipSuccess) {
+      std::memset(h, 0, flags);
+      g->narrow_flags = static_cast<unsigned *>(h);
+      HIP_TRY(hipHostGetDevicePointer(&d, h, 0));
+      g->narrow_flags_dev = static_cast<unsigned *>(d);
+      g->narrow = static_cast<unsigned char *>(h) + flags;
+      g->narrow_dev = static_cast<unsigned char *>(d) + flags;
+    } else {
+      ignore(hipGetLastError());
+    }
+  }
   g->h_bad = reinterpret_cast<unsigned *>(g->h_mir + 2 * kHostStateWords);
   g->h_bad_dev = reinterpret_cast<unsigned *>(g->h_mir_dev + 2 * kHostStateWords);
   // The parent call's result sits behind the mirror's words.
@@ -2155,6 +2182,93 @@ int copy_to_host(ent_graph *g, void *dst, const void *src, size_t bytes) {
   return drain(nchunks - 1);
 }
 
+// Depths of a search of at most 255 levels as bytes (depth + 1, so 0 is -1) in
+// pinned memory, kNarrowBlock per block. Every block's stores are at the host
+// before its flag.
+__global__ __launch_bounds__(256) void k_narrow(const int *depth, long long n, unsigned char *out, unsigned *flags,
+                                                unsigned tag) {
+  const long long b0 = (long long)blockIdx.x * kNarrowBlock;
+#pragma unroll
+  for (int k = 0; k < kNarrowBlock / (256 * 16); ++k) {
+    const long long v = b0 + (k * 256 + int(threadIdx.x)) * 16;
+    if (v + 16 <= n) {
+      unsigned w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int4 d = *reinterpret_cast<const int4 *>(depth + v + 4 * j);
+        w[j] = unsigned(d.x + 1) | unsigned(d.y + 1) << 8 | unsigned(d.z + 1) << 16 | unsigned(d.w + 1) << 24;
+      }
+      *reinterpret_cast<uint4 *>(out + v) = make_uint4(w[0], w[1], w[2], w[3]);
+    } else {
+      for (long long x = v; x < n; ++x) out[x] = (unsigned char)(depth[x] + 1);
+    }
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(flags + blockIdx.x, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Waits for a flag of k_narrow; the stream is queried every 256 spins, so an
+// error or a drained stream ends the wait too.
+int wait_narrow(ent_graph *g, const unsigned *flag, unsigned tag) {
+  for (unsigned long spins = 0; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != tag; ++spins) {
+    if ((spins & 255) == 255) {
+      const hipError_t e = hipStreamQuery(g->stream);
+      if (e == hipSuccess && __atomic_load_n(flag, __ATOMIC_ACQUIRE) != tag)
+        return set_error(ENT_EINTERNAL, "depth copy ended without its flag");
+      if (e != hipSuccess && e != hipErrorNotReady)
+        return set_error(ENT_EDEVICE, "depth copy failed: %s", hipGetErrorString(e));
+    }
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+  }
+  return ENT_OK;
+}
+
+// The handle's depths, of a search of `levels` levels, into host memory.
+// Pageable destinations get them as bytes through pinned memory, widened here
+// block by block as they arrive: the runtime's own copy to pageable memory
+// moves four times the bytes and alternates transfer and host copy. The
+// transfer of 2^20 ints alone takes 83 us, of as many bytes 28, one thread's
+// widening 54. A search with its copy, before and now, R-MAT, edge factor 8:
+// 32,768 vertices 120 and 108 us, 2^18 196 and 143, 2^20 370 and 185, 2^22 870
+// and 436.
+int copy_depths(ent_graph *g, int32_t *dst, int levels) {
+  hipPointerAttribute_t attr;
+  bool pageable = true;
+  if (hipPointerGetAttributes(&attr, dst) == hipSuccess) pageable = attr.type == hipMemoryTypeUnregistered;
+  else ignore(hipGetLastError());  // pageable memory is unknown to the runtime
+  if (!g->narrow || !pageable || levels > 255)
+    return copy_to_host(g, dst, g->depth, sizeof(int32_t) * size_t(g->n));
+  const int64_t halves = (g->n + kNarrowHalf - 1) / kNarrowHalf;
+  unsigned tags[2];
+  auto half_of = [&](int64_t c) { return std::min(kNarrowHalf, g->n - c * kNarrowHalf); };
+  auto launch_half = [&](int64_t c) -> int {
+    const int b = int(c & 1);
+    if (++g->narrow_seq == 0) ++g->narrow_seq;
+    tags[b] = g->narrow_seq;
+    hipLaunchKernelGGL(k_narrow, dim3(unsigned((half_of(c) + kNarrowBlock - 1) / kNarrowBlock)), dim3(256), 0,
+                       g->stream, g->depth + c * kNarrowHalf, (long long)half_of(c), g->narrow_dev + b * kNarrowHalf,
+                       g->narrow_flags_dev + b * (kNarrowHalf / kNarrowBlock), tags[b]);
+    HIP_TRY(hipGetLastError());
+    return ENT_OK;
+  };
+  int rc = launch_half(0);
+  for (int64_t c = 0; c < halves && !rc; ++c) {
+    if (c + 1 < halves && (rc = launch_half(c + 1))) break;  // half c - 1 is drained
+    const int b = int(c & 1);
+    const unsigned char *src = g->narrow + b * kNarrowHalf;
+    const unsigned *flags = g->narrow_flags + b * (kNarrowHalf / kNarrowBlock);
+    for (int64_t v = 0; v < half_of(c) && !rc; v += kNarrowBlock) {
+      rc = wait_narrow(g, flags + v / kNarrowBlock, tags[b]);
+      if (!rc) widen_depths(src + v, dst + c * kNarrowHalf + v, std::min<int64_t>(kNarrowBlock, half_of(c) - v));
+    }
+  }
+  if (rc) ignore(hipStreamSynchronize(g->stream));  // nothing writes the halves any more
+  return rc;
+}
+
 // One single-source search from root into depth (device memory), with the
 // handle's lock held and ev0 already recorded; fills *st (may be NULL). t0 is
 // the start of the caller's host window.
@@ -2293,15 +2407,19 @@ int ent_get_config(const ent_graph *g, ent_bfs_config *cfg) {
 
 int32_t *ent_depth_device_ptr(ent_graph *g) { return g ? g->depth : nullptr; }
 
+static int search_on_handle(ent_graph *g, int32_t root, int32_t *depth, ent_stats *st) {
+  const auto t0 = std::chrono::steady_clock::now();
+  HIP_TRY(hipSetDevice(g->device));
+  HIP_TRY(hipEventRecord(g->ev0, g->stream));
+  return ent::search_locked(g, root, depth, st, t0);
+}
+
 int ent_bfs_device(ent_graph *g, int32_t root, int32_t *depth_dev, ent_stats *st) {
   clear_error();
   if (!g) return set_error(ENT_EINVAL, "NULL graph");
   if (root < 0 || root >= g->n) return set_error(ENT_EINVAL, "root %d outside [0, %lld)", root, (long long)g->n);
   std::lock_guard<std::mutex> lk(g->mu);
-  const auto t0 = std::chrono::steady_clock::now();
-  HIP_TRY(hipSetDevice(g->device));
-  HIP_TRY(hipEventRecord(g->ev0, g->stream));
-  return ent::search_locked(g, root, depth_dev ? depth_dev : g->depth, st, t0);
+  return search_on_handle(g, root, depth_dev ? depth_dev : g->depth, st);
 }
 
 int ent_last_device_ms(ent_graph *g, double *ms) {
@@ -2317,9 +2435,15 @@ int ent_last_device_ms(ent_graph *g, double *ms) {
 }
 
 int ent_bfs(ent_graph *g, int32_t root, int32_t *depth_host, ent_stats *st) {
-  int rc = ent_bfs_device(g, root, nullptr, st);
+  clear_error();
+  if (!g) return set_error(ENT_EINVAL, "NULL graph");
+  if (root < 0 || root >= g->n) return set_error(ENT_EINVAL, "root %d outside [0, %lld)", root, (long long)g->n);
+  std::lock_guard<std::mutex> lk(g->mu);
+  ent_stats own;
+  if (!st) st = &own;
+  const int rc = search_on_handle(g, root, g->depth, st);
   if (rc || !depth_host) return rc;
-  return ent_copy_to_host(g, g->depth, depth_host, g->n);
+  return ent::copy_depths(g, depth_host, st->levels);
 }
 
 int ent_copy_to_host(ent_graph *g, const int32_t *src_dev, int32_t *dst_host, int64_t count) {

@@ -46,6 +46,9 @@ void parallel_for(int64_t n, int64_t grain, F &&fn) {
   for (auto &t : pool) t.join();
 }
 
+// dst[i] = src[i] - 1 for i < n.
+void widen_depths(const unsigned char *src, int32_t *dst, int64_t n);
+
 // SplitMix64 (Steele, Lea, Flood 2014): a bijective 64-bit mixer. Used both as
 // a sequential stream (state += golden gamma) and as a hash of (seed, index).
 static inline uint64_t mix64(uint64_t z) {

@@ -79,6 +79,9 @@ struct ent_graph {
   int trace_launches = 0;  // launches recorded by the last counting search
   void *stage[2] = {nullptr, nullptr};  // pinned staging for copies to pageable host memory
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  unsigned *narrow_flags = nullptr, *narrow_flags_dev = nullptr;  // pinned: copy_depths' flags, then its bytes
+  unsigned char *narrow = nullptr, *narrow_dev = nullptr;
+  unsigned narrow_seq = 0;  // tag of the latest k_narrow launch
   unsigned long long *visited = nullptr;
   unsigned long long *front[2] = {nullptr, nullptr};
   unsigned char *mark = nullptr;

@@ -45,6 +45,13 @@ int host_threads() {
   return hc > 16 ? 16 : int(hc);
 }
 
+#if defined(__x86_64__)
+__attribute__((target_clones("avx2", "default")))
+#endif
+void widen_depths(const unsigned char *src, int32_t *dst, int64_t n) {
+  for (int64_t i = 0; i < n; ++i) dst[i] = int32_t(src[i]) - 1;
+}
+
 namespace {
 
 template <class T>

@@ -1,6 +1,7 @@
 """GPU parity of the single-source BFS (through the C ABI) against the CPU
 oracle: bit-exact int32 depth arrays and exact reached-vertex / reached-edge
 counts, for every direction policy and launch form."""
+import ctypes as C
 import sys
 
 import numpy as np
@@ -473,3 +474,33 @@ def test_queue_level_groups(oracle, fan, deg):
             for launch in ("stream", "persistent"):
                 dg.configure(direction=L.DIR_TOPDOWN, grid_blocks=blocks, launch=LAUNCHES[launch])
                 _check(oracle, g, dg, 0, f"groups fan={fan} deg={deg} blocks={blocks}/{launch}")
+
+
+@pytest.mark.parametrize("n,levels", [(32767, 3), (32768, 3), (32768 + 5, 254), (40000, 255), (40001, 256), (40002, 257),
+                                      (1 << 20, 3), ((1 << 20) + 1, 255), ((1 << 21) + 16387, 9), ((1 << 23) - 1, 3),
+                                      (1 << 23, 3)])
+def test_depths_to_host(n, levels):
+    """Depths copied to pageable and to pinned host memory equal the device's,
+    for whole and ragged blocks, one to three halves, more halves than there are
+    buffers, and either side of the level count that a byte holds. A path of
+    `levels` vertices, its last one a hub that keeps other forms out."""
+    path = np.arange(levels - 2)
+    leaves = np.arange(levels, n - 7)
+    src = np.concatenate([path, np.full(leaves.size, levels - 2)])
+    dst = np.concatenate([path + 1, leaves])
+    g = HostGraph.from_edges(n, src, dst)
+    want = np.full(n, -1, dtype=np.int32)
+    want[: levels - 1] = np.arange(levels - 1)
+    want[leaves] = levels - 1
+    with DeviceGraph(g) as dg:
+        for rep in range(2):
+            got, st = dg.bfs(0)
+            assert st["levels"] == levels
+            assert np.array_equal(got, want), (n, levels, rep)
+            back, _ = dg.bfs(levels - 2)
+            assert back[levels - 2] == 0 and back[0] == levels - 2 and np.all(back[leaves] == 1)
+            assert back[n - 1] == -1
+        import torch
+        pinned = torch.empty(n, dtype=torch.int32, pin_memory=True)
+        L.check(L.lib().ent_bfs(dg.handle, 0, C.cast(pinned.data_ptr(), L.i32p), None))
+        assert np.array_equal(pinned.numpy(), want)
