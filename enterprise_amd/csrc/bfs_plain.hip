@@ -73,6 +73,9 @@ constexpr int kStripeU64 = 16;   // 128 B between stripes
 
 // Per-stripe counter words.
 enum : int { K_NF = 0, K_MF = 1, K_QN = 2, K_MAXDEG = 3, K_QOVF = 4 };
+// A queue-driven level with a vertex of this degree or more may deal out its
+// edges (tdq_flat); a wavefront takes rows below it in one step.
+constexpr unsigned long long kFlatDegree = 256;
 constexpr int kQStage = 512;  // queue entries one block stages in LDS per phase
 
 struct Counters {
@@ -104,6 +107,7 @@ struct State {
   int pending;   // phase to run after PH_REBUILD
   int search;    // the host's search number, carried from launch to launch
   int fz;        // bit p: front[p] is all zero (a queue-driven level may OR its output into it)
+  int flat;      // a queue-driven level deals out its edges (tdq_flat)
   unsigned int qn[kStripes];  // entries per queue stripe
 };
 // Leading words of State the host reads after a search (everything before
@@ -187,6 +191,7 @@ struct Args {
   int chunk_words;
   int qcap_s;   // entries per queue stripe
   int q_small;  // largest frontier expanded from the queue
+  int flat_n, flat_m;  // largest one, and its edges, that tdq_flat expands (0: none)
   int q_maxdeg; // queue-driven levels need every frontier degree below this
   // LDS hub cache (hub_mask = entries - 1, or -1 when off): hub_slot[s] is
   // the highest-degree vertex v with v & hub_mask == s (or -1), hub_tag[s]
@@ -717,6 +722,38 @@ __device__ __forceinline__ int queue_entry(const Args &a, const Smem<BS> &sm, co
   return qin[(long long)lo * a.qcap_s + (k - sm.qpre[lo])];
 }
 
+// Claims the unvisited among four edges' ends u for level L + 1. The levels
+// expanded here are short latency chains, so each goes straight to the claiming
+// atomic (no visited-bit load first) and its row offsets are loaded alongside:
+// adjacency, then atomics and offsets together, two memory round trips a step.
+template <int BS>
+__device__ __forceinline__ void tdq_claim(const Args &a, Smem<BS> &sm, int L, const int (&u)[4], const bool (&in)[4],
+                                          unsigned long long &nf, unsigned long long &mf, unsigned &md) {
+  unsigned long long old[4];
+  long long us[4], ue[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    old[j] = in[j] ? atomicOr(a.visited + (u[j] >> 6), 1ull << (u[j] & 63)) : ~0ull;
+    us[j] = in[j] ? a.off[u[j]] : 0;
+    ue[j] = in[j] ? a.off[u[j] + 1] : 0;
+  }
+  // Every atomic result is read before the first depth store: a wait
+  // for a result issued behind a store would wait for the store too.
+  bool won[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) won[j] = !(old[j] & (1ull << (u[j] & 63)));
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (won[j]) {
+      const long long d = ue[j] - us[j];
+      a.depth[u[j]] = L + 1;
+      nf += 1;
+      mf += (unsigned long long)d;
+      md = deg_max(md, d);
+      stage_push(sm, u[j]);
+    }
+}
+
 // Top-down level L from the striped queue (small frontiers whose vertices all
 // have degree < queue_max_degree): one launch per level. A group of lanes (or, for
 // degree >= t_wave, the whole wavefront) expands a frontier vertex; each
@@ -734,7 +771,65 @@ __device__ __forceinline__ int queue_entry(const Args &a, const Smem<BS> &sm, co
 // 252 (213 with this kernel's registers held to 8 wavefronts per SIMD);
 // R-MAT, 30,000 vertices 84, 79, 78, 78 and 78.
 constexpr int kTdqGroupLog = 4;
+// The same for at most flat_n frontier vertices with at most flat_m edges, one of
+// them a hub: lane k of the grid takes edges k, k + lanes, ... of the frontier's
+// rows laid end to end, whose starts every block sums up for itself. A level
+// whose hubs rule out whole rows per wavefront otherwise marks bytes in one
+// launch and finds them by a sweep in another, both over all vertices, although
+// its frontier is a few hubs: R-MAT, 2^24 vertices, 7 vertices with 31,157 edges
+// took 50 and 42 us. Searches before and now: R-MAT, edge factor 16, 20,000
+// vertices 66 and 58 us, 2^18 75 and 70, 2^20 96 and 86, 2^22 137 and 119, 2^24
+// 485 and 407 from one root, 397 and 316 from another. Testing the visited bits
+// before the atomics costs up to 10% (2^19 84 and 93).
 template <int BS, bool COUNT>
+__device__ void tdq_flat(const Args &a, Smem<BS> &sm, int L, int total, Tally<COUNT> &tl, unsigned long long &nf,
+                         unsigned long long &mf, unsigned &md) {
+  long long *start = reinterpret_cast<long long *>(&sm.cand[0][0]);  // row starts
+  int *pre = &sm.excl[0][0];                                         // edges before each row
+  int *wsum = reinterpret_cast<int *>(&sm.found[0][0]);
+  const int t = threadIdx.x;
+  int d = 0;
+  if (t < total) {
+    const int v = queue_entry(a, sm, a.qbuf[L & 1], t);
+    const long long s = a.off[v];
+    d = int(a.off[v + 1] - s);
+    start[t] = s;
+    tl.v(blockIdx.x == 0 ? 1 : 0);
+  }
+  const int incl = wave_incl_scan(d);
+  if (lane_id() == kWave - 1) wsum[t / kWave] = incl;
+  __syncthreads();
+  int base = 0, edges = 0;
+#pragma unroll
+  for (int w = 0; w < BS / kWave; ++w) {
+    if (w == t / kWave) base = edges;
+    edges += wsum[w];
+  }
+  pre[t] = base + incl - d;
+  __syncthreads();
+  const int nt = int(gridDim.x) * BS;
+  for (int i = int(blockIdx.x) * BS + t; i < edges; i += 4 * nt) {
+    int u[4];
+    bool in[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int k = i + j * nt;
+      in[j] = k < edges;
+      int lo = 0, hi = total - 1;
+      if (in[j])
+        while (lo < hi) {
+          const int mid = (lo + hi + 1) >> 1;
+          if (pre[mid] <= k) lo = mid;
+          else hi = mid - 1;
+        }
+      u[j] = in[j] ? a.adj[start[lo] + (k - pre[lo])] : 0;
+      tl.e(in[j] ? 1 : 0);
+    }
+    tdq_claim(a, sm, L, u, in, nf, mf, md);
+  }
+}
+
+template <int BS, bool COUNT, bool FLAT>
 __device__ void tdq_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COUNT> &tl) {
   const int lane = lane_id();
   if (threadIdx.x < kWave) {
@@ -756,17 +851,18 @@ __device__ void tdq_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<CO
   }
   unsigned long long nf = 0, mf = 0;
   unsigned md = 0;
+  if (FLAT && sm.S.flat) {
+    tdq_flat<BS, COUNT>(a, sm, L, total, tl, nf, mf, md);
+    wave_add_counts(sm, nf, mf, md);
+    add_counts(a, sm, slot, (L + 1) & 1, tdq_writes_bitmap(a, sm.S, L) ? a.front[(L + 1) & 1] : nullptr);
+    return;
+  }
   // Claims the unvisited among adj[i], i = i0, i0 + stride, ... < e, four
-  // edges per step. The levels expanded here are short latency chains, so
-  // each neighbour goes straight to the claiming atomic (no visited-bit load
-  // first) and its row offsets are loaded alongside: adjacency, then atomics
-  // and offsets together, two memory round trips per step.
+  // edges per step.
   auto visit_range = [&](long long i0, long long e, int stride) {
     for (long long i = i0; i < e; i += 4LL * stride) {
       int u[4];
       bool in[4];
-      unsigned long long old[4];
-      long long us[4], ue[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const long long ij = i + (long long)j * stride;
@@ -774,27 +870,7 @@ __device__ void tdq_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<CO
         u[j] = in[j] ? a.adj[ij] : 0;
         tl.e(in[j] ? 1 : 0);
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        old[j] = in[j] ? atomicOr(a.visited + (u[j] >> 6), 1ull << (u[j] & 63)) : ~0ull;
-        us[j] = in[j] ? a.off[u[j]] : 0;
-        ue[j] = in[j] ? a.off[u[j] + 1] : 0;
-      }
-      // Every atomic result is read before the first depth store: a wait
-      // for a result issued behind a store would wait for the store too.
-      bool won[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) won[j] = !(old[j] & (1ull << (u[j] & 63)));
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (won[j]) {
-          const long long d = ue[j] - us[j];
-          a.depth[u[j]] = L + 1;
-          nf += 1;
-          mf += (unsigned long long)d;
-          md = deg_max(md, d);
-          stage_push(sm, u[j]);
-        }
+      tdq_claim(a, sm, L, u, in, nf, mf, md);
     }
   };
   // 64-entry chunks go to wavefronts of consecutive blocks (wavefront j of
@@ -933,7 +1009,11 @@ __device__ __forceinline__ void next_state(const Args &a, State &s, const unsign
   if (next_bu) {
     s.phase = bm ? PH_BU : PH_REBUILD;
     s.pending = PH_BU;
-  } else if (q && nf <= (unsigned long long)a.q_small && tot[K_MAXDEG] < (unsigned long long)a.q_maxdeg) {
+  } else if (const bool flat = tot[K_MAXDEG] >= kFlatDegree && nf <= (unsigned long long)a.flat_n &&
+                               mf <= (unsigned long long)a.flat_m;
+             q && nf <= (unsigned long long)a.q_small &&
+             (flat || tot[K_MAXDEG] < (unsigned long long)a.q_maxdeg)) {
+    s.flat = flat;
     s.phase = PH_TDQ;
   } else {
     s.phase = bm ? PH_TD : PH_REBUILD;
@@ -1107,7 +1187,7 @@ __global__ __launch_bounds__(BS) void k_init(Args a, int root, int first_bu, int
   }
 }
 
-template <int BS, bool HUB, bool COUNT, bool HEAD = false>
+template <int BS, bool HUB, bool COUNT, bool FLAT, bool HEAD>
 __device__ __forceinline__ void run_phase(const Args &a, Smem<BS> &sm, long long i) {
   const int L = sm.S.level;
   const int slot = int(i % 3);
@@ -1119,7 +1199,7 @@ __device__ __forceinline__ void run_phase(const Args &a, Smem<BS> &sm, long long
       break;
     case PH_BU: bu_phase<BS, HUB, COUNT, HEAD>(a, sm, L, slot, tl); break;
     case PH_INSPECT: inspect_phase<BS, HUB, COUNT>(a, sm, L, slot, tl); break;
-    case PH_TDQ: tdq_phase<BS, COUNT>(a, sm, L, slot, tl); break;
+    case PH_TDQ: tdq_phase<BS, COUNT, FLAT>(a, sm, L, slot, tl); break;
     default: rebuild_phase<BS, HUB, COUNT>(a, sm, L, tl); break;
   }
   if (COUNT) {  // one atomic per wavefront and counter, on the block's stripe
@@ -1148,19 +1228,20 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_
   __shared__ Smem<BS> sm;
   begin_launch<BS, COUNT>(a, sm, i, false);
   if (sm.S.done) return;
-  run_phase<BS, HUB, COUNT>(a, sm, i);
+  run_phase<BS, HUB, COUNT, COUNT && !HUB, false>(a, sm, i);
 }
 
-// The same with heads in its bottom-up phase, for graphs that have them. That
+// The same for skewed graphs: its queue-driven levels deal out the edges of hubs,
+// and with HEAD its bottom-up levels read heads, for graphs that have them. That
 // phase wants 68 VGPRs and 88 SGPRs, which leaves 7 wavefronts per SIMD and a
 // grid of 8 blocks per CU with a last wave of its own (a search of 2^22 vertices
 // then takes 174 us); held to 8, at 7 spilled SGPRs, it is 138.
-template <int BS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_level_heads(Args a, long long i) {
+template <int BS, bool HEAD>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_level_skew(Args a, long long i) {
   __shared__ Smem<BS> sm;
   begin_launch<BS, false>(a, sm, i, false);
   if (sm.S.done) return;
-  run_phase<BS, false, false, true>(a, sm, i);
+  run_phase<BS, false, false, true, HEAD>(a, sm, i);
 }
 
 // A small graph's search in one block (ent_tiny.h). The first wavefront
@@ -1272,7 +1353,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
   for (long long i = 0;; ++i) {
     begin_launch<BS, COUNT>(a, sm, i, true);
     if (sm.S.done || sm.S.error) break;
-    run_phase<BS, HUB, COUNT>(a, sm, i);
+    run_phase<BS, HUB, COUNT, false, false>(a, sm, i);
     const bool ok = grid_sync(&a.ctl->sync, 400000000ull);
     if (threadIdx.x == 0) {
       if (!ok) {
@@ -1504,6 +1585,12 @@ LevelShape level_shape(const ent_graph *g) {
   return s;
 }
 
+// Limits of tdq_flat: beyond 2^18 edges the atomics of a level cost more than the
+// two sweeps (2^16 loses 20% of 2^22 and 2^24 searches, 2^20 gains nothing), and
+// beyond four a lane a small grid's stages overflow. Graphs without hubs have no
+// such levels and keep the kernel without it.
+constexpr int64_t kFlatEdges = 1 << 18;
+constexpr int64_t kFlatPer = 4;
 Args make_args(ent_graph *g, int *depth) {
   Args a{};
   a.off = g->off;
@@ -1524,6 +1611,10 @@ Args make_args(ent_graph *g, int *depth) {
   if (g->cfg.queue_small < 0) a.q_small = 0;
   else if (g->cfg.queue_small > 0) a.q_small = int(std::min<int64_t>(g->cfg.queue_small, int64_t(kStripes) * g->qcap_s / 2));
   else a.q_small = int(std::min<int64_t>(std::max<int64_t>(4096, g->n / 256), int64_t(kStripes) * g->qcap_s / 2));
+  const bool flat = g->store->skewed && g->hub_slots == 0 && g->cfg.launch != ENT_LAUNCH_PERSISTENT &&
+                    g->cfg.queue_max_degree == 0;
+  a.flat_n = flat ? std::min(g->cfg.block_size, 256) : 0;
+  a.flat_m = int(std::min<int64_t>(kFlatEdges, kFlatPer * int64_t(level_shape(g).grid) * g->cfg.block_size));
   a.q_maxdeg = g->cfg.queue_max_degree > 0 ? g->cfg.queue_max_degree : g->cfg.t_block;
   a.ctl = g->ctl;
   a.hmir = g->h_mir_dev;
@@ -1564,21 +1655,22 @@ KernelSet kernel_set_of() {
 }
 
 template <int BS>
-KernelSet kernel_set(bool hub, bool count, bool head) {
+KernelSet kernel_set(bool hub, bool count, bool skew, bool head) {
   if (count) return hub ? kernel_set_of<BS, true, true>() : kernel_set_of<BS, false, true>();
   if (hub) return kernel_set_of<BS, true, false>();
   KernelSet ks = kernel_set_of<BS, false, false>();
-  if (head) ks.level = reinterpret_cast<const void *>(&k_level_heads<BS>);
+  if (head) ks.level = reinterpret_cast<const void *>(&k_level_skew<BS, true>);
+  else if (skew) ks.level = reinterpret_cast<const void *>(&k_level_skew<BS, false>);
   return ks;
 }
 
-KernelSet kernels_for(int bs, bool hub, bool count, bool head) {
+KernelSet kernels_for(int bs, bool hub, bool count, bool skew, bool head) {
   switch (bs) {
-    case 64: return kernel_set<64>(hub, count, head);
-    case 128: return kernel_set<128>(hub, count, head);
-    case 512: return kernel_set<512>(hub, count, head);
-    case 1024: return kernel_set<1024>(hub, count, head);
-    default: return kernel_set<256>(hub, count, head);
+    case 64: return kernel_set<64>(hub, count, skew, head);
+    case 128: return kernel_set<128>(hub, count, skew, head);
+    case 512: return kernel_set<512>(hub, count, skew, head);
+    case 1024: return kernel_set<1024>(hub, count, skew, head);
+    default: return kernel_set<256>(hub, count, skew, head);
   }
 }
 
@@ -1756,7 +1848,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
   int rc = build_lists(g);
   if (rc) return rc;
   const bool count = cfg.count_examined != 0;
-  const KernelSet ks = kernels_for(cfg.block_size, g->hub_slots > 0, count, g->store->head != nullptr);
+  const KernelSet ks = kernels_for(cfg.block_size, g->hub_slots > 0, count, g->store->skewed, g->store->head != nullptr);
   if (count) HIP_TRY(hipMemsetAsync(g->ctl->exam, 0, sizeof(g->ctl->exam), g->stream));
   if (ks.smem + hub_lds_bytes(cfg) > 65536)
     return set_error(ENT_EINVAL, "hub_cache %d with block_size %d needs %zu bytes of LDS per block (64 KiB max)",
@@ -2018,14 +2110,14 @@ int ent_graph_upload_ex(const int64_t *beg_pos, const int32_t *adj, int64_t n, i
 
 namespace ent {
 
-// Graphs that get heads (bu_phase): only skewed ones, whose first neighbours are
-// hubs. Uniform random graphs of edge factor 8 have a largest degree of 2-3
+// A graph is skewed if its largest degree is kSkew times the mean or more. Only
+// such graphs get heads (bu_phase), as their first neighbours are hubs. Uniform random graphs of edge factor 8 have a largest degree of 2-3
 // times the mean and lose by them (200,000 vertices 132 us without, 136 with);
 // R-MAT ones have 30 times and more at every size. Below 2^19 vertices a level
 // is launch-bound (2^18: 74.5 us without, 75.2 with; 2^19 91.8 and 90.2).
 // Rows in the caller's order find less with their first neighbour: 2^21
 // vertices 131 and 133 us, 2^22 160 and 152, 2^23 559 and 419.
-constexpr int kHeadSkew = 16;
+constexpr int kSkew = 16;
 constexpr int64_t kHeadVertices = 1 << 19;
 constexpr int64_t kHeadVerticesKept = 1 << 22;
 
@@ -2113,8 +2205,8 @@ int upload_graph(const int64_t *beg_pos, const int32_t *adj, bool adj_on_device,
   UP_TRY(hipMemcpy(g->nzmask, nz.data(), sizeof(unsigned long long) * size_t(g->nwords), hipMemcpyHostToDevice));
   rc = alloc_workspace(g);
   if (!rc && !(flags & ENT_UPLOAD_KEEP_ORDER)) rc = order_rows_by_degree(g);
-  const bool heads = n >= (flags & ENT_UPLOAD_KEEP_ORDER ? kHeadVerticesKept : kHeadVertices) &&
-                     g->store->max_deg / kHeadSkew >= m / n;
+  g->store->skewed = g->store->max_deg / kSkew >= m / n;
+  const bool heads = g->store->skewed && n >= (flags & ENT_UPLOAD_KEEP_ORDER ? kHeadVerticesKept : kHeadVertices);
   if (!rc && heads && device_malloc(device, reinterpret_cast<void **>(&g->store->head), sizeof(int) * size_t(n)) != hipSuccess) {
     g->store->head = nullptr;  // no room: the levels scan the rows alone
     ignore(hipGetLastError());

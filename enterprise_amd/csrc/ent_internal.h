@@ -31,6 +31,7 @@ struct GraphStore {
   unsigned long long *nzmask = nullptr;  // bit v: degree(v) > 0
   std::vector<int32_t> h_deg;            // host copy of degrees (for the static lists)
   int32_t max_deg = 0;
+  bool skewed = false;                   // largest degree far above the mean (kSkew)
   int *head = nullptr;                   // first neighbour of each row, or null (bfs_plain.hip)
   std::mutex rows_mu;                    // guards rows, rows_width (ent_deep.h)
   int *rows = nullptr;

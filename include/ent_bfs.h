@@ -90,7 +90,8 @@ typedef struct ent_bfs_config {
                               (expander.cuh:96-109, :172-185) */
   int32_t queue_max_degree; /* a frontier goes through the queue only if all
                                its vertices have degree below this
-                               (0 = t_block) */
+                               (0 = t_block, or small frontiers of skewed
+                               graphs whatever their degrees) */
   int32_t count_examined;   /* 1: run the kernel variant that counts the
                                work it examines (ent_stats.examined_*);
                                for measurement, not speed */

@@ -504,3 +504,33 @@ def test_depths_to_host(n, levels):
         pinned = torch.empty(n, dtype=torch.int32, pin_memory=True)
         L.check(L.lib().ent_bfs(dg.handle, 0, C.cast(pinned.data_ptr(), L.i32p), None))
         assert np.array_equal(pinned.numpy(), want)
+
+
+@pytest.mark.parametrize("fan", [1, 2, 255, 256, 257])
+@pytest.mark.parametrize("deg", [255, 256, 1030])
+def test_queue_level_hubs(oracle, fan, deg):
+    """A root with `fan` children, one of degree `deg` and the others of degree 1
+    to `deg`, whose leaves partly coincide, beside a larger star: frontiers on
+    either side of the sizes and degrees whose edges are dealt out over the grid,
+    with the usual grid and with ones of a few blocks."""
+    rng = np.random.default_rng(fan * 10 + deg)
+    child = 1 + np.arange(fan)
+    degs = rng.integers(1, deg + 1, fan)
+    degs[fan // 2] = deg
+    if fan >= 255 and deg == 1030:
+        degs[:] = deg  # 262,650 edges and more
+    leaves = np.arange(1 + fan, 1 + fan + 4 * deg)
+    hub = int(leaves[-1]) + 1
+    n = hub + 1 + 30000
+    src = np.concatenate([np.zeros(fan, np.int64)] + [np.full(d - 1, c) for c, d in zip(child, degs)]
+                         + [np.full(30000, hub)])
+    dst = np.concatenate([child] + [rng.choice(leaves, d - 1, replace=False) for d in degs]
+                         + [hub + 1 + np.arange(30000)])
+    g = HostGraph.from_edges(n, src, dst)
+    with DeviceGraph(g) as dg:
+        for bs, blocks in ((256, 0), (256, 1), (64, 3), (1024, 2)):
+            for launch in ("stream", "levels"):
+                for count in (0, 1):
+                    dg.configure(direction=L.DIR_AUTO if blocks else L.DIR_TOPDOWN, block_size=bs, grid_blocks=blocks,
+                                 launch=LAUNCHES[launch], count_examined=count)
+                    _check(oracle, g, dg, 0, f"hubs fan={fan} deg={deg} bs={bs} blocks={blocks}/{launch}/{count}")
