@@ -28,7 +28,9 @@
 //    pass turns marks into the next frontier bitmap and queue, the depth
 //    writes and the frontier counts, one wavefront per bitmap word.
 //  - Small frontiers expand straight from the queue in one launch per level,
-//    claiming vertices with an atomic OR on their visited word.
+//    claiming vertices with an atomic OR on their visited word; small graphs
+//    are searched by one block, and low-degree graphs go over to several
+//    levels per launch (bfs_deep.hip).
 //  - Bottom-up owns whole bitmap words per wavefront, so it updates visited,
 //    next frontier and depth without atomics.
 //  - Launch i derives its phase from the state and the finished counters of
@@ -37,10 +39,13 @@
 //    cache lines so few blocks contend for one address.
 //  - Two kernel variants are launched only when configured: the LDS hub
 //    table (HUB) and the examined-work tally (COUNT). The default variant
-//    carries neither, which keeps its registers and code at their minimum.
+//    carries neither, which keeps its registers and code at their minimum;
+//    skewed graphs have one of their own (k_level_skew), with what pays only
+//    where there are hubs.
 //
 // Device state (HBM, sized at upload):
-//   off int64[n+1], adj int32[m], nzmask u64[W] (degree > 0), W = ceil(n/64)
+//   off int64[n+1], adj int32[m], nzmask u64[W] (degree > 0), W = ceil(n/64),
+//   head int32[n] (first neighbours; large skewed graphs)
 //   hub_block int32[] (t_block <= degree < t_grid), piece_v/piece_k int32[]
 //   (degree >= t_grid, split into `piece`-edge pieces)
 //   depth int32[n], visited u64[W], front[2] u64[W], mark u8[n],
@@ -754,26 +759,10 @@ __device__ __forceinline__ void tdq_claim(const Args &a, Smem<BS> &sm, int L, co
     }
 }
 
-// Top-down level L from the striped queue (small frontiers whose vertices all
-// have degree < queue_max_degree): one launch per level. A group of lanes (or, for
-// degree >= t_wave, the whole wavefront) expands a frontier vertex; each
-// unvisited neighbour is claimed with an atomic OR on its visited word, and the
-// claiming lane writes its depth and stages it for the next queue.
-//
-// Such a level is one chain of memory round trips, two per four edges of a
-// lane, and with a lane per vertex a row of 17 takes ten of them. Sixteen lanes
-// per vertex, or as many as leave a lane of the grid to every entry's group,
-// take rows below t_wave in one step. It also spreads what a few hundred
-// vertices find over as many blocks: one block's found more than its stage
-// holds, and the next level was left to the three launches of the bitmap form.
-// A search with 1, 4, 8, 16 and 32 lanes per vertex: uniform, edge factor 8,
-// 200,000 vertices 130, 97, 92, 89 and 89 us; 3 million 268, 262, 250, 249 and
-// 252 (213 with this kernel's registers held to 8 wavefronts per SIMD);
-// R-MAT, 30,000 vertices 84, 79, 78, 78 and 78.
-constexpr int kTdqGroupLog = 4;
-// The same for at most flat_n frontier vertices with at most flat_m edges, one of
-// them a hub: lane k of the grid takes edges k, k + lanes, ... of the frontier's
-// rows laid end to end, whose starts every block sums up for itself. A level
+// A queue-driven level of at most flat_n frontier vertices with at most flat_m
+// edges, one of them a hub (kFlatDegree): lane k of the grid takes edges k,
+// k + lanes, ... of the frontier's rows laid end to end, whose starts every block
+// sums up for itself. A level
 // whose hubs rule out whole rows per wavefront otherwise marks bytes in one
 // launch and finds them by a sweep in another, both over all vertices, although
 // its frontier is a few hubs: R-MAT, 2^24 vertices, 7 vertices with 31,157 edges
@@ -829,6 +818,23 @@ __device__ void tdq_flat(const Args &a, Smem<BS> &sm, int L, int total, Tally<CO
   }
 }
 
+// Top-down level L from the striped queue (small frontiers whose vertices all
+// have degree < queue_max_degree): one launch per level. A group of lanes (or, for
+// degree >= t_wave, the whole wavefront) expands a frontier vertex; each
+// unvisited neighbour is claimed with an atomic OR on its visited word, and the
+// claiming lane writes its depth and stages it for the next queue.
+//
+// Such a level is one chain of memory round trips, two per four edges of a
+// lane, and with a lane per vertex a row of 17 takes ten of them. Sixteen lanes
+// per vertex, or as many as leave a lane of the grid to every entry's group,
+// take rows below t_wave in one step. It also spreads what a few hundred
+// vertices find over as many blocks: one block's found more than its stage
+// holds, and the next level was left to the three launches of the bitmap form.
+// A search with 1, 4, 8, 16 and 32 lanes per vertex: uniform, edge factor 8,
+// 200,000 vertices 130, 97, 92, 89 and 89 us; 3 million 268, 262, 250, 249 and
+// 252 (213 with this kernel's registers held to 8 wavefronts per SIMD);
+// R-MAT, 30,000 vertices 84, 79, 78, 78 and 78.
+constexpr int kTdqGroupLog = 4;
 template <int BS, bool COUNT, bool FLAT>
 __device__ void tdq_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COUNT> &tl) {
   const int lane = lane_id();
@@ -2117,7 +2123,7 @@ namespace ent {
 // is launch-bound (2^18: 74.5 us without, 75.2 with; 2^19 91.8 and 90.2).
 // Rows in the caller's order find less with their first neighbour: 2^21
 // vertices 131 and 133 us, 2^22 160 and 152, 2^23 559 and 419.
-constexpr int kSkew = 16;
+constexpr int64_t kSkew = 16;
 constexpr int64_t kHeadVertices = 1 << 19;
 constexpr int64_t kHeadVerticesKept = 1 << 22;
 
@@ -2205,7 +2211,7 @@ int upload_graph(const int64_t *beg_pos, const int32_t *adj, bool adj_on_device,
   UP_TRY(hipMemcpy(g->nzmask, nz.data(), sizeof(unsigned long long) * size_t(g->nwords), hipMemcpyHostToDevice));
   rc = alloc_workspace(g);
   if (!rc && !(flags & ENT_UPLOAD_KEEP_ORDER)) rc = order_rows_by_degree(g);
-  g->store->skewed = g->store->max_deg / kSkew >= m / n;
+  g->store->skewed = int64_t(g->store->max_deg) * n >= kSkew * m;
   const bool heads = g->store->skewed && n >= (flags & ENT_UPLOAD_KEEP_ORDER ? kHeadVerticesKept : kHeadVertices);
   if (!rc && heads && device_malloc(device, reinterpret_cast<void **>(&g->store->head), sizeof(int) * size_t(n)) != hipSuccess) {
     g->store->head = nullptr;  // no room: the levels scan the rows alone
