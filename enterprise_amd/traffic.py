@@ -20,7 +20,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 # Kernels of one search, by mode: (kernels counted, kernel that starts a search).
 SEARCH_KERNELS = {
-    "plain": (("ent::k_init", "ent::k_level"), "ent::k_init"),
+    "plain": (("ent::k_init", "ent::k_level", "ent::k_level_skew"), "ent::k_init"),
     "batch": (("ent::k_binit_zero", "ent::k_binit_src", "ent::k_blevel", "ent::k_blevel_bu"), "ent::k_binit_zero"),
 }
 

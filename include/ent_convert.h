@@ -7,8 +7,9 @@
  * text file of "u v" tuples, shifts ids by the smallest one, and writes a CSR
  * whose rows hold their tuples in file order, duplicates and self-loops kept
  * (both directions with reverse = 1). Here the CSR is built on the device by
- * radix sort, with options the reference lacks: self-loop removal, sorted
- * rows and duplicate removal. The ent_convert CLI is the drop-in for the
+ * sorting (a partition for sorted rows without weights, radix sort otherwise),
+ * with options the reference lacks: self-loop removal, sorted rows and
+ * duplicate removal. The ent_convert CLI is the drop-in for the
  * converter binary.
  *
  * All functions return ENT_OK (0) or a negative ENT_E* code (ent_graph.h);
@@ -67,7 +68,7 @@ int ent_gen_rmat_tuples(int32_t scale, int32_t edgefactor, double a, double b,
 typedef struct ent_build_stats {
   int64_t records;   /* sorted records: ne, or 2 ne with ENT_CSR_REVERSE */
   int64_t m;         /* CSR entries */
-  int32_t key_bits;  /* radix sort key width */
+  int32_t key_bits;  /* sort key width */
   int32_t pad;
   double device_ms;  /* sort and CSR assembly, HIP events on the build stream */
 } ent_build_stats;
