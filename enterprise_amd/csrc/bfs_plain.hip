@@ -518,11 +518,12 @@ __device__ void inspect_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tall
 // time, so that many head loads, then frontier loads, are in flight. The scan
 // alone is bound by those scattered row reads: R-MAT searches, edge factor 16,
 // without and with heads, 2^20 vertices 102 and 97 us, 2^22 157 and 138, 2^23
-// 610 and 438, 2^24 568 and 488. kBuDense 8, 16 and 32 give 507, 509 and 614 us
-// at 2^23 (two neighbours per head); kBuWords 2, 4 and 8 give 436, 434 and 508;
-// heads of one, two and four neighbours 434, 509 and 605, since the array is
-// then no longer the smaller read.
-constexpr int kBuDense = 16;
+// 610 and 438, 2^24 568 and 488. With kBuDense 4, 8, 16 and 24, in later searches:
+// 2^22 from two roots 122, 119, 119, 119 and 142, 142, 148, 149 us, 2^23 402, 400,
+// 400, 567, 2^24 375, 375, 408, 407 and 302, 319, 316, 316. kBuWords 2, 4 and 8
+// give 436, 434 and 508 at 2^23; heads of one, two and four neighbours 434, 509
+// and 605, since the array is then no longer the smaller read.
+constexpr int kBuDense = 8;
 constexpr int kBuWords = 4;
 template <int BS, bool HUB, bool COUNT, bool HEAD>
 __device__ void bu_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COUNT> &tl) {
