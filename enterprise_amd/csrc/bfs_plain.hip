@@ -1291,8 +1291,9 @@ __global__ __launch_bounds__(kTinyThreads) void k_tiny(const long long *off, con
 // have and, if that is another queue-driven level whose frontier does not
 // grow by more than half, makes it the first state of that form (else
 // DEEP_NOT_TAKEN). Writes nothing the ordinary launches read, so launch i can
-// still follow. One wavefront.
-__global__ __launch_bounds__(kWave) void k_deep_take(Args a, long long i, DeepCtl *d) {
+// still follow. `number` names this try: several tries of one search publish
+// their ends in the same mirror. One wavefront.
+__global__ __launch_bounds__(kWave) void k_deep_take(Args a, long long i, DeepCtl *d, int number) {
   __shared__ State S;
   __shared__ unsigned long long tot[8];
   const int lane = threadIdx.x;
@@ -1321,7 +1322,7 @@ __global__ __launch_bounds__(kWave) void k_deep_take(Args a, long long i, DeepCt
     const bool was_queue = !S.done && S.phase == PH_TDQ;
     const unsigned long long prev = S.prev_nf;
     next_state(a, S, tot, q_fit);
-    D.search = S.search;
+    D.search = number;
     if (was_queue && !S.done && S.phase == PH_TDQ && 2 * nf <= 3 * prev + 16) {
       D.level = S.level;
       D.par = S.level & 1;
@@ -1802,6 +1803,8 @@ constexpr int kDeepFirstLevel = 8;
 // After launch `next` - 1, a queue-driven level whose state is *fin: runs the
 // rest of the search with several levels per launch. *taken: 1 done, 0 the
 // frontier is not one for it, -1 it outgrew the queues there (start again).
+// Every try has a search number of its own, so that the end of a refused one,
+// still in the mirror, is not read as this one's.
 int run_deep(ent_graph *g, Args &a, long long next, State *fin, int *taken) {
   *taken = 0;
   int rc = deep_reserve(g, 1, 0);
@@ -1818,10 +1821,13 @@ int run_deep(ent_graph *g, Args &a, long long next, State *fin, int *taken) {
   d.nstripe = kDeepStripes;
   int width = 0;
   if ((rc = deep_rows(g, &width, &d.rows))) return rc;
-  void *args[] = {&a, &next, &d.ctl};
+  if (++g->search_seq == 0) g->search_seq = 1;
+  const unsigned search = g->search_seq;
+  int number = int(search);
+  void *args[] = {&a, &next, &d.ctl, &number};
   HIP_TRY(launch(reinterpret_cast<const void *>(&k_deep_take), 1, kWave, args, g->stream));
   DeepState D;
-  rc = deep_run(g, d, width, 1, g->cus * 2, unsigned(fin->search), &D);
+  rc = deep_run(g, d, width, 1, g->cus * 2, search, &D);
   if (rc) return rc;
   if (D.error == DEEP_NOT_TAKEN) return ENT_OK;
   if (D.error) {
@@ -1920,7 +1926,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
         HIP_TRY(queue_phases(g, ks, &a, i, k));
         HIP_TRY(hipEventRecord(g->ev1, g->stream));  // end of the search once it is done
         i += k;
-        rc = wait_state(g, i - 1, g->search_seq, fin);
+        rc = wait_state(g, i - 1, unsigned(search), fin);
         if (rc) return rc;
         if (fin->done) break;
         if (i > max_launches) return set_error(ENT_EINTERNAL, "search did not finish in %lld launches", i);
@@ -1966,7 +1972,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
       for (long long i = 0;; i += k) {
         HIP_TRY(hipGraphLaunch(g->gexec, g->stream));
         HIP_TRY(hipEventRecord(g->ev1, g->stream));
-        rc = wait_state(g, i + k - 1, g->search_seq, fin);
+        rc = wait_state(g, i + k - 1, unsigned(search), fin);
         if (rc) return rc;
         if (fin->done) break;
         if (i > max_launches) return set_error(ENT_EINTERNAL, "search did not finish in %lld launches", i);

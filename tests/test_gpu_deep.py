@@ -94,6 +94,46 @@ def test_deep_search(oracle, name, launch):
             assert st["levels"] == 300 and st["phases"] < 100, st
 
 
+def _refused_then_tail(legs, tail):
+    """More vertices than one block searches: a binary tree whose frontiers
+    double until level 13 (a hand-over there is refused), a path of `tail`
+    vertices at its last leaf, `legs` leaves at each of them."""
+    levels = 14
+    leaf = (1 << levels) - 2
+    e = [(v, (v - 1) // 2) for v in range(1, leaf + 1)]
+    spine = [leaf] + list(range(leaf + 1, leaf + 1 + tail))
+    e += list(zip(spine[:-1], spine[1:]))
+    n = spine[-1] + 1
+    for v in spine[1:]:
+        e += [(v, n + j) for j in range(legs)]
+        n += legs
+    return graphs.edges_graph(max(n, (1 << 14) + 1), e)
+
+
+@pytest.mark.parametrize("launch", list(LAUNCHES))
+@pytest.mark.parametrize("legs", [0, 5, 14])
+def test_deep_refused_hand_over(oracle, legs, launch):
+    """Hand-overs refused early in a search (its frontiers grow), then one that
+    is taken, with a tail of several launches behind it: depths and counts on
+    the same handle again and again, and from roots inside the tail. One case
+    per row form (padded rows of 4 and 8 entries, CSR)."""
+    for tail in (30, 60, 700):
+        g = _refused_then_tail(legs, tail)
+        deg = np.diff(g.beg_pos)
+        assert deg.max() == max(3, legs + 2)
+        with DeviceGraph(g) as dg:
+            for direction in (L.DIR_TOPDOWN, L.DIR_AUTO):
+                dg.configure(launch=LAUNCHES[launch], direction=direction)
+                for r in (0, 1, 0, (1 << 14) - 2 + tail // 2, 0):
+                    want = oracle.bfs(g.beg_pos, g.adj, r)
+                    _say(f"[gpu] deep refused hand-over legs={legs} tail={tail} {launch} dir={direction} root={r}")
+                    got, st = dg.bfs(r)
+                    assert np.array_equal(got, want), (r, np.flatnonzero(got != want)[:8])
+                    edges, verts = oracle.report(g.beg_pos, want)
+                    assert (st["reached_edges"], st["reached_vertices"]) == (edges, verts), st
+                    assert st["levels"] == int(want.max()) + 1, st
+
+
 def test_deep_directed_topdown(oracle):
     """Forced top-down on a directed ring with chords and vertices that have
     in-edges only."""
