@@ -331,24 +331,6 @@ struct Carver {
   }
 };
 
-// Leaf bits and partition passes for sorted rows without weights. False
-// when the rest of a key would not fit 32 bits (n above 2^24): those keys
-// take the radix sort.
-bool msd_plan(const BuildShape &s, MsdPlan *p) {
-  p->cb = s.cb;
-  const int least = std::max(0, 2 * s.cb - 32), most = std::min(s.cb, kMaxLeafBits);
-  if (least > most) return false;
-  int b = 0;
-  while (b < most && (s.records >> b) > kLeafTarget) ++b;
-  p->b = std::max(b, least);
-  p->b1 = std::min(p->b, 8);
-  p->b2 = p->b - p->b1;
-  p->rem = 2 * s.cb - p->b;
-  p->nb = int(std::min<long long>(256, (s.ne + (1 << 14) - 1) >> 14));
-  p->halves = p->b > kHistBits ? 2 : 1;
-  return true;
-}
-
 hipError_t allow_lds(const void *fn, size_t bytes) {
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
 }
@@ -563,7 +545,7 @@ int build_csr(BuildContext &c, long long n, long long ne, const int *src, const 
   const size_t o_cnt = cv.take(16), o_gaps = cv.take(sizeof(Gap) * kGapCap);
   MsdBuild msd;
   RadixBuild radix;
-  const bool part = s.records && s.sorted && !w_in && msd_plan(s, &msd.p);
+  const bool part = s.records && s.sorted && !w_in && msd_plan(s.records, s.ne, s.cb, &msd.p);
   int rc = ENT_OK;
   if (part) msd.plan(s, cv);
   else if ((rc = radix.plan(s, kbits, w_in != nullptr, c.stream, cv))) return rc;

@@ -27,6 +27,8 @@
 // least-significant-digit sort of 45-bit keys that the other forms take.
 #pragma once
 
+#include "csr_plan.h"
+
 namespace ent {
 namespace {
 
@@ -36,17 +38,11 @@ namespace {
 // buckets get longer runs); the second, to 128 leaves a bucket, 450 us with
 // 4,096 (four blocks fit a CU) and 570 with 8,192.
 constexpr int kPart1Threads = 1024, kPart1Items = 16;
-constexpr int kPart2Threads = 512, kPart2Items = 8;
-constexpr int kPart2Tile = kPart2Threads * kPart2Items;
 constexpr int kMaxFan = 256;                          // buckets of one partition pass
-constexpr int kHistBits = 15;                         // leaf counters one block holds (128 KiB of LDS)
-constexpr int kMaxLeafBits = 16;
 constexpr int kHistThreads = 1024;
 constexpr int kLeafItems = 16;     // records per thread of the leaf sorts
 constexpr int kLeafClasses = 3;    // leaves of at most 4096, 8192, 16384 records: 256, 512, 1024 threads
 constexpr int kLeafSmall = 4096;
-constexpr int kChunk = 16384;      // largest leaf sorted whole; chunk of a merged one
-constexpr int kLeafTarget = 4096;  // mean records per leaf aimed at
 constexpr int kGroups = 256;       // key ranges a leaf's bins are spread over
 constexpr unsigned kBinMax = 64;   // a bin of more records sends its leaf to k_leaf_sort
 constexpr int kScanThreads = 1024;
@@ -56,12 +52,6 @@ constexpr int kMergeThreads = 256;
 constexpr int kEmitThreads = 256;
 constexpr int kEmitShift = 10;     // a wavefront emits 1024 consecutive records
 constexpr unsigned kEmitTile = 1u << kEmitShift;
-
-struct MsdPlan {
-  int cb, b, b1, b2, rem;
-  int nb;     // histogram blocks
-  int halves; // ranges of kHistBits-bit counters
-};
 
 struct Chunk {
   unsigned start, size;         // records of this chunk
@@ -763,7 +753,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit(BuildShape s, MsdPlan p, 
   };
   unsigned carry = first ? keys[first - 1] : 0u;
   int carry_row = first ? int(row_of(lo, carry)) : -1;
-  constexpr int kStep = 4;  // loads in flight
+  constexpr int kStep = kEmitStep / kWave;  // loads in flight
   for (unsigned i0 = first; i0 < last; i0 += kStep * kWave) {
     unsigned key[kStep];
 #pragma unroll

@@ -1,0 +1,66 @@
+"""The partition plan of sorted CSR construction (csrc/csr_plan.h), compiled
+for the host: near the 2^32 - 1 records that the entry points accept, the
+positions that the kernels form in 32 bits must not wrap."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "enterprise_amd", "csrc")
+
+# Prints "cb records accepted wraps" for every row width and record count:
+# wraps = 1 if one of the 32-bit expressions of the kernels, taken at the end
+# of the records, differs from its value in 64 bits.
+PROGRAM = r"""
+#include <cstdio>
+#include "csr_plan.h"
+using namespace ent;
+int main() {
+  const int64_t top = INT64_C(0xFFFFFFFF);
+  const int64_t counts[] = {1, 4096, INT64_C(1) << 31, kMsdMaxRecords - 1, kMsdMaxRecords, kMsdMaxRecords + 1,
+                            top - kPart2Tile, top - kEmitStep, top - 1, top};
+  for (int cb = 0; cb <= 31; ++cb)
+    for (int64_t r : counts) {
+      MsdPlan p{};
+      const bool in = msd_plan(r, r, cb, &p);
+      const uint64_t last = uint64_t(r);  // one past the last record
+      int wraps = 0;
+      // k_emit: i0 += kEmitStep until i0 >= last.
+      const uint64_t i0 = (last - 1) / kEmitStep * kEmitStep;
+      wraps |= uint64_t(uint32_t(uint32_t(i0) + kEmitStep)) != i0 + kEmitStep;
+      // k_msd_part2: positions of a tile that starts at the last record, and
+      // a bucket's tiles (a bucket may hold every record).
+      wraps |= uint64_t(uint32_t(uint32_t(last - 1) + uint32_t(kPart2Tile - 1))) != last - 1 + kPart2Tile - 1;
+      wraps |= uint64_t(uint32_t(uint32_t(last) + uint32_t(kPart2Tile - 1))) != last + kPart2Tile - 1;
+      // k_msd_reduce: a leaf's chunks.
+      wraps |= uint64_t(uint32_t(uint32_t(last) + uint32_t(kChunk - 1))) != last + kChunk - 1;
+      std::printf("%d %lld %d %d\n", cb, (long long)r, in ? 1 : 0, wraps);
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rows(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("plan")
+    src, exe = d / "plan.cpp", d / "plan"
+    src.write_text(PROGRAM)
+    subprocess.run([cxx, "-std=c++17", "-O1", "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    return [tuple(int(x) for x in line.split()) for line in out.splitlines()]
+
+
+def test_positions_do_not_wrap(rows):
+    assert any(wraps for _, _, _, wraps in rows)  # the check itself sees the wrapping sizes
+    bad = [(cb, r) for cb, r, accepted, wraps in rows if accepted and wraps]
+    assert not bad, bad
+
+
+def test_partition_keeps_its_range(rows):
+    """Row widths up to 24 bits and any count below the limit."""
+    for cb, r, accepted, _ in rows:
+        assert accepted == (cb <= 24 and r <= (1 << 32) - 1 - 16384), (cb, r)
