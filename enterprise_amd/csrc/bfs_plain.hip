@@ -771,6 +771,12 @@ __device__ __forceinline__ void tdq_claim(const Args &a, Smem<BS> &sm, int L, co
 // vertices 66 and 58 us, 2^18 75 and 70, 2^20 96 and 86, 2^22 137 and 119, 2^24
 // 485 and 407 from one root, 397 and 316 from another. Testing the visited bits
 // before the atomics costs up to 10% (2^19 84 and 93).
+//
+// Limits: beyond 2^18 edges the atomics of a level cost more than the two sweeps
+// (2^16 loses 20% of 2^22 and 2^24 searches, 2^20 gains nothing), and beyond four
+// a lane a small grid's stages overflow.
+constexpr int kFlatEdges = 1 << 18;
+constexpr int kFlatPer = 4;
 template <int BS, bool COUNT>
 __device__ void tdq_flat(const Args &a, Smem<BS> &sm, int L, int total, Tally<COUNT> &tl, unsigned long long &nf,
                          unsigned long long &mf, unsigned &md) {
@@ -797,8 +803,11 @@ __device__ void tdq_flat(const Args &a, Smem<BS> &sm, int L, int total, Tally<CO
   }
   pre[t] = base + incl - d;
   __syncthreads();
-  const int nt = int(gridDim.x) * BS;
-  for (int i = int(blockIdx.x) * BS + t; i < edges; i += 4 * nt) {
+  // No more lanes than a level may have edges take part: with grid_blocks set,
+  // the grid's lanes times four do not fit 32 bits.
+  const int nt = int(min(gridDim.x * unsigned(BS), unsigned(kFlatEdges)));
+  const int i0 = int(blockIdx.x) * BS + t;
+  for (int i = i0 < nt ? i0 : edges; i < edges; i += 4 * nt) {
     int u[4];
     bool in[4];
 #pragma unroll
@@ -1593,12 +1602,6 @@ LevelShape level_shape(const ent_graph *g) {
   return s;
 }
 
-// Limits of tdq_flat: beyond 2^18 edges the atomics of a level cost more than the
-// two sweeps (2^16 loses 20% of 2^22 and 2^24 searches, 2^20 gains nothing), and
-// beyond four a lane a small grid's stages overflow. Graphs without hubs have no
-// such levels and keep the kernel without it.
-constexpr int64_t kFlatEdges = 1 << 18;
-constexpr int64_t kFlatPer = 4;
 Args make_args(ent_graph *g, int *depth) {
   Args a{};
   a.off = g->off;
@@ -1619,10 +1622,11 @@ Args make_args(ent_graph *g, int *depth) {
   if (g->cfg.queue_small < 0) a.q_small = 0;
   else if (g->cfg.queue_small > 0) a.q_small = int(std::min<int64_t>(g->cfg.queue_small, int64_t(kStripes) * g->qcap_s / 2));
   else a.q_small = int(std::min<int64_t>(std::max<int64_t>(4096, g->n / 256), int64_t(kStripes) * g->qcap_s / 2));
+  // Graphs without hubs have no such levels and keep the kernel without tdq_flat.
   const bool flat = g->store->skewed && g->hub_slots == 0 && g->cfg.launch != ENT_LAUNCH_PERSISTENT &&
                     g->cfg.queue_max_degree == 0;
   a.flat_n = flat ? std::min(g->cfg.block_size, 256) : 0;
-  a.flat_m = int(std::min<int64_t>(kFlatEdges, kFlatPer * int64_t(level_shape(g).grid) * g->cfg.block_size));
+  a.flat_m = int(std::min<int64_t>(kFlatEdges, int64_t(kFlatPer) * level_shape(g).grid * g->cfg.block_size));
   a.q_maxdeg = g->cfg.queue_max_degree > 0 ? g->cfg.queue_max_degree : g->cfg.t_block;
   a.ctl = g->ctl;
   a.hmir = g->h_mir_dev;

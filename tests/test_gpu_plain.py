@@ -534,3 +534,14 @@ def test_queue_level_hubs(oracle, fan, deg):
                     dg.configure(direction=L.DIR_AUTO if blocks else L.DIR_TOPDOWN, block_size=bs, grid_blocks=blocks,
                                  launch=LAUNCHES[launch], count_examined=count)
                     _check(oracle, g, dg, 0, f"hubs fan={fan} deg={deg} bs={bs} blocks={blocks}/{launch}/{count}")
+
+
+@pytest.mark.parametrize("blocks", [700_000, 1 << 20])
+def test_queue_level_hubs_largest_grids(oracle, blocks):
+    """The same levels on the largest grids that the configuration allows: four
+    edges a lane reach past 2^31."""
+    g = HostGraph.rmat(15, 8, seed=3)
+    with DeviceGraph(g) as dg:
+        dg.configure(direction=L.DIR_TOPDOWN, block_size=1024, grid_blocks=blocks)
+        root = int(g.pick_roots(1, 4)[0])
+        _check(oracle, g, dg, root, f"hubs, {blocks} blocks")
