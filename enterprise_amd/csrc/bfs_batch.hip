@@ -1442,6 +1442,7 @@ struct BatchWorkspace {
   // frontiers' bytes of a batch searched side by side.
   unsigned long long *h_mir = nullptr, *h_mir_dev = nullptr;
   int expect_launches = 16;
+  DeepWorkspace *deep = nullptr;  // low-degree graphs: several levels per launch (bfs_deep.hip)
   int *rows = nullptr;     // device rows of ent_bfs_batch (grown on demand)
   size_t rows_bytes = 0;
   // Every nonzero mask in the lv ring belongs to a vertex in its slot's
@@ -1463,10 +1464,16 @@ constexpr int kDefaultLevels = 32;
 
 int words_for(int k) { return k <= 64 ? 1 : k <= 128 ? 2 : k <= 256 ? 4 : 8; }
 
-size_t ws_bytes(int64_t n, int W, int lcap) {
+// Whether a workspace also gets tables for searches side by side.
+bool wants_deep(const ent_graph *g) {
+  return g->store->max_deg <= kDeepMaxDegree && g->n >= kDeepBatchVertices && !g->deep_batch_off;
+}
+
+size_t ws_bytes(const ent_graph *g, int W, int lcap) {
+  const int64_t n = g->n;
   const size_t nW = size_t(n) * size_t(W);
   const size_t nwords = size_t((n + 63) / 64);
-  return 8 * nW + (8 * nW + 8 * nwords) * size_t(lcap + 3) + sizeof(BControl) + 8 * ENT_BATCH_MAX_SOURCES;
+  return (wants_deep(g) ? deep_bytes(64 * W, kDeepQueue) : 0) + 8 * nW + (8 * nW + 8 * nwords) * size_t(lcap + 3) + sizeof(BControl) + 8 * ENT_BATCH_MAX_SOURCES;
 }
 
 int reserve(ent_graph *g, int k, int lcap) {
@@ -1506,7 +1513,9 @@ int reserve(ent_graph *g, int k, int lcap) {
     return set_error(ENT_ENOMEM, "pinned host memory");
   }
   std::memset(b->h_mir, 0, mir_bytes);  // search 0, which no search uses
-  b->bytes = ws_bytes(g->n, W, lcap);
+  b->bytes = ws_bytes(g, W, lcap);
+  // Without room for these the batches run as joint searches.
+  if (wants_deep(g)) b->deep = deep_alloc(g, 64 * W, kDeepQueue);
   return ENT_OK;
 }
 
@@ -1769,6 +1778,7 @@ void batch_release(ent_graph *g) {
   dev_free(g, b->roots, 8 * ENT_BATCH_MAX_SOURCES);
   dev_free(g, b->ctl, sizeof(BControl));
   dev_free(g, b->rows, b->rows_bytes);
+  deep_free(g, b->deep);
   if (b->h_ctl) ignore(hipHostFree(b->h_ctl));
   if (b->h_mir) ignore(hipHostFree(b->h_mir));
   delete b;
@@ -1779,19 +1789,17 @@ void batch_release(ent_graph *g) {
 namespace {
 
 // Whether a batch runs as k searches side by side, several levels per launch
-// (bfs_deep.hip), instead of on joint masks: no vertex of more than
-// kDeepMaxDegree edges, the default kind of configuration, and a graph of at
-// least kDeepBatchVertices (below it, uniform random graphs have no larger
+// (bfs_deep.hip), instead of on joint masks: tables for it in the workspace, the
+// default kind of configuration, no vertex of more than kDeepMaxDegree edges and
+// a graph of at least kDeepBatchVertices (below it, uniform random graphs have no larger
 // degrees either, and those spread too fast). 4-neighbour grids, joint search
 // against this one: 2048 x 2048 with 4, 16 and 64 sources 76, 87 and 151
 // against 6.3, 11.1 and 35.8 ms; 1024 x 1024 with 512 sources 223 against 65;
 // 300 x 300 with 32 sources 14.4 against 1.2. Sources close together, whose
 // joint frontiers coincide, cost the joint search no less than 4 sources do.
-constexpr int64_t kDeepBatchVertices = 1 << 12;
-bool deep_batch_fits(const ent_graph *g, int k) {
+bool deep_batch_fits(const ent_graph *g) {
   const ent_bfs_config &c = g->cfg;
-  return g->store->max_deg <= kDeepMaxDegree && g->n >= kDeepBatchVertices &&
-         !g->deep_batch_off && c.launch != ENT_LAUNCH_PERSISTENT && c.batch_fused > 0 &&
+  return g->batch->deep && !g->deep_batch_off && c.launch != ENT_LAUNCH_PERSISTENT && c.batch_fused > 0 &&
          (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN);
 }
 
@@ -1851,11 +1859,10 @@ int run_tiny_batch(ent_graph *g, const int32_t *roots, int k, int *out, bool wan
 // *ran stays false when a frontier outgrew the queues (the rows are then
 // written again by the joint search).
 int run_deep_batch(ent_graph *g, const int32_t *roots, int k, int *out, bool want_bytes, BState *fin, bool *ran) {
-  int rc = deep_reserve(g, k, kDeepQueue);
+  int rc = upload_sources(g, roots, k);
   if (rc) return rc;
-  if ((rc = upload_sources(g, roots, k))) return rc;
   std::vector<DeepState> st(static_cast<size_t>(k));
-  if ((rc = deep_batch(g, g->batch->roots, k, out, st.data()))) return rc;
+  if ((rc = deep_batch(g, g->batch->deep, g->batch->roots, k, out, st.data()))) return rc;
   for (const DeepState &s : st)
     if (s.error) {
       HIP_TRY(hipStreamSynchronize(g->stream));
@@ -1887,7 +1894,7 @@ int batch_locked(ent_graph *g, const int32_t *roots, int k, int32_t *depths_dev,
   if (tiny_fits(g) && g->cfg.batch_fused > 0) {
     rc = run_tiny_batch(g, roots, k, depths_dev, st != nullptr, &fin);
     ran = true;
-  } else if (deep_batch_fits(g, k)) {
+  } else if (deep_batch_fits(g)) {
     rc = run_deep_batch(g, roots, k, depths_dev, st != nullptr, &fin, &ran);
     if (!rc && !ran) g->deep_batch_off = true;
   }
@@ -1934,7 +1941,7 @@ extern "C" {
 
 int64_t ent_batch_workspace_bytes(const ent_graph *g, int32_t k, int32_t max_levels) {
   if (!g || k < 1 || k > ENT_BATCH_MAX_SOURCES) return -1;
-  return int64_t(ws_bytes(g->n, words_for(k), max_levels > 0 ? max_levels : kDefaultLevels));
+  return int64_t(ws_bytes(g, words_for(k), max_levels > 0 ? max_levels : kDefaultLevels));
 }
 
 int ent_batch_reserve(ent_graph *g, int32_t k, int32_t max_levels) {

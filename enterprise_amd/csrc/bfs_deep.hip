@@ -447,8 +447,11 @@ bool read_deep(const DeepWorkspace *w, int s, int slot, DeepState *out, unsigned
 
 }  // namespace
 
-void deep_release(ent_graph *g) {
-  DeepWorkspace *w = g->deep;
+size_t deep_bytes(int k, int qcap_s) {
+  return size_t(k) * (sizeof(DeepCtl) + 2 * sizeof(int) * kDeepStripes * size_t(qcap_s));
+}
+
+void deep_free(ent_graph *g, DeepWorkspace *w) {
   if (!w) return;
   const size_t qb = sizeof(int) * size_t(w->kcap) * kDeepStripes * size_t(w->qcap_s);
   dev_free(g, w->ctl, sizeof(DeepCtl) * size_t(w->kcap));
@@ -456,71 +459,52 @@ void deep_release(ent_graph *g) {
   dev_free(g, w->q[1], qb);
   if (w->h_mir) ignore(hipHostFree(w->h_mir));
   delete w;
-  g->deep = nullptr;
 }
 
-int deep_reserve(ent_graph *g, int k, int qcap_s) {
-  if (g->deep && g->deep->kcap >= k && g->deep->qcap_s >= qcap_s) return ENT_OK;
-  if (g->deep) {
-    HIP_TRY(hipStreamSynchronize(g->stream));
-    k = std::max(k, g->deep->kcap);
-    qcap_s = std::max(qcap_s, g->deep->qcap_s);
-    deep_release(g);
-  }
+DeepWorkspace *deep_alloc(ent_graph *g, int k, int qcap_s) {
   DeepWorkspace *w = new (std::nothrow) DeepWorkspace();
-  if (!w) return set_error(ENT_ENOMEM, "out of host memory");
-  g->deep = w;
+  if (!w) return nullptr;
   w->kcap = k;
   w->qcap_s = qcap_s;
   const size_t qb = sizeof(int) * size_t(k) * kDeepStripes * size_t(qcap_s);
   const size_t mb = sizeof(unsigned long long) * 2 * kDeepHostWords * size_t(k);
-  int rc;
-  if ((rc = dev_alloc(g, reinterpret_cast<void **>(&w->ctl), sizeof(DeepCtl) * size_t(k))) ||
-      (qcap_s && ((rc = dev_alloc(g, reinterpret_cast<void **>(&w->q[0]), qb)) ||
-                  (rc = dev_alloc(g, reinterpret_cast<void **>(&w->q[1]), qb))))) {
-    deep_release(g);
-    return rc;
-  }
   void *dev = nullptr;
-  if (hipHostMalloc(reinterpret_cast<void **>(&w->h_mir), mb, hipHostMallocCoherent) != hipSuccess ||
+  if (dev_alloc(g, reinterpret_cast<void **>(&w->ctl), sizeof(DeepCtl) * size_t(k)) ||
+      (qcap_s && (dev_alloc(g, reinterpret_cast<void **>(&w->q[0]), qb) ||
+                  dev_alloc(g, reinterpret_cast<void **>(&w->q[1]), qb))) ||
+      hipHostMalloc(reinterpret_cast<void **>(&w->h_mir), mb, hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer(&dev, w->h_mir, 0) != hipSuccess) {
     ignore(hipGetLastError());
-    deep_release(g);
-    return set_error(ENT_ENOMEM, "pinned host memory");
+    clear_error();
+    deep_free(g, w);
+    return nullptr;
   }
   w->h_mir_dev = static_cast<unsigned long long *>(dev);
   std::memset(w->h_mir, 0, mb);
-  return ENT_OK;
+  return w;
 }
 
-int deep_rows(ent_graph *g, int *width, const int **rows) {
+int deep_build_rows(ent_graph *g) {
   GraphStore &st = *g->store;
   const int want = st.max_deg <= 4 ? 1 : st.max_deg <= 8 ? 2 : 0;
-  std::lock_guard<std::mutex> lk(st.rows_mu);
-  if (st.rows_width < 0) {
-    st.rows_width = 0;
-    if (want) {
-      const int rc = dev_alloc(g, reinterpret_cast<void **>(&st.rows), 16 * size_t(want) * size_t(g->n));
-      if (rc == ENT_OK) {
-        const dim3 grid(unsigned(g->cus) * 8);
-        int4 *out = reinterpret_cast<int4 *>(st.rows);
-        if (want == 1) hipLaunchKernelGGL(k_deep_rows<1>, grid, dim3(256), 0, g->stream, g->off, g->adj, (long long)g->n, out);
-        else hipLaunchKernelGGL(k_deep_rows<2>, grid, dim3(256), 0, g->stream, g->off, g->adj, (long long)g->n, out);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipStreamSynchronize(g->stream));  // other handles read them on their own streams
-        st.rows_width = want;
-      } else {
-        clear_error();  // no room: the CSR form
-      }
-    }
+  if (!want || g->n < kDeepBatchVertices) return ENT_OK;
+  if (dev_alloc(g, reinterpret_cast<void **>(&st.rows), 16 * size_t(want) * size_t(g->n))) {
+    clear_error();  // no room: the CSR form
+    return ENT_OK;
   }
-  *width = st.rows_width;
-  *rows = st.rows;
+  const dim3 grid(unsigned(g->cus) * 8);
+  int4 *out = reinterpret_cast<int4 *>(st.rows);
+  if (want == 1) hipLaunchKernelGGL(k_deep_rows<1>, grid, dim3(256), 0, g->stream, g->off, g->adj, (long long)g->n, out);
+  else hipLaunchKernelGGL(k_deep_rows<2>, grid, dim3(256), 0, g->stream, g->off, g->adj, (long long)g->n, out);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(g->stream));  // other handles read them on their own streams
+  st.rows_width = want;
   return ENT_OK;
 }
 
-int deep_run(ent_graph *g, const DeepArgs &a, int width, int k, int blocks, unsigned search, DeepState *fin) {
-  const DeepWorkspace *w = g->deep;
+int deep_run(ent_graph *g, const DeepWorkspace *w, const DeepArgs &a, int k, int blocks, unsigned search,
+             DeepState *fin) {
+  const int width = a.rows ? g->store->rows_width : 0;
   const bool skip = k > kDeepLatencySources;
   const void *kernel = width == 0 ? reinterpret_cast<const void *>(&k_deep<0, false>)
                        : width == 1
@@ -580,8 +564,7 @@ int deep_run(ent_graph *g, const DeepArgs &a, int width, int k, int blocks, unsi
   return ENT_OK;
 }
 
-int deep_batch(ent_graph *g, const int32_t *roots, int k, int *rows, DeepState *fin) {
-  const DeepWorkspace *w = g->deep;
+int deep_batch(ent_graph *g, const DeepWorkspace *w, const int32_t *roots, int k, int *rows, DeepState *fin) {
   DeepArgs a{};
   a.off = g->off;
   a.adj = g->adj;
@@ -592,9 +575,7 @@ int deep_batch(ent_graph *g, const int32_t *roots, int k, int *rows, DeepState *
   a.qstride = (long long)kDeepStripes * w->qcap_s;
   a.ctl = w->ctl;
   a.hmir = w->h_mir_dev;
-  int width = 0;
-  const int rc = deep_rows(g, &width, &a.rows);
-  if (rc) return rc;
+  a.rows = g->store->rows;
   // About 1,024 blocks over all sources (four per CU fit their LDS).
   const int blocks = std::max(8, std::min(2 * g->cus, 4 * g->cus / k));
   a.nstripe = std::min(blocks, kDeepStripes);
@@ -606,7 +587,7 @@ int deep_batch(ent_graph *g, const int32_t *roots, int k, int *rows, DeepState *
                      (long long)k * (long long)g->n);
   hipLaunchKernelGGL(k_deep_seed, dim3(unsigned(k)), dim3(256), 0, g->stream, a, roots, int(search));
   HIP_TRY(hipGetLastError());
-  return deep_run(g, a, width, k, blocks, search, fin);
+  return deep_run(g, w, a, k, blocks, search, fin);
 }
 
 int deep_queue_joint_bytes(ent_graph *g, const int *rows, const int *order_dev, int k, unsigned long long *host) {

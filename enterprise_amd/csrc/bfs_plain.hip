@@ -1414,7 +1414,8 @@ void release(ent_graph *g) {
   ignore(hipSetDevice(g->device));
   if (g->stream) ignore(hipStreamSynchronize(g->stream));  // launches queued behind a finished search
   batch_release(g);
-  deep_release(g);
+  deep_free(g, g->deep);
+  g->deep = nullptr;
   if (g->gexec) ignore(hipGraphExecDestroy(g->gexec));
   if (g->graph) ignore(hipGraphDestroy(g->graph));
   g->store.reset();
@@ -1790,13 +1791,13 @@ int wait_state(ent_graph *g, long long last, unsigned search, State *out) {
   }
 }
 
-// Whether searches on g may go on with several levels per launch: no vertex
-// of more than kDeepMaxDegree edges (a lane takes a whole row), and a
-// configuration that neither asks for bottom-up levels, for the reference's
-// switch, for a tally nor for no queues.
+// Whether searches on g may go on with several levels per launch: tables for
+// it (made for graphs without a vertex of more than kDeepMaxDegree edges: a
+// lane takes a whole row), and a configuration that neither asks for bottom-up
+// levels, for the reference's switch, for a tally nor for no queues.
 bool deep_fits(const ent_graph *g) {
   const ent_bfs_config &c = g->cfg;
-  return g->store->max_deg <= kDeepMaxDegree && !g->deep_off && !c.count_examined && g->hub_slots == 0 &&
+  return g->deep && !g->deep_off && !c.count_examined && g->hub_slots == 0 &&
          c.queue_small >= 0 && (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN);
 }
 
@@ -1811,8 +1812,6 @@ constexpr int kDeepFirstLevel = 8;
 // still in the mirror, is not read as this one's.
 int run_deep(ent_graph *g, Args &a, long long next, State *fin, int *taken) {
   *taken = 0;
-  int rc = deep_reserve(g, 1, 0);
-  if (rc) return rc;
   DeepArgs d{};
   d.off = a.off;
   d.adj = a.adj;
@@ -1823,15 +1822,14 @@ int run_deep(ent_graph *g, Args &a, long long next, State *fin, int *taken) {
   d.hmir = g->deep->h_mir_dev;
   d.qcap_s = a.qcap_s;
   d.nstripe = kDeepStripes;
-  int width = 0;
-  if ((rc = deep_rows(g, &width, &d.rows))) return rc;
+  d.rows = g->store->rows;
   if (++g->search_seq == 0) g->search_seq = 1;
   const unsigned search = g->search_seq;
   int number = int(search);
   void *args[] = {&a, &next, &d.ctl, &number};
   HIP_TRY(launch(reinterpret_cast<const void *>(&k_deep_take), 1, kWave, args, g->stream));
   DeepState D;
-  rc = deep_run(g, d, width, 1, g->cus * 2, search, &D);
+  const int rc = deep_run(g, g->deep, d, 1, g->cus * 2, search, &D);
   if (rc) return rc;
   if (D.error == DEEP_NOT_TAKEN) return ENT_OK;
   if (D.error) {
@@ -2052,6 +2050,7 @@ int alloc_workspace(ent_graph *g) {
   HIP_TRY(hipMemset(g->aux, 0, kAuxBytes + kParentCountBytes));
   HIP_TRY(hipMemset(g->ctl, 0, sizeof(Control)));
   HIP_TRY(hipDeviceSynchronize());
+  if (g->store->max_deg <= kDeepMaxDegree && !tiny_graph(g)) g->deep = deep_alloc(g, 1, 0);
   return build_lists(g);
 }
 
@@ -2077,6 +2076,7 @@ int ent_graph_share(ent_graph *src, ent_graph **out) {
     g->adj = src->adj;
     g->nzmask = src->nzmask;
     g->cfg = src->cfg;
+    g->dev_limit = src->dev_limit;
   }
   const int rc = alloc_workspace(g);
   if (rc) {
@@ -2235,6 +2235,7 @@ int upload_graph(const int64_t *beg_pos, const int32_t *adj, bool adj_on_device,
     UP_TRY(hipGetLastError());
     UP_TRY(hipStreamSynchronize(g->stream));
   }
+  if (!rc && g->store->max_deg <= kDeepMaxDegree) rc = deep_build_rows(g);
   if (rc) {
     release(g);
     return rc;
@@ -2511,6 +2512,16 @@ int ent_get_config(const ent_graph *g, ent_bfs_config *cfg) {
   clear_error();
   if (!g || !cfg) return set_error(ENT_EINVAL, "NULL argument");
   *cfg = g->cfg;
+  return ENT_OK;
+}
+
+// For tests, not in the public headers: device allocations of the handle, and
+// of handles made from it, fail beyond `bytes` in all (0: no limit).
+int ent_internal_limit_device_bytes(ent_graph *g, int64_t bytes) {
+  clear_error();
+  if (!g || bytes < 0) return set_error(ENT_EINVAL, "bad argument");
+  std::lock_guard<std::mutex> lk(g->mu);
+  g->dev_limit = size_t(bytes);
   return ENT_OK;
 }
 

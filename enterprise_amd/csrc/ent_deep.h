@@ -12,6 +12,7 @@
 namespace ent {
 
 constexpr int kDeepMaxDegree = 16;  // largest degree of a graph searched this way
+constexpr int64_t kDeepBatchVertices = 1 << 12;  // smallest graph whose batches are
 constexpr int kDeepLevels = 24;     // levels per launch
 constexpr int kDeepQueue = 512;     // queue entries per stripe and source of a batch
 constexpr int kDeepStripes = 64;    // counter and queue stripes
@@ -49,7 +50,7 @@ struct DeepCtl {
 struct DeepArgs {
   const long long *off;
   const int *adj;
-  const int *rows;    // padded rows (deep_rows), or null
+  const int *rows;    // padded rows (deep_build_rows), or null
   int *depth;         // source s: depth + s * dstride
   long long dstride;
   int *q[2];          // source s: q[p] + s * qstride, stripe t at + t * qcap_s
@@ -60,7 +61,11 @@ struct DeepArgs {
   int nstripe;        // stripes in use: min(blocks per source, kDeepStripes)
 };
 
-// Per-handle tables for up to kcap sources.
+// Tables for up to kcap sources. A handle has one for its single-source
+// searches (no queues: those of the search), its batch workspace one for its
+// batches; both are made with the workspace they belong to, so that a search
+// allocates nothing. Where there is no room for one, that handle's searches
+// (batches) stay in the ordinary form.
 struct DeepWorkspace {
   int kcap = 0, qcap_s = 0;
   DeepCtl *ctl = nullptr;
@@ -68,24 +73,26 @@ struct DeepWorkspace {
   unsigned long long *h_mir = nullptr, *h_mir_dev = nullptr;
 };
 
-// Width of g's padded rows in int4 (0: none; degrees above 8), built on first
-// use for every handle on the graph: vertex v's neighbours at
-// rows[4 * width * v], -1 behind the last.
-int deep_rows(ent_graph *g, int *width, const int **rows);
+// Builds the store's padded rows, for every handle on the graph: vertex v's
+// neighbours at rows[4 * rows_width * v], -1 behind the last. None for degrees
+// above 8, for small graphs, and where there is no room.
+int deep_build_rows(ent_graph *g);
 
-// Makes g->deep hold at least k sources with queues of qcap_s entries per
-// stripe (0: the caller's own queues).
-int deep_reserve(ent_graph *g, int k, int qcap_s);
-void deep_release(ent_graph *g);
+// Tables for k sources with queues of qcap_s entries per stripe (0: none), or
+// null where there is no room.
+DeepWorkspace *deep_alloc(ent_graph *g, int k, int qcap_s);
+void deep_free(ent_graph *g, DeepWorkspace *w);
+size_t deep_bytes(int k, int qcap_s);
 
 // Runs launches of `blocks` blocks per source until every one of the k
-// searches whose states are in ctl[s].st[1] is done; their final states go to
+// searches whose states are in w->ctl[s].st[1] is done; their final states go to
 // fin[0 .. k). The host spins on the mirror, as for the other forms.
-int deep_run(ent_graph *g, const DeepArgs &a, int width, int k, int blocks, unsigned search, DeepState *fin);
+int deep_run(ent_graph *g, const DeepWorkspace *w, const DeepArgs &a, int k, int blocks, unsigned search,
+             DeepState *fin);
 
 // Batch of k sources from their roots (device memory) into rows of n
 // entries.
-int deep_batch(ent_graph *g, const int32_t *roots, int k, int *rows, DeepState *fin);
+int deep_batch(ent_graph *g, const DeepWorkspace *w, const int32_t *roots, int k, int *rows, DeepState *fin);
 
 // Queues the algorithmic bytes of the joint frontiers, 8 + 12 deg(v) for each
 // distinct (vertex, depth) pair of each 64-source group (rows order[64 g] on),

@@ -33,9 +33,8 @@ struct GraphStore {
   int32_t max_deg = 0;
   bool skewed = false;                   // largest degree far above the mean (kSkew)
   int *head = nullptr;                   // first neighbour of each row, or null (bfs_plain.hip)
-  std::mutex rows_mu;                    // guards rows, rows_width (ent_deep.h)
-  int *rows = nullptr;
-  int rows_width = -1;                   // -1: not built yet
+  int *rows = nullptr;                   // padded rows, or null (ent_deep.h)
+  int rows_width = 0;                    // their width in int4
   ~GraphStore() {
     if (hipSetDevice(device) != hipSuccess) return;
     ignore(hipFree(off));
@@ -105,9 +104,10 @@ struct ent_graph {
   unsigned char graph_args[512] = {};  // launch arguments baked into the captured graph
   int graph_bs = 0, graph_grid = 0, graph_k = 0;
   size_t dev_bytes = 0;
+  size_t dev_limit = 0;  // dev_alloc fails beyond it (tests; 0: none)
   int last_grid = 0;
   int expect_launches = 12;
-  ent::DeepWorkspace *deep = nullptr;    // several levels per launch (ent_deep.h)
+  ent::DeepWorkspace *deep = nullptr;    // several levels per launch (ent_deep.h), or null
   // A search (batch) of that form outgrew its queues: the graph spreads too
   // fast for it, and later ones start in the ordinary form.
   bool deep_off = false, deep_batch_off = false;
@@ -144,7 +144,8 @@ inline hipError_t device_malloc(int device, void **p, size_t bytes) {
 
 inline int dev_alloc(ent_graph *g, void **p, size_t bytes) {
   if (bytes == 0) bytes = 8;
-  hipError_t e = device_malloc(g->device, p, bytes);
+  const bool over = g->dev_limit && g->dev_bytes + bytes > g->dev_limit;
+  hipError_t e = over ? hipErrorOutOfMemory : device_malloc(g->device, p, bytes);
   if (e != hipSuccess) {
     *p = nullptr;
     ignore(hipGetLastError());

@@ -142,13 +142,15 @@ __device__ __forceinline__ TinyResult tiny_search(TinySmem &sm, const long long 
   return TinyResult{L, total_nf};
 }
 
+inline bool tiny_graph(const ent_graph *g) { return g->n <= kTinyVertices && g->m <= kTinyEdges; }
+
 // Whether searches on g run in one block each: at most kTinyVertices vertices
 // and kTinyEdges edges, and a configuration that neither asks for bottom-up
 // levels, for the reference's switch, for a launch form that keeps levels
 // apart, for a tally nor for no queues.
 inline bool tiny_fits(const ent_graph *g) {
   const ent_bfs_config &c = g->cfg;
-  return g->n <= kTinyVertices && g->m <= kTinyEdges && !c.count_examined && g->hub_slots == 0 && c.queue_small >= 0 &&
+  return tiny_graph(g) && !c.count_examined && g->hub_slots == 0 && c.queue_small >= 0 &&
          (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN) &&
          (c.launch == ENT_LAUNCH_STREAM || c.launch == ENT_LAUNCH_GRAPH);
 }

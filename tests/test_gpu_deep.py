@@ -4,6 +4,8 @@ at the edges of a launch's levels, on graphs with odd cycles (a block can
 reach a vertex by the longer way first), at the largest degree of the rule,
 and on graphs that spread too fast and fall back; batches of few sources
 against single-source rows and the joint search's counts."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -196,3 +198,67 @@ def test_deep_batch_spreading_graph(oracle):
             out, st = dg.bfs_batch(np.array(roots, np.int32))
             for i, r in enumerate(roots):
                 assert np.array_equal(out[i], oracle.bfs(g.beg_pos, g.adj, r))
+
+
+def _limit(dg, nbytes):
+    f = L.lib().ent_internal_limit_device_bytes
+    f.argtypes, f.restype = [C.c_void_p, C.c_int64], C.c_int
+    assert f(dg.handle, nbytes) == L.ENT_OK
+
+
+def test_deep_search_without_room(oracle):
+    """A handle whose tables for several levels per launch cannot be had
+    searches in the ordinary form."""
+    g = _random_grid(200, 150, 0.1, 4)
+    roots = [int(r) for r in g.pick_roots(3, 2)]
+    with DeviceGraph(g) as dg, DeviceGraph(share=dg) as roomy:
+        _limit(dg, roomy.info()["device_bytes"] - 64)
+        with DeviceGraph(share=dg) as tight:
+            for launch in LAUNCHES.values():
+                for h in (tight, roomy):
+                    h.configure(launch=launch)
+                for r in roots:
+                    _say(f"[gpu] deep search without room, launch {launch} root={r}")
+                    want = oracle.bfs(g.beg_pos, g.adj, r)
+                    got, st = tight.bfs(r)
+                    assert np.array_equal(got, want)
+                    got, sr = roomy.bfs(r)
+                    assert np.array_equal(got, want)
+                    assert 2 * sr["phases"] < sr["levels"] < st["phases"]
+                    for key in COUNTS[:3]:
+                        assert st[key] == sr[key], (key, st, sr)
+
+
+def test_deep_batch_without_room(oracle):
+    """A batch workspace that has room for the joint search alone serves the
+    batch as one, and the same handle side by side once there is room."""
+    g = _random_grid(300, 250, 0.1, 7)
+    k = 70
+    roots = g.pick_roots(k, 11)
+    want = np.stack([oracle.bfs(g.beg_pos, g.adj, int(r)) for r in roots])
+    with DeviceGraph(g) as dg:
+        # One byte less than all of it, which leaves room for the library's own
+        # rows of bfs_batch.
+        need = L.lib().ent_batch_workspace_bytes(dg.handle, k, 40)
+        _limit(dg, dg.info()["device_bytes"] + need - 1)
+        dg.batch_reserve(k, 40)
+        _say("[gpu] deep batch without room")
+        out, st = dg.bfs_batch(roots)
+        assert np.array_equal(out, want)
+        assert st["phases"] >= st["levels"]
+        dg.batch_release()
+        _limit(dg, 0)
+        before = dg.info()["device_bytes"]
+        dg.batch_reserve(k, 40)
+        assert dg.info()["device_bytes"] - before == need
+        side, ss = dg.bfs_batch(roots)
+        assert np.array_equal(side, want)
+        assert 8 * ss["phases"] < st["phases"]
+        for key in ("levels", "reached_vertices", "reached_edges", "alg_bytes", "words", "k", "flushes"):
+            assert st[key] == ss[key], (key, st, ss)
+        # A smaller batch, then one as large as the workspace takes.
+        for m in (3, 128):
+            r = g.pick_roots(m, m)
+            out, ss = dg.bfs_batch(r)
+            assert np.array_equal(out, np.stack([oracle.bfs(g.beg_pos, g.adj, int(x)) for x in r]))
+            assert 8 * ss["phases"] < st["phases"]
