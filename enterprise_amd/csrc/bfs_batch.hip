@@ -1466,7 +1466,7 @@ int words_for(int k) { return k <= 64 ? 1 : k <= 128 ? 2 : k <= 256 ? 4 : 8; }
 
 // Whether a workspace also gets tables for searches side by side.
 bool wants_deep(const ent_graph *g) {
-  return g->store->max_deg <= kDeepMaxDegree && g->n >= kDeepBatchVertices && !g->deep_batch_off;
+  return g->store->max_deg <= kDeepMaxDegree && g->n >= kDeepBatchVertices && !g->store->deep_batch_off;
 }
 
 size_t ws_bytes(const ent_graph *g, int W, int lcap) {
@@ -1799,7 +1799,7 @@ namespace {
 // joint frontiers coincide, cost the joint search no less than 4 sources do.
 bool deep_batch_fits(const ent_graph *g) {
   const ent_bfs_config &c = g->cfg;
-  return g->batch->deep && !g->deep_batch_off && c.launch != ENT_LAUNCH_PERSISTENT && c.batch_fused > 0 &&
+  return g->batch->deep && !g->store->deep_batch_off && c.launch != ENT_LAUNCH_PERSISTENT && c.batch_fused > 0 &&
          (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN);
 }
 
@@ -1896,7 +1896,7 @@ int batch_locked(ent_graph *g, const int32_t *roots, int k, int32_t *depths_dev,
     ran = true;
   } else if (deep_batch_fits(g)) {
     rc = run_deep_batch(g, roots, k, depths_dev, st != nullptr, &fin, &ran);
-    if (!rc && !ran) g->deep_batch_off = true;
+    if (!rc && !ran) g->store->deep_batch_off = true;
   }
   if (!rc && !ran) rc = run_batch(g, roots, k, depths_dev, &fin);
   if (rc) {

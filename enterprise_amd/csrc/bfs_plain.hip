@@ -1797,7 +1797,7 @@ int wait_state(ent_graph *g, long long last, unsigned search, State *out) {
 // levels, for the reference's switch, for a tally nor for no queues.
 bool deep_fits(const ent_graph *g) {
   const ent_bfs_config &c = g->cfg;
-  return g->deep && !g->deep_off && !c.count_examined && g->hub_slots == 0 &&
+  return g->deep && !g->store->deep_off && !c.count_examined && g->hub_slots == 0 &&
          c.queue_small >= 0 && (c.direction == ENT_DIR_AUTO || c.direction == ENT_DIR_TOPDOWN);
 }
 
@@ -1890,7 +1890,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
     const int e = run_deep(g, a, next, fin, &taken);
     if (taken == 0) --deep_tries;
     if (taken < 0) {
-      g->deep_off = true;
+      g->store->deep_off = true;
       HIP_TRY(hipStreamSynchronize(g->stream));
     }
     return e;

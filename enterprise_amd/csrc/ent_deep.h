@@ -85,8 +85,10 @@ void deep_free(ent_graph *g, DeepWorkspace *w);
 size_t deep_bytes(int k, int qcap_s);
 
 // Runs launches of `blocks` blocks per source until every one of the k
-// searches whose states are in w->ctl[s].st[1] is done; their final states go to
-// fin[0 .. k). The host spins on the mirror, as for the other forms.
+// searches whose states are in w->ctl[s].st[1] is done, or one of them has
+// failed (the caller then runs all of them the ordinary way, behind what is
+// queued); their final states go to fin[0 .. k). The host spins on the mirror, as
+// for the other forms.
 int deep_run(ent_graph *g, const DeepWorkspace *w, const DeepArgs &a, int k, int blocks, unsigned search,
              DeepState *fin);
 

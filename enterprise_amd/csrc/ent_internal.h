@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <algorithm>
 #include <cstdint>
 #include <memory>
@@ -35,6 +36,10 @@ struct GraphStore {
   int *head = nullptr;                   // first neighbour of each row, or null (bfs_plain.hip)
   int *rows = nullptr;                   // padded rows, or null (ent_deep.h)
   int rows_width = 0;                    // their width in int4
+  // A search (batch) of several levels per launch outgrew its queues: the graph
+  // spreads too fast for that form, and later ones, on any handle, start in the
+  // ordinary one.
+  std::atomic<bool> deep_off{false}, deep_batch_off{false};
   ~GraphStore() {
     if (hipSetDevice(device) != hipSuccess) return;
     ignore(hipFree(off));
@@ -108,9 +113,6 @@ struct ent_graph {
   int last_grid = 0;
   int expect_launches = 12;
   ent::DeepWorkspace *deep = nullptr;    // several levels per launch (ent_deep.h), or null
-  // A search (batch) of that form outgrew its queues: the graph spreads too
-  // fast for it, and later ones start in the ordinary form.
-  bool deep_off = false, deep_batch_off = false;
   ent::BatchWorkspace *batch = nullptr;  // lazily allocated multi-source workspace
   std::mutex mu;
 };

@@ -262,3 +262,26 @@ def test_deep_batch_without_room(oracle):
             out, ss = dg.bfs_batch(r)
             assert np.array_equal(out, np.stack([oracle.bfs(g.beg_pos, g.adj, int(x)) for x in r]))
             assert 8 * ss["phases"] < st["phases"]
+
+
+def test_deep_spreading_graph_is_known_to_every_handle(oracle):
+    """What one handle's first batch (search) finds out about the graph holds
+    for the others: their workspaces leave the tables out, and their first
+    batch is a joint search."""
+    rng = np.random.default_rng(3)
+    n = 1 << 15
+    e = rng.integers(0, n, (2, n))  # mean degree 2: outgrows a block within ten levels
+    g = HostGraph.from_edges(n, e[0], e[1])
+    assert 8 < np.diff(g.beg_pos).max() <= 16
+    roots = g.pick_roots(40, 3)
+    want = np.stack([oracle.bfs(g.beg_pos, g.adj, int(r)) for r in roots])
+    with DeviceGraph(g) as dg, DeviceGraph(share=dg) as other:
+        before = L.lib().ent_batch_workspace_bytes(other.handle, 40, 32)
+        other.batch_reserve(40, 32)
+        for h in (dg, dg, other):
+            _say("[gpu] deep spreading batch")
+            out, st = h.bfs_batch(roots)
+            assert np.array_equal(out, want)
+            assert st["phases"] >= st["levels"]  # the joint search
+        for h in (dg, other):
+            assert L.lib().ent_batch_workspace_bytes(h.handle, 40, 32) < before
