@@ -285,3 +285,103 @@ def test_deep_spreading_graph_is_known_to_every_handle(oracle):
             assert st["phases"] >= st["levels"]  # the joint search
         for h in (dg, other):
             assert L.lib().ent_batch_workspace_bytes(h.handle, 40, 32) < before
+
+
+ABOVE_ONE_BLOCK = (1 << 14) + 1  # vertices; smaller graphs are searched by one block
+
+
+def _padded(g):
+    """g with isolated vertices behind it, so that one block does not take it."""
+    n = max(g.n, ABOVE_ONE_BLOCK)
+    beg = np.concatenate([g.beg_pos, np.full(n - g.n, g.beg_pos[-1], dtype=np.int64)])
+    return HostGraph.from_arrays(beg, np.array(g.adj, dtype=np.int32))
+
+
+def _agrees(oracle, g, dg, root):
+    want = oracle.bfs(g.beg_pos, g.adj, root)
+    got, st = dg.bfs(root)
+    assert np.array_equal(got, want), (root, np.flatnonzero(got != want)[:8])
+    assert (st["reached_edges"], st["reached_vertices"]) == oracle.report(g.beg_pos, want), st
+    assert st["levels"] == int(want.max()) + 1, st
+    return st
+
+
+@pytest.mark.parametrize("launch", list(LAUNCHES))
+@pytest.mark.parametrize("direction", ["topdown", "auto"])
+def test_deep_ends_of_launches(oracle, direction, launch):
+    """Paths of every length from 8 to 100 in one graph: searches that end
+    before the hand-over and at each level of the first launches behind it."""
+    lengths = range(8, 101)
+    edges, first = [], []
+    n = 0
+    for k in lengths:
+        first.append(n)
+        edges += [(n + i, n + i + 1) for i in range(k - 1)]
+        n += k
+    g = _padded(graphs.edges_graph(n, edges))
+    with DeviceGraph(g) as dg:
+        dg.configure(launch=LAUNCHES[launch], direction=L.DIR_TOPDOWN if direction == "topdown" else L.DIR_AUTO)
+        for k, v in zip(lengths, first):
+            _say(f"[gpu] deep path of {k}, {direction}, {launch}")
+            st = _agrees(oracle, g, dg, v)
+            _agrees(oracle, g, dg, v + k // 2)
+            # Several levels a launch, behind as many launches as the search
+            # before it took (at most k / 2 + 2).
+            if k >= 64:
+                assert 1 < st["phases"] < st["levels"], st
+
+
+@pytest.mark.parametrize("launch", list(LAUNCHES))
+@pytest.mark.parametrize("legs", [0, 2, 3, 6, 7, 14, 15])
+def test_deep_row_forms(oracle, legs, launch):
+    """Long spines whose vertices have `legs` leaves: both sides of the degrees
+    at which rows are padded to 4 and 8 entries, the CSR form up to the largest
+    degree, and the degree beyond it."""
+    g = _padded(_caterpillar(1200, legs))
+    assert np.diff(g.beg_pos).max() == legs + 2
+    with DeviceGraph(g) as dg:
+        for direction in (L.DIR_TOPDOWN, L.DIR_AUTO):
+            dg.configure(launch=LAUNCHES[launch], direction=direction)
+            for root in (0, 1, 599, 1199):
+                _say(f"[gpu] deep caterpillar legs={legs} {launch} dir={direction} root={root}")
+                st = _agrees(oracle, g, dg, root)
+                if legs <= 14:
+                    assert 1 < 4 * st["phases"] < st["levels"], st
+                else:
+                    assert st["phases"] >= st["levels"], st
+
+
+@pytest.mark.parametrize("launch", list(LAUNCHES))
+@pytest.mark.parametrize("branch,levels", [(3, 9), (7, 5), (15, 4)])
+def test_deep_outgrown(oracle, branch, levels, launch):
+    """A path into a tree, for each row form: the search is handed over on the
+    path, outgrows a block's queue in the tree and starts again, the next ones
+    stay in the ordinary form, also on another handle."""
+    g = _padded(_path_then_tree(40, branch, levels))
+    assert np.diff(g.beg_pos).max() == branch + 1
+    with DeviceGraph(g) as dg, DeviceGraph(share=dg) as other:
+        for h in (dg, other):
+            h.configure(launch=LAUNCHES[launch], direction=L.DIR_TOPDOWN)
+            for root in (0, 20, 0):
+                _say(f"[gpu] deep outgrown branch={branch} {launch} root={root}")
+                st = _agrees(oracle, g, h, root)
+        assert st["phases"] >= st["levels"], st
+
+
+def test_deep_directed_topdown_large(oracle):
+    """Forced top-down on a directed ring with chords and vertices that have
+    in-edges only, too many for one block."""
+    n, ring = 17000, 600
+    beg, adj = [0], []
+    for v in range(n):
+        row = sorted({(v + 1) % ring, ring + v * 20 % (n - ring)} | ({(v + 7) % ring} if v % 3 == 0 else set())) \
+            if v < ring else []
+        adj += row
+        beg.append(len(adj))
+    g = HostGraph.from_arrays(np.array(beg, np.int64), np.array(adj, np.int32))
+    with DeviceGraph(g, keep_order=True) as dg:
+        dg.configure(direction=L.DIR_TOPDOWN)
+        for r in (0, 1, ring - 1):
+            _say(f"[gpu] deep directed, large, root={r}")
+            st = _agrees(oracle, g, dg, r)
+            assert 1 < 2 * st["phases"] < st["levels"], st
