@@ -158,6 +158,7 @@ SIGNATURES = [
     ("ent_csr_build_device", C.c_int, [C.c_int32, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p,
                                        C.c_int32, C.c_void_p, C.c_void_p, C.c_int64,
                                        C.POINTER(C.c_int64), C.POINTER(BuildStats)]),
+    ("ent_csr_release_scratch", C.c_int, [C.c_int32]),
     ("ent_graph_upload_edges", C.c_int, [i32p, i32p, C.c_int64, C.c_int64, C.c_int32, C.c_int32,
                                          C.c_int32, C.POINTER(C.c_void_p)]),
     ("ent_csr_write_ref_files", C.c_int, [C.POINTER(CSR), i32p, C.c_char_p]),

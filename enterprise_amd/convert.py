@@ -69,6 +69,11 @@ def csr_build_device(n, ne, src_dev, dst_dev, flags, beg_pos_dev, adj_dev, adj_c
     return m.value, st.as_dict()
 
 
+def release_scratch(device=0):
+    """Frees the device memory that constructions on `device` keep for the next one."""
+    check(lib().ent_csr_release_scratch(int(device)))
+
+
 def write_ref_files(graph, prefix, weight=None):
     """The reference converter's output files for `prefix`."""
     w = None if weight is None else np.ascontiguousarray(weight, dtype=np.int32)

@@ -230,8 +230,10 @@ struct DevBuf {
 // each device waits here for the next one: allocating and freeing the scratch
 // costs 0.6 ms a call at 1.6 GB, and the driver's clearing of freed memory
 // stalls calls in a row for 10 to 1,000 ms. Bounded: one context per device,
-// of at most kIdleBytes; concurrent calls make their own. Given back when a
-// library allocation fails and when a graph handle of the device is freed.
+// of at most kIdleBytes; concurrent calls make their own. Given back by
+// ent_csr_release_scratch, when a library allocation fails and when a graph
+// handle of the device is freed. A call takes it only once its own buffers are
+// allocated, so that they can still have its memory.
 constexpr size_t kIdleBytes = size_t(4) << 30;
 
 struct BuildContext {
@@ -244,6 +246,7 @@ struct BuildContext {
   } *host = nullptr;
   void *mem = nullptr;
   size_t bytes = 0;
+  BuildContext *next = nullptr;  // of the idle ones
 
   ~BuildContext() {
     if (hipSetDevice(device) != hipSuccess) return;
@@ -280,11 +283,8 @@ struct BuildContext {
 };
 
 std::mutex g_idle_mu;
-std::vector<std::unique_ptr<BuildContext>> &idle_contexts() {
-  // Never destroyed: the runtime may be gone when static objects are.
-  static auto *v = new std::vector<std::unique_ptr<BuildContext>>();
-  return *v;
-}
+// Never destroyed: the runtime may be gone when static objects are.
+BuildContext *g_idle = nullptr;
 
 // A call's hold on a context. The stream is drained before the context is
 // idle again, also after an error.
@@ -293,11 +293,11 @@ struct ContextLease {
   int take(int device) {
     {
       std::lock_guard<std::mutex> lk(g_idle_mu);
-      auto &v = idle_contexts();
-      for (size_t i = 0; i < v.size(); ++i)
-        if (v[i]->device == device) {
-          c = std::move(v[i]);
-          v.erase(v.begin() + long(i));
+      for (BuildContext **p = &g_idle; *p; p = &(*p)->next)
+        if ((*p)->device == device) {
+          c.reset(*p);
+          *p = c->next;
+          c->next = nullptr;
           return ENT_OK;
         }
     }
@@ -310,14 +310,19 @@ struct ContextLease {
     std::unique_ptr<BuildContext> c = std::move(this->c);
     if (!c) return;
     if (!c->stream || !c->host || hipStreamSynchronize(c->stream) != hipSuccess || c->bytes > kIdleBytes) return;
+    std::unique_ptr<BuildContext> other;  // freed behind the lock
     std::lock_guard<std::mutex> lk(g_idle_mu);
-    auto &v = idle_contexts();
-    for (auto &x : v)
-      if (x->device == c->device) {  // another call came back first: keep the larger block
-        if (x->bytes < c->bytes) std::swap(x, c);
+    BuildContext **p = &g_idle;
+    while (*p && (*p)->device != c->device) p = &(*p)->next;
+    if (*p) {  // another call came back first: keep the larger block
+      if ((*p)->bytes >= c->bytes) {
+        other = std::move(c);
         return;
       }
-    v.push_back(std::move(c));
+      other.reset(*p);
+      c->next = other->next;
+    }
+    *p = c.release();
   }
 };
 
@@ -593,13 +598,21 @@ int check_tuples(int64_t n, int64_t ne, const int32_t *src, const int32_t *dst) 
   return ENT_OK;
 }
 
-// Copies host tuples (and weights) to new device buffers on `stream`.
-struct DevTuples {
-  DevBuf s, d, w;
-  int upload(int device, hipStream_t stream, int64_t ne, const int32_t *src, const int32_t *dst, const int32_t *weight) {
+// Device buffers for host tuples (and weights), and the CSR built of them.
+struct HostBuild {
+  DevBuf s, d, w, beg, adj, w_out;
+  int alloc(int device, int64_t n, int64_t ne, int64_t records, bool weights) {
     int rc;
-    if ((rc = s.alloc(device, 4 * size_t(ne), "tuples")) || (rc = d.alloc(device, 4 * size_t(ne), "tuples"))) return rc;
-    if (weight && (rc = w.alloc(device, 4 * size_t(ne), "weights"))) return rc;
+    if ((rc = s.alloc(device, 4 * size_t(ne), "tuples")) || (rc = d.alloc(device, 4 * size_t(ne), "tuples")) ||
+        (rc = beg.alloc(device, 8 * size_t(n + 1), "offsets")) ||
+        (rc = adj.alloc(device, 4 * size_t(records), "adjacency")))
+      return rc;
+    if (weights && ((rc = w.alloc(device, 4 * size_t(ne), "weights")) ||
+                    (rc = w_out.alloc(device, 4 * size_t(records), "weights"))))
+      return rc;
+    return ENT_OK;
+  }
+  int upload(hipStream_t stream, int64_t ne, const int32_t *src, const int32_t *dst, const int32_t *weight) {
     if (ne) {
       HIP_TRY(hipMemcpyAsync(s.p, src, 4 * size_t(ne), hipMemcpyHostToDevice, stream));
       HIP_TRY(hipMemcpyAsync(d.p, dst, 4 * size_t(ne), hipMemcpyHostToDevice, stream));
@@ -612,10 +625,14 @@ struct DevTuples {
 }  // namespace
 
 void build_give_back(int device) {
+  std::unique_ptr<BuildContext> c;  // freed behind the lock
   std::lock_guard<std::mutex> lk(g_idle_mu);
-  auto &v = idle_contexts();
-  for (size_t i = v.size(); i-- > 0;)
-    if (v[i]->device == device) v.erase(v.begin() + long(i));
+  for (BuildContext **p = &g_idle; *p; p = &(*p)->next)
+    if ((*p)->device == device) {
+      c.reset(*p);
+      *p = c->next;
+      return;  // there is one per device
+    }
 }
 
 }  // namespace ent
@@ -623,6 +640,18 @@ void build_give_back(int device) {
 using namespace ent;
 
 extern "C" {
+
+int ent_csr_release_scratch(int32_t device) {
+  clear_error();
+  int ndev = 0;
+  if (hipGetDeviceCount(&ndev) != hipSuccess) {
+    ignore(hipGetLastError());
+    ndev = 0;
+  }
+  if (device < 0 || device >= ndev) return set_error(ENT_EINVAL, "device %d of %d", device, ndev);
+  build_give_back(device);
+  return ENT_OK;
+}
 
 int ent_csr_build_device(int32_t device, int64_t n, int64_t ne, const int32_t *src_dev, const int32_t *dst_dev,
                          int32_t flags, int64_t *beg_pos_dev, int32_t *adj_dev, int64_t adj_capacity,
@@ -635,8 +664,8 @@ int ent_csr_build_device(int32_t device, int64_t n, int64_t ne, const int32_t *s
   int rc = ctx.take(device);
   if (rc) return rc;
   long long m = 0;
-  rc = build_csr(*ctx.c, n, ne, src_dev, dst_dev, nullptr, flags,
-                           reinterpret_cast<long long *>(beg_pos_dev), adj_dev, adj_capacity, nullptr, &m, st);
+  rc = build_csr(*ctx.c, n, ne, src_dev, dst_dev, nullptr, flags, reinterpret_cast<long long *>(beg_pos_dev), adj_dev,
+                 adj_capacity, nullptr, &m, st);
   if (rc) return rc;
   *m_out = m;
   return ENT_OK;
@@ -651,18 +680,15 @@ int ent_csr_build(int32_t device, int64_t n, int64_t ne, const int32_t *src, con
   std::memset(out, 0, sizeof *out);
   if (weight_out) *weight_out = nullptr;
   HIP_TRY(hipSetDevice(device));
-  ContextLease ctx;
-  if ((rc = ctx.take(device))) return rc;
-  hipStream_t stream = ctx.c->stream;
   const int64_t records = ne * ((flags & ENT_CSR_REVERSE) ? 2 : 1);
-  DevTuples dt;
-  DevBuf db, da, dwo;
-  if ((rc = dt.upload(device, stream, ne, src, dst, weight)) || (rc = db.alloc(device, 8 * size_t(n + 1), "offsets")) ||
-      (rc = da.alloc(device, 4 * size_t(records), "adjacency")) || (weight && (rc = dwo.alloc(device, 4 * size_t(records), "weights"))))
-    return rc;
+  HostBuild hb;
+  ContextLease ctx;
+  if ((rc = hb.alloc(device, n, ne, records, weight != nullptr)) || (rc = ctx.take(device))) return rc;
+  hipStream_t stream = ctx.c->stream;
   long long m = 0;
-  if ((rc = build_csr(*ctx.c, n, ne, dt.s.as<int>(), dt.d.as<int>(), weight ? dt.w.as<int>() : nullptr, flags,
-                      db.as<long long>(), da.as<int>(), records, weight ? dwo.as<int>() : nullptr, &m, st)))
+  if ((rc = hb.upload(stream, ne, src, dst, weight)) ||
+      (rc = build_csr(*ctx.c, n, ne, hb.s.as<int>(), hb.d.as<int>(), hb.w.as<int>(), flags, hb.beg.as<long long>(),
+                      hb.adj.as<int>(), records, hb.w_out.as<int>(), &m, st)))
     return rc;
   int64_t *beg = static_cast<int64_t *>(std::malloc(8 * size_t(n + 1)));
   int32_t *adj = static_cast<int32_t *>(std::malloc(4 * size_t(std::max<long long>(m, 1))));
@@ -675,9 +701,9 @@ int ent_csr_build(int32_t device, int64_t n, int64_t ne, const int32_t *src, con
   };
   if (!beg || !adj || (weight_out && weight && !wh))
     return fail(set_error(ENT_ENOMEM, "out of host memory (%lld entries)", m));
-  hipError_t e = hipMemcpyAsync(beg, db.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, stream);
-  if (e == hipSuccess && m) e = hipMemcpyAsync(adj, da.p, 4 * size_t(m), hipMemcpyDeviceToHost, stream);
-  if (e == hipSuccess && wh && m) e = hipMemcpyAsync(wh, dwo.p, 4 * size_t(m), hipMemcpyDeviceToHost, stream);
+  hipError_t e = hipMemcpyAsync(beg, hb.beg.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, stream);
+  if (e == hipSuccess && m) e = hipMemcpyAsync(adj, hb.adj.p, 4 * size_t(m), hipMemcpyDeviceToHost, stream);
+  if (e == hipSuccess && wh && m) e = hipMemcpyAsync(wh, hb.w_out.p, 4 * size_t(m), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (e != hipSuccess) return fail(set_error(ENT_EDEVICE, "copy of the CSR to the host failed: %s", hipGetErrorString(e)));
   out->n = n;
@@ -698,26 +724,23 @@ int ent_graph_upload_edges(const int32_t *src, const int32_t *dst, int64_t n, in
   int rc = check_tuples(n, ne, src, dst);
   if (rc) return rc;
   HIP_TRY(hipSetDevice(device));
-  ContextLease ctx;
-  if ((rc = ctx.take(device))) return rc;
-  hipStream_t stream = ctx.c->stream;
   const int64_t records = ne * ((flags & ENT_CSR_REVERSE) ? 2 : 1);
-  DevTuples dt;
-  DevBuf db, da;
-  if ((rc = dt.upload(device, stream, ne, src, dst, nullptr)) || (rc = db.alloc(device, 8 * size_t(n + 1), "offsets")) ||
-      (rc = da.alloc(device, 4 * size_t(records), "adjacency")))
-    return rc;
+  HostBuild hb;
+  ContextLease ctx;
+  if ((rc = hb.alloc(device, n, ne, records, false)) || (rc = ctx.take(device))) return rc;
+  hipStream_t stream = ctx.c->stream;
   long long m = 0;
-  if ((rc = build_csr(*ctx.c, n, ne, dt.s.as<int>(), dt.d.as<int>(), nullptr, flags, db.as<long long>(),
-                      da.as<int>(), records, nullptr, &m, nullptr)))
+  if ((rc = hb.upload(stream, ne, src, dst, nullptr)) ||
+      (rc = build_csr(*ctx.c, n, ne, hb.s.as<int>(), hb.d.as<int>(), nullptr, flags, hb.beg.as<long long>(),
+                      hb.adj.as<int>(), records, nullptr, &m, nullptr)))
     return rc;
   // The offsets come back for the host-side degree tables; the adjacency is
   // copied device to device into the handle's CSR.
   std::vector<int64_t> beg(size_t(n) + 1);
-  HIP_TRY(hipMemcpyAsync(beg.data(), db.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, stream));
+  HIP_TRY(hipMemcpyAsync(beg.data(), hb.beg.p, 8 * size_t(n + 1), hipMemcpyDeviceToHost, stream));
   HIP_TRY(hipStreamSynchronize(stream));
   ctx.give();
-  return upload_graph(beg.data(), da.as<int32_t>(), true, n, m, device, upload_flags, out);
+  return upload_graph(beg.data(), hb.adj.as<int32_t>(), true, n, m, device, upload_flags, out);
 }
 
 }  // extern "C"

@@ -83,14 +83,22 @@ int ent_csr_build(int32_t device, int64_t n, int64_t ne, const int32_t *src,
 
 /* The same on device-resident arrays of `device`: src_dev, dst_dev (ne
  * each), beg_pos_dev (n + 1), adj_dev (adj_capacity >= records). *m_out
- * receives m. Scratch memory is allocated and released inside. The ids are
- * not checked here (they are for host arrays): ids outside [0, n) give a
+ * receives m. The scratch memory (16 to 20 bytes a record) of the last
+ * construction on a device, up to 4 GiB, is kept for the next one, see
+ * ent_csr_release_scratch. The ids are not checked here (they are for host arrays): ids outside [0, n) give a
  * wrong CSR, though every write stays inside the given arrays. */
 int ent_csr_build_device(int32_t device, int64_t n, int64_t ne,
                          const int32_t *src_dev, const int32_t *dst_dev,
                          int32_t flags, int64_t *beg_pos_dev, int32_t *adj_dev,
                          int64_t adj_capacity, int64_t *m_out,
                          ent_build_stats *st);
+
+/* Frees the construction scratch memory kept on `device`, if there is any.
+ * The library does so by itself when one of its own allocations fails and
+ * when a BFS handle of the device is freed; a program that needs the memory
+ * for something else calls this. Constructions running in other threads keep
+ * theirs. */
+int ent_csr_release_scratch(int32_t device);
 
 /* A BFS handle whose CSR is built on the device from host tuples (no host
  * CSR); upload_flags as ent_graph_upload_ex. */

@@ -6,6 +6,7 @@ built from tuples."""
 import os
 import subprocess
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -213,3 +214,50 @@ def test_partition_drops_every_record():
     ids = np.arange(3000, dtype=np.int32)
     g, _, st = convert.csr_build(3000, ids, ids, L.CSR_SIMPLE)
     assert g.m == 0 and st["m"] == 0 and not g.beg_pos.any()
+
+
+def test_scratch_is_kept_and_given_back():
+    """The scratch of a construction serves the next one, and goes back when
+    the program asks for it and when a handle of the device is freed."""
+    import torch
+    n, ne = 1 << 20, 1 << 24
+    src = torch.randint(0, n, (ne,), dtype=torch.int32, device="cuda")
+    dst = torch.randint(0, n, (ne,), dtype=torch.int32, device="cuda")
+    beg = torch.empty(n + 1, dtype=torch.int64, device="cuda")
+    adj = torch.empty(2 * ne, dtype=torch.int32, device="cuda")
+
+    def build():
+        torch.cuda.synchronize()
+        m, _ = convert.csr_build_device(n, ne, src.data_ptr(), dst.data_ptr(), convert.SIMPLE, beg.data_ptr(),
+                                        adj.data_ptr(), 2 * ne)
+        return m
+
+    def free():
+        """Free device memory once it has settled: the driver clears what was
+        freed, by earlier tests too, in its own time before it counts."""
+        torch.cuda.synchronize()
+        seen = []
+        for _ in range(100):
+            seen.append(torch.cuda.mem_get_info()[0])
+            if len(seen) > 8 and len(set(seen[-8:])) == 1:
+                break
+            time.sleep(0.2)
+        return seen[-1]
+
+    m = build()
+    convert.release_scratch()
+    start = free()
+    slack = 64 << 20
+    for give_back in (convert.release_scratch, lambda: DeviceGraph(HostGraph.rmat(8, 4, seed=1)).free()):
+        _say("[gpu] construction scratch")
+        assert build() == m
+        kept = start - free()
+        assert kept > 8 * 2 * ne  # more than the records' keys
+        assert build() == m
+        assert abs(start - free() - kept) < slack
+        give_back()
+        assert abs(start - free()) < slack
+    convert.release_scratch()  # nothing left: no error
+    for device in (-1, 1 << 20):
+        with pytest.raises(EntError):
+            convert.release_scratch(device)
