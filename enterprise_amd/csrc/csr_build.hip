@@ -336,10 +336,6 @@ struct Carver {
   }
 };
 
-hipError_t allow_lds(const void *fn, size_t bytes) {
-  return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
-}
-
 // Sorted rows without weights by partition (csr_msd.h). plan() sizes the
 // scratch, run() queues the kernels.
 struct MsdBuild {
@@ -390,8 +386,10 @@ struct MsdBuild {
     hipStream_t stream = c.stream;
     const unsigned L = 1u << p.b;
     const size_t hist_lds = size_t(4) << std::min(p.b, kHistBits);
+    // The attribute belongs to the function, not to this launch: always the
+    // largest, whatever another thread builds meanwhile.
     HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_msd_hist), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                int(hist_lds)));
+                                4 << kHistBits));
     hipLaunchKernelGGL(k_msd_hist, dim3(unsigned(p.nb), unsigned(p.halves)), dim3(kHistThreads), hist_lds, stream, s,
                        p, src, dst, hist, mc, tile_cnt, tiles, ngaps);
     hipLaunchKernelGGL(k_msd_reduce, dim3((L + kWave - 1) / kWave), dim3(256), 0, stream, p, hist, counts, lists,

@@ -261,3 +261,30 @@ def test_scratch_is_kept_and_given_back():
     for device in (-1, 1 << 20):
         with pytest.raises(EntError):
             convert.release_scratch(device)
+
+
+def test_builds_of_different_sizes_at_once(oracle):
+    """Four threads whose histograms take 4 bytes to 128 KiB of LDS: what one
+    asks of the runtime for its launch is no limit for another's."""
+    import threading
+    wrong = []
+
+    def work(n, ne, seed):
+        try:
+            for i in range(10):
+                src, dst = _tuples(1000 * seed + i, n, ne)
+                g, _, _ = convert.csr_build(n, src, dst, L.CSR_SORT)
+                b, a, _ = oracle.csr_build(n, src, dst, L.CSR_SORT)
+                if not (np.array_equal(g.beg_pos, b) and np.array_equal(g.adj, a)):
+                    wrong.append((n, i))
+        except Exception as e:  # an error in a thread fails the test
+            wrong.append((n, e))
+
+    threads = [threading.Thread(target=work, args=x)
+               for x in ((1 << 24, 3000, 1), (1, 10, 2), (10, 100, 3), (1 << 22, 20000, 4))]
+    _say("[gpu] csr_build in four threads")
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:3]
