@@ -374,8 +374,10 @@ struct MsdBuild {
                        nullptr, &mc->leaves[k], off, k32, k32, tile_cnt, crowded, &mc->crowded[0]);
   }
 
+  // With `radix`, a build whose leaves would be merged too much ends behind the
+  // first partition pass, with *radix set: the caller sorts the tuples.
   int run(BuildContext &c, const BuildShape &s, const int *src, const int *dst, long long *beg, int *adj, Gap *gaps,
-          unsigned long long *ngaps) const {
+          unsigned long long *ngaps, bool *radix) const {
     char *base = static_cast<char *>(c.mem);
     auto u = [&](size_t o) { return reinterpret_cast<unsigned *>(base + o); };
     unsigned *k32 = u(o_keys), *counts = u(o_counts), *off = u(o_off), *cur1 = u(o_cur1), *cur2 = u(o_cur2),
@@ -401,13 +403,21 @@ struct MsdBuild {
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(kScanThreads), 0, stream, counts, off, L, cur1, cur2, p.b2);
     const long long per = (s.rev ? kPart1Items / 2 : kPart1Items) * (long long)kPart1Threads;
     const unsigned t1 = unsigned((s.ne + per - 1) / per);
-    if (p.b2) {
+    if (p.b2)
       hipLaunchKernelGGL(k_msd_part1<unsigned long long>, dim3(t1), dim3(kPart1Threads), 0, stream, s, p, src, dst,
                          cur1, k64);
+    else
+      hipLaunchKernelGGL(k_msd_part1<unsigned>, dim3(t1), dim3(kPart1Threads), 0, stream, s, p, src, dst, cur1, k32);
+    MsdCounts h{};
+    if (radix) {
+      HIP_TRY(hipGetLastError());
+      HIP_TRY(hipEventSynchronize(c.e_counts));
+      h = c.host->counts;
+      if ((*radix = merges_too_much(s.records, h.merged, h.max_size))) return ENT_OK;
+    }
+    if (p.b2) {
       const unsigned t2 = unsigned(s.records / kPart2Tile) + (1u << p.b1);
       hipLaunchKernelGGL(k_msd_part2, dim3(t2), dim3(kPart2Threads), 0, stream, p, k64, off, cur2, k32);
-    } else {
-      hipLaunchKernelGGL(k_msd_part1<unsigned>, dim3(t1), dim3(kPart1Threads), 0, stream, s, p, src, dst, cur1, k32);
     }
     sort_class<256>(0, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
     sort_class<512>(1, stream, c.cus, s, lists, mc, off, k32, tile_cnt, crowded);
@@ -419,14 +429,15 @@ struct MsdBuild {
     if (s.records > kChunk) {
       // The copy was queued before the partition passes, so the device is
       // still busy with them when the host has it.
-      HIP_TRY(hipEventSynchronize(c.e_counts));
-      const MsdCounts h = c.host->counts;
+      if (!radix) {
+        HIP_TRY(hipEventSynchronize(c.e_counts));
+        h = c.host->counts;
+      }
       if (h.chunks) {
         // The number of merge passes follows from the largest leaf; the
         // sorted chunks go where it leaves the result in k32.
         unsigned *other = reinterpret_cast<unsigned *>(k64);
-        int passes = 0;
-        while (((unsigned long long)kChunk << passes) < h.max_size) ++passes;
+        const int passes = merge_passes(h.max_size);
         hipLaunchKernelGGL(k_chunk_place, dim3(std::min((h.chunks + 255) / 256, 1024u)), dim3(256), 0, stream, mc, off,
                            chunks);
         unsigned *from = (passes & 1) ? other : k32, *to = (passes & 1) ? k32 : other;
@@ -550,17 +561,24 @@ int build_csr(BuildContext &c, long long n, long long ne, const int *src, const 
   RadixBuild radix;
   const bool part = s.records && s.sorted && !w_in && msd_plan(s.records, s.ne, s.cb, &msd.p);
   int rc = ENT_OK;
+  // A large build by partition may turn to the radix sort, in the same scratch.
+  bool turn = part && s.records >= kSwitchRecords, turned = false;
+  Carver cr = cv;
   if (part) msd.plan(s, cv);
-  else if ((rc = radix.plan(s, kbits, w_in != nullptr, c.stream, cv))) return rc;
+  if ((!part || turn) && (rc = radix.plan(s, kbits, w_in != nullptr, c.stream, cr))) return rc;
+  if (!part) cv = cr;
+  if (turn && c.reserve(std::max(cv.at, cr.at))) {
+    clear_error();
+    turn = false;  // no room for that
+  }
   if ((rc = c.reserve(cv.at))) return rc;
   char *mem = static_cast<char *>(c.mem);
   unsigned long long *ngaps = reinterpret_cast<unsigned long long *>(mem + o_cnt);
   Gap *gaps = reinterpret_cast<Gap *>(mem + o_gaps);
   hipStream_t stream = c.stream;
   HIP_TRY(hipEventRecord(c.e0, stream));
-  if ((rc = part ? msd.run(c, s, src, dst, beg, adj, gaps, ngaps)
-                 : radix.run(c, s, src, dst, w_in, beg, adj, w_out, gaps, ngaps)))
-    return rc;
+  if (part && (rc = msd.run(c, s, src, dst, beg, adj, gaps, ngaps, turn ? &turned : nullptr))) return rc;
+  if ((!part || turned) && (rc = radix.run(c, s, src, dst, w_in, beg, adj, w_out, gaps, ngaps))) return rc;
   hipLaunchKernelGGL(k_fill_gaps, dim3(c.cus * 4), dim3(kBuildBlock), 0, stream, gaps, ngaps, beg);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(c.e1, stream));

@@ -64,6 +64,7 @@ struct MsdCounts {
   unsigned crowded[2];            // leaves, chunks left to the radix sort
   unsigned chunks;                // chunks of the leaves above kChunk
   unsigned max_size;              // largest leaf
+  unsigned merged;                // records of the leaves above kChunk
 };
 
 // The (up to two) valid records of tuple i: bit 0 (u, v), bit 1 (v, u).
@@ -167,6 +168,7 @@ __global__ __launch_bounds__(256) void k_msd_reduce(MsdPlan p, const unsigned *h
     for (unsigned j = 0; j < k; ++j)
       chunks[at + j] = Chunk{j * kChunk, min(unsigned(kChunk), c - j * kChunk), leaf, 0u};
     atomicMax(&mc->max_size, c);
+    atomicAdd(&mc->merged, c);
   }
 }
 

@@ -1,6 +1,7 @@
 """The partition plan of sorted CSR construction (csrc/csr_plan.h), compiled
 for the host: near the 2^32 - 1 records that the entry points accept, the
-positions that the kernels form in 32 bits must not wrap."""
+positions that the kernels form in 32 bits must not wrap; and the rules that
+leave records with few or long rows to the radix sort."""
 import os
 import shutil
 import subprocess
@@ -14,11 +15,18 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 # of the records, differs from its value in 64 bits.
 PROGRAM = r"""
 #include <cstdio>
+#include <cstdlib>
 #include "csr_plan.h"
 using namespace ent;
-int main() {
+int main(int argc, char **argv) {
+  if (argc == 4) {  // records, records of merged leaves, the largest leaf
+    std::printf("%d %d\n", merge_passes(std::atoll(argv[3])),
+                merges_too_much(std::atoll(argv[1]), std::atoll(argv[2]), std::atoll(argv[3])) ? 1 : 0);
+    return 0;
+  }
   const int64_t top = INT64_C(0xFFFFFFFF);
-  const int64_t counts[] = {1, 4096, INT64_C(1) << 31, kMsdMaxRecords - 1, kMsdMaxRecords, kMsdMaxRecords + 1,
+  const int64_t counts[] = {1, 4096, INT64_C(1) << 31, 8 * kChunk - 1,
+                            8 * kChunk, 16 * kChunk - 1, 16 * kChunk, kMsdMaxRecords - 1, kMsdMaxRecords, kMsdMaxRecords + 1,
                             top - kPart2Tile, top - kEmitStep, top - 1, top};
   for (int cb = 0; cb <= 31; ++cb)
     for (int64_t r : counts) {
@@ -42,7 +50,7 @@ int main() {
 
 
 @pytest.fixture(scope="module")
-def rows(tmp_path_factory):
+def program(tmp_path_factory):
     cxx = shutil.which("g++")
     if cxx is None:
         pytest.skip("no host compiler")
@@ -50,8 +58,16 @@ def rows(tmp_path_factory):
     src, exe = d / "plan.cpp", d / "plan"
     src.write_text(PROGRAM)
     subprocess.run([cxx, "-std=c++17", "-O1", "-I", CSRC, "-o", str(exe), str(src)], check=True)
-    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
-    return [tuple(int(x) for x in line.split()) for line in out.splitlines()]
+
+    def run(*args):
+        out = subprocess.run([str(exe), *map(str, args)], check=True, capture_output=True, text=True).stdout
+        return [tuple(int(x) for x in line.split()) for line in out.splitlines()]
+    return run
+
+
+@pytest.fixture(scope="module")
+def rows(program):
+    return program()
 
 
 def test_positions_do_not_wrap(rows):
@@ -61,6 +77,21 @@ def test_positions_do_not_wrap(rows):
 
 
 def test_partition_keeps_its_range(rows):
-    """Row widths up to 24 bits and any count below the limit."""
+    """Row widths up to 24 bits and any count below the limit, unless the mean
+    leaf (at most 2^16 of them, one per row at least) is eight chunks or more."""
     for cb, r, accepted, _ in rows:
-        assert accepted == (cb <= 24 and r <= (1 << 32) - 1 - 16384), (cb, r)
+        few_rows = r >> min(cb, 16) >= 8 * 16384
+        assert accepted == (cb <= 24 and r <= (1 << 32) - 1 - 16384 and not few_rows), (cb, r)
+
+
+@pytest.mark.parametrize("records,merged,largest,passes,radix", [
+    (1 << 24, 0, 0, 0, 0),                           # no leaf above a chunk
+    (1 << 24, 16385, 16385, 1, 0),
+    (1 << 24, 1 << 24, 8 * 16384, 3, 0),             # all of them, three times
+    (1 << 24, 1 << 24, 8 * 16384 + 1, 4, 1),         # ... four times
+    (1 << 26, 3 << 23, 1 << 22, 8, 0),               # three eighths of them, eight times: 3 on average
+    (1 << 26, (3 << 23) + 1, 1 << 22, 8, 1),
+    ((1 << 32) - 1 - 16384, (1 << 32) - 1 - 16384, (1 << 32) - 1 - 16384, 18, 1),
+])
+def test_long_rows_turn_to_radix(program, records, merged, largest, passes, radix):
+    assert program(records, merged, largest) == [(passes, radix)]

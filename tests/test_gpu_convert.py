@@ -288,3 +288,59 @@ def test_builds_of_different_sizes_at_once(oracle):
     for t in threads:
         t.join()
     assert not wrong, wrong[:3]
+
+
+def _sorted_csr(n, src, dst, reverse, dedup):
+    """The CSR by one sort of 64-bit keys on the device, torch's."""
+    import torch
+    u, v = src.long(), dst.long()
+    key = u * n + v
+    if reverse:
+        key = torch.cat([key, v * n + u])
+    key = torch.unique(key) if dedup else torch.sort(key).values
+    beg = torch.searchsorted(torch.div(key, n, rounding_mode="floor"), torch.arange(n + 1, device="cuda"))
+    return beg, (key % n).int()
+
+
+@pytest.mark.parametrize("share", [0.0, 0.2, 0.35, 1.0])
+@pytest.mark.parametrize("rows", [3000, 1 << 18])
+def test_long_row_turns_to_radix(rows, share):
+    """2^24 records and one row with a share of the tuples: on both sides of
+    the share at which a large build leaves the partition for the radix sort
+    (3 of 9 merge passes at 2^23 records, a third of the forward half). A
+    second build in the same scratch follows each."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(rows + int(100 * share))
+    ne = 1 << 24
+    src, dst = (torch.randint(0, rows, (ne,), generator=gen, device="cuda", dtype=torch.int32) for _ in range(2))
+    src[torch.rand(ne, generator=gen, device="cuda") < share] = 7
+    for flags, tuples in ((L.CSR_SORT, ne), (L.CSR_SORT | L.CSR_REVERSE, ne // 2), (L.CSR_DEDUP | L.CSR_REVERSE, ne // 2),
+                          (L.CSR_SORT, 5000)):
+        s, d = src[:tuples].contiguous(), dst[:tuples].contiguous()
+        rev = bool(flags & L.CSR_REVERSE)
+        beg = torch.empty(rows + 1, dtype=torch.int64, device="cuda")
+        adj = torch.empty(tuples * (2 if rev else 1), dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        _say(f"[gpu] csr_build, one row with {share} of {tuples} tuples, {rows} rows, flags={flags}")
+        m, _ = convert.csr_build_device(rows, tuples, s.data_ptr(), d.data_ptr(), flags, beg.data_ptr(), adj.data_ptr(),
+                                        adj.numel())
+        want_beg, want_adj = _sorted_csr(rows, s, d, rev, bool(flags & L.CSR_DEDUP))
+        assert m == want_adj.numel()
+        assert torch.equal(beg, want_beg) and torch.equal(adj[:m], want_adj), flags
+
+
+@pytest.mark.parametrize("rows,ne", [(1, 131071), (1, 131072), (2, 262143), (2, 262144), (64, 8 << 20), (64, (8 << 20) - 1)])
+def test_few_rows(rows, ne):
+    """Both sides of eight chunks a row, from where the radix sort is taken."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(ne)
+    src, dst = (torch.randint(0, rows, (ne,), generator=gen, device="cuda", dtype=torch.int32) for _ in range(2))
+    beg = torch.empty(rows + 1, dtype=torch.int64, device="cuda")
+    adj = torch.empty(ne, dtype=torch.int32, device="cuda")
+    for flags in (L.CSR_SORT, L.CSR_DEDUP):
+        torch.cuda.synchronize()
+        _say(f"[gpu] csr_build, {rows} rows, {ne} tuples, flags={flags}")
+        m, _ = convert.csr_build_device(rows, ne, src.data_ptr(), dst.data_ptr(), flags, beg.data_ptr(), adj.data_ptr(), ne)
+        want_beg, want_adj = _sorted_csr(rows, src, dst, False, bool(flags & L.CSR_DEDUP))
+        assert m == want_adj.numel()
+        assert torch.equal(beg, want_beg) and torch.equal(adj[:m], want_adj), flags
