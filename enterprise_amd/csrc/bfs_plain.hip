@@ -563,6 +563,7 @@ __device__ void bu_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COU
           cw[x] = j0 + x < CW ? wc[j0 + x] : 0ull;
           const long long hv = (w0 + j0 + x) * 64 + lane;
           h[x] = ((cw[x] >> lane) & 1) ? a.head[hv] : INT32_MAX;
+          tl.e(int((cw[x] >> lane) & 1));
         }
 #pragma unroll
         for (int x = 0; x < kBuWords; ++x) {
@@ -583,6 +584,7 @@ __device__ void bu_phase(const Args &a, Smem<BS> &sm, int L, int slot, Tally<COU
           if (bit[x]) {
             const int hv = int((w0 + j0 + x) * 64) + lane;
             const long long d = a.off[hv + 1] - a.off[hv];
+            tl.v(1);
             a.depth[hv] = L + 1;
             nf += 1;
             mf += (unsigned long long)d;
@@ -1233,7 +1235,7 @@ __device__ __forceinline__ void run_phase(const Args &a, Smem<BS> &sm, long long
 
 // Launch i of a search: one phase. No end-of-launch synchronisation: the next
 // launch derives the next state itself.
-// HUB: the variant with the LDS hub table; COUNT: the variant that tallies
+// HUB: the variant with the LDS hub table; COUNT: the variants that tally
 // examined work (each only launched when configured).
 //
 // Held to 8 wavefronts per SIMD: with 7, which 82 SGPRs leave it, the grid has a
@@ -1244,7 +1246,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_
   __shared__ Smem<BS> sm;
   begin_launch<BS, COUNT>(a, sm, i, false);
   if (sm.S.done) return;
-  run_phase<BS, HUB, COUNT, COUNT && !HUB, false>(a, sm, i);
+  run_phase<BS, HUB, COUNT, false, false>(a, sm, i);
 }
 
 // The same for skewed graphs: its queue-driven levels deal out the edges of hubs,
@@ -1252,12 +1254,12 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_
 // phase wants 68 VGPRs and 88 SGPRs, which leaves 7 wavefronts per SIMD and a
 // grid of 8 blocks per CU with a last wave of its own (a search of 2^22 vertices
 // then takes 174 us); held to 8, at 7 spilled SGPRs, it is 138.
-template <int BS, bool HEAD>
+template <int BS, bool HEAD, bool COUNT>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8))) void k_level_skew(Args a, long long i) {
   __shared__ Smem<BS> sm;
-  begin_launch<BS, false>(a, sm, i, false);
+  begin_launch<BS, COUNT>(a, sm, i, false);
   if (sm.S.done) return;
-  run_phase<BS, false, false, true, HEAD>(a, sm, i);
+  run_phase<BS, false, COUNT, true, HEAD>(a, sm, i);
 }
 
 // A small graph's search in one block (ent_tiny.h). The first wavefront
@@ -1667,14 +1669,18 @@ KernelSet kernel_set_of() {
           reinterpret_cast<const void *>(&k_persist<BS, HUB, COUNT>), sizeof(Smem<BS>)};
 }
 
+template <int BS, bool COUNT>
+KernelSet kernel_set(bool hub, bool skew, bool head) {
+  if (hub) return kernel_set_of<BS, true, COUNT>();
+  KernelSet ks = kernel_set_of<BS, false, COUNT>();
+  if (head) ks.level = reinterpret_cast<const void *>(&k_level_skew<BS, true, COUNT>);
+  else if (skew) ks.level = reinterpret_cast<const void *>(&k_level_skew<BS, false, COUNT>);
+  return ks;
+}
+
 template <int BS>
 KernelSet kernel_set(bool hub, bool count, bool skew, bool head) {
-  if (count) return hub ? kernel_set_of<BS, true, true>() : kernel_set_of<BS, false, true>();
-  if (hub) return kernel_set_of<BS, true, false>();
-  KernelSet ks = kernel_set_of<BS, false, false>();
-  if (head) ks.level = reinterpret_cast<const void *>(&k_level_skew<BS, true>);
-  else if (skew) ks.level = reinterpret_cast<const void *>(&k_level_skew<BS, false>);
-  return ks;
+  return count ? kernel_set<BS, true>(hub, skew, head) : kernel_set<BS, false>(hub, skew, head);
 }
 
 KernelSet kernels_for(int bs, bool hub, bool count, bool skew, bool head) {

@@ -122,8 +122,11 @@ typedef struct ent_stats {
   int32_t grid_blocks;      /* blocks per level launch / persistent grid */
   int32_t block_size;       /* threads per block */
   int64_t examined_edges;   /* with count_examined: adjacency entries loaded
-                               (every direction, the early exits included);
-                               else -1 */
+                               (every direction, the early exits included, and
+                               the first neighbours tried from their own
+                               array); else -1. Small and low-degree graphs,
+                               which other kernels search uncounted, are
+                               counted in the form of a launch per level */
   int64_t examined_bytes;   /* with count_examined: 8 B per adjacency entry
                                loaded (entry + its status lookup), 8 B per
                                vertex whose offsets were loaded, and the bytes

@@ -545,3 +545,22 @@ def test_queue_level_hubs_largest_grids(oracle, blocks):
         dg.configure(direction=L.DIR_TOPDOWN, block_size=1024, grid_blocks=blocks)
         root = int(g.pick_roots(1, 4)[0])
         _check(oracle, g, dg, root, f"hubs, {blocks} blocks")
+
+
+def test_examined_counts_of_first_neighbours(oracle):
+    """The tally describes the kernel that runs uncounted: on a large skewed
+    graph bottom-up levels try a vertex's first neighbour alone before its row.
+    Four hubs that share every leaf, from the first hub: a leaf examines one
+    entry (its row, four), the other hubs their whole rows once, and a few at
+    their own level."""
+    hubs, n = 4, 1 << 19
+    leaves = n - hubs
+    src = np.repeat(np.arange(hubs), leaves)
+    dst = np.tile(np.arange(hubs, n), hubs)
+    g = HostGraph.from_edges(n, src, dst)
+    with DeviceGraph(g) as dg:
+        dg.configure(direction=L.DIR_BOTTOMUP, count_examined=1)
+        st = _check(oracle, g, dg, 0, "count/first neighbours")
+        assert (hubs - 1) * leaves + leaves <= st["examined_edges"] < ((hubs - 1) + 1.05) * leaves, st
+        dg.configure(count_examined=0)
+        _check(oracle, g, dg, 0, "first neighbours")
