@@ -51,6 +51,8 @@
 //   depth int32[n], visited u64[W], front[2] u64[W], mark u8[n],
 //   qbuf[2] int32[64 * 4096], Control (states, counters, grid barrier).
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <chrono>
@@ -1998,13 +2000,17 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
 // queues and control block.
 // Pinned memory of copy_depths: blocks and halves of this many vertices, for graphs
 // of kNarrowVertices to kNarrowEnd - 1. Smaller ones gain nothing (one block
-// searches them, and their copy is one short transfer); at 2^23, 32 MiB of
-// depths, C libraries hand out fresh pages for every array, and several threads
-// (copy_to_host) write those sooner than one: 12 million vertices 2,640 us
-// there, 2,770 here, but 8 million 1,430 and 900.
+// searches them, and their copy is one short transfer). From kNarrowFresh on, a
+// destination whose pages are not mapped yet is left to copy_to_host: its
+// several threads meet the page faults sooner than the one that widens here. A
+// search with its copy, there and here (us): into arrays used before 2^22 vertices
+// 1,120 and 600, 6 x 2^20 1,510 and 750, 2^23 1,880 and 1,290; into new ones 1,330
+// and 1,430, 1,640 and 1,900, 2,090 and 2,490. At 2^23, 32 MiB of depths, C
+// libraries map new pages for every array, and the rule ends.
 constexpr int kNarrowBlock = 1 << 14;
 constexpr int64_t kNarrowHalf = 1 << 20;
 constexpr int64_t kNarrowVertices = 1 << 15;
+constexpr int64_t kNarrowFresh = 1 << 22;
 constexpr int64_t kNarrowEnd = 1 << 23;
 
 int alloc_workspace(ent_graph *g) {
@@ -2342,20 +2348,38 @@ int wait_narrow(ent_graph *g, const unsigned *flag, unsigned tag) {
   return ENT_OK;
 }
 
+// Whether most of the pages behind [p, p + bytes) are mapped already, from 16
+// of them.
+bool pages_mapped(const void *p, size_t bytes) {
+  const uintptr_t page = uintptr_t(sysconf(_SC_PAGESIZE));
+  constexpr int kSamples = 16;
+  int mapped = 0;
+  for (int k = 0; k < kSamples; ++k) {
+    unsigned char in = 1;
+    const uintptr_t at = (reinterpret_cast<uintptr_t>(p) + bytes / kSamples * size_t(k)) & ~(page - 1);
+    if (mincore(reinterpret_cast<void *>(at), page, &in) != 0) return true;
+    mapped += in & 1;
+  }
+  return 2 * mapped > kSamples;
+}
+
 // The handle's depths, of a search of `levels` levels, into host memory.
 // Pageable destinations get them as bytes through pinned memory, widened here
 // block by block as they arrive: the runtime's own copy to pageable memory
 // moves four times the bytes and alternates transfer and host copy. The
 // transfer of 2^20 ints alone takes 83 us, of as many bytes 28, one thread's
-// widening 54. A search with its copy, before and now, R-MAT, edge factor 8:
-// 32,768 vertices 120 and 108 us, 2^18 196 and 143, 2^20 370 and 185, 2^22 870
-// and 436.
+// widening 54. A search with its copy into the same array again, before and now,
+// R-MAT, edge factor 8: 32,768 vertices 120 and 108 us, 2^18 196 and 143, 2^20 370
+// and 185, 2^22 870 and 436. Into a new array every time the page faults are the
+// larger part: uniform, edge factor 6, 2^18 497 and 264, 2^20 1,049 and 573, 2^21
+// 1,565 and 830.
 int copy_depths(ent_graph *g, int32_t *dst, int levels) {
   hipPointerAttribute_t attr;
   bool pageable = true;
   if (hipPointerGetAttributes(&attr, dst) == hipSuccess) pageable = attr.type == hipMemoryTypeUnregistered;
   else ignore(hipGetLastError());  // pageable memory is unknown to the runtime
-  if (!g->narrow || !pageable || levels > 255)
+  if (!g->narrow || !pageable || levels > 255 ||
+      (g->n >= kNarrowFresh && !pages_mapped(dst, sizeof(int32_t) * size_t(g->n))))
     return copy_to_host(g, dst, g->depth, sizeof(int32_t) * size_t(g->n));
   const int64_t halves = (g->n + kNarrowHalf - 1) / kNarrowHalf;
   unsigned tags[2];

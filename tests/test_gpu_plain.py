@@ -564,3 +564,22 @@ def test_examined_counts_of_first_neighbours(oracle):
         assert (hubs - 1) * leaves + leaves <= st["examined_edges"] < ((hubs - 1) + 1.05) * leaves, st
         dg.configure(count_examined=0)
         _check(oracle, g, dg, 0, "first neighbours")
+
+
+@pytest.mark.parametrize("n", [(1 << 22) - 1, (1 << 22) + 1, (1 << 23) - 5])
+def test_depths_to_new_and_used_arrays(n):
+    """Depths into arrays whose pages are mapped, not mapped, and mapped in part,
+    on both sides of the size from where they take different ways."""
+    src = np.arange(n - 9)
+    g = HostGraph.from_edges(n, np.zeros(n - 9, np.int64), src)  # a star and eight vertices apart
+    want = np.full(n, -1, dtype=np.int32)
+    want[: n - 9] = 1
+    want[0] = 0
+    with DeviceGraph(g) as dg:
+        part = np.empty(n + 3, dtype=np.int32)
+        part[: n // 3] = 7
+        for name, out in (("new", np.empty(n, dtype=np.int32)), ("used", np.full(n, 7, dtype=np.int32)),
+                          ("part", part[:n]), ("part, unaligned", part[3:])):
+            print(f"[gpu] depths to host, {name} array, n={n}", flush=True)
+            L.check(L.lib().ent_bfs(dg.handle, 0, out.ctypes.data_as(L.i32p), None))
+            assert np.array_equal(out, want), name
