@@ -1957,7 +1957,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
       // parity (state slot) and residue mod 3 (counter slot) across replays.
       const int k = std::max(6, (cfg.graph_levels + 5) / 6 * 6);
       const int grid = level_grid(g);
-      if (!g->gexec || g->graph_bs != bs || g->graph_grid != grid || g->graph_k != k ||
+      if (!g->gexec || g->graph_fn != ks.level || g->graph_bs != bs || g->graph_grid != grid || g->graph_k != k ||
           std::memcmp(g->graph_args, &a, sizeof(Args)) != 0) {
         if (g->gexec) ignore(hipGraphExecDestroy(g->gexec));
         if (g->graph) ignore(hipGraphDestroy(g->graph));
@@ -1972,6 +1972,7 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
         g->graph = gr;
         HIP_TRY(hipGraphInstantiate(&g->gexec, g->graph, nullptr, nullptr, 0));
         std::memcpy(g->graph_args, &a, sizeof(Args));
+        g->graph_fn = ks.level;
         g->graph_bs = bs;
         g->graph_grid = grid;
         g->graph_k = k;

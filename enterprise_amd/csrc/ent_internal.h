@@ -107,6 +107,7 @@ struct ent_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   unsigned char graph_args[512] = {};  // launch arguments baked into the captured graph
+  const void *graph_fn = nullptr;           // and its kernel
   int graph_bs = 0, graph_grid = 0, graph_k = 0;
   size_t dev_bytes = 0;
   size_t dev_limit = 0;  // dev_alloc fails beyond it (tests; 0: none)

@@ -583,3 +583,18 @@ def test_depths_to_new_and_used_arrays(n):
             print(f"[gpu] depths to host, {name} array, n={n}", flush=True)
             L.check(L.lib().ent_bfs(dg.handle, 0, out.ctypes.data_as(L.i32p), None))
             assert np.array_equal(out, want), name
+
+
+def test_graph_launch_follows_the_kernel(oracle, rmat16):
+    """A captured graph is not replayed for another kernel: the tally is on and
+    off in turn with everything else as it was."""
+    g, dg = rmat16
+    base = dg.config
+    root = int(g.pick_roots(1, 405)[0])
+    try:
+        for count in (0, 1, 0, 1, 1):
+            dg.configure(direction=L.DIR_TOPDOWN, launch=L.LAUNCH_GRAPH, count_examined=count)
+            st = _check(oracle, g, dg, root, f"graph/count={count}")
+            assert st["examined_edges"] == (st["reached_edges"] if count else -1), st
+    finally:
+        dg.set_config(base)
