@@ -2001,13 +2001,14 @@ int run_search(ent_graph *g, int root, int *depth_dev, State *fin) {
 // queues and control block.
 // Pinned memory of copy_depths: blocks and halves of this many vertices, for graphs
 // of kNarrowVertices to kNarrowEnd - 1. Smaller ones gain nothing (one block
-// searches them, and their copy is one short transfer). From kNarrowFresh on, a
-// destination whose pages are not mapped yet is left to copy_to_host: its
-// several threads meet the page faults sooner than the one that widens here. A
-// search with its copy, there and here (us): into arrays used before 2^22 vertices
-// 1,120 and 600, 6 x 2^20 1,510 and 750, 2^23 1,880 and 1,290; into new ones 1,330
-// and 1,430, 1,640 and 1,900, 2,090 and 2,490. At 2^23, 32 MiB of depths, C
-// libraries map new pages for every array, and the rule ends.
+// searches them, and their copy is one short transfer). The thread that widens
+// meets the page faults of a destination that is not mapped yet, so from
+// kNarrowFresh on several threads touch its pages first. A search with its copy
+// by copy_to_host, here, and here without that (us): into new arrays 2^22 vertices
+// 1,390, 1,370 and 1,430, 6 x 2^20 1,810, 1,760 and 1,880, 2^23 2,220, 2,340 and
+// 2,440 (a handle's first 4,300, 3,400 and 2,980); into arrays used before 1,120 and
+// 600, 1,510 and 750, 1,880 and 1,290. At 2^23, 32 MiB of depths, C libraries map
+// new pages for every array, and the rule ends.
 constexpr int kNarrowBlock = 1 << 14;
 constexpr int64_t kNarrowHalf = 1 << 20;
 constexpr int64_t kNarrowVertices = 1 << 15;
@@ -2141,10 +2142,11 @@ int ent_graph_upload_ex(const int64_t *beg_pos, const int32_t *adj, int64_t n, i
 namespace ent {
 
 // A graph is skewed if its largest degree is kSkew times the mean or more. Only
-// such graphs get heads (bu_phase), as their first neighbours are hubs. Uniform random graphs of edge factor 8 have a largest degree of 2-3
-// times the mean and lose by them (200,000 vertices 132 us without, 136 with);
-// R-MAT ones have 30 times and more at every size. Below 2^19 vertices a level
-// is launch-bound (2^18: 74.5 us without, 75.2 with; 2^19 91.8 and 90.2).
+// such graphs get heads (bu_phase), as their first neighbours are hubs. Uniform
+// random graphs of edge factor 8 have a largest degree of 2-3 times the mean and
+// lose by them (200,000 vertices 132 us without, 136 with); R-MAT ones have 30
+// times and more at every size. Below 2^19 vertices a level is launch-bound
+// (2^18: 74.5 us without, 75.2 with; 2^19 91.8 and 90.2).
 // Rows in the caller's order find less with their first neighbour: 2^21
 // vertices 131 and 133 us, 2^22 160 and 152, 2^23 559 and 419.
 constexpr int64_t kSkew = 16;
@@ -2379,8 +2381,7 @@ int copy_depths(ent_graph *g, int32_t *dst, int levels) {
   bool pageable = true;
   if (hipPointerGetAttributes(&attr, dst) == hipSuccess) pageable = attr.type == hipMemoryTypeUnregistered;
   else ignore(hipGetLastError());  // pageable memory is unknown to the runtime
-  if (!g->narrow || !pageable || levels > 255 ||
-      (g->n >= kNarrowFresh && !pages_mapped(dst, sizeof(int32_t) * size_t(g->n))))
+  if (!g->narrow || !pageable || levels > 255)
     return copy_to_host(g, dst, g->depth, sizeof(int32_t) * size_t(g->n));
   const int64_t halves = (g->n + kNarrowHalf - 1) / kNarrowHalf;
   unsigned tags[2];
@@ -2396,6 +2397,11 @@ int copy_depths(ent_graph *g, int32_t *dst, int levels) {
     return ENT_OK;
   };
   int rc = launch_half(0);
+  if (!rc && g->n >= kNarrowFresh && !pages_mapped(dst, sizeof(int32_t) * size_t(g->n)))
+    parallel_for(g->n, 1 << 19, [&](int64_t b, int64_t e) {
+      volatile int32_t *d = dst;
+      for (int64_t v = b; v < e; v += 1024) d[v] = 0;  // one write per 4 KiB, wherever pages begin
+    });
   for (int64_t c = 0; c < halves && !rc; ++c) {
     if (c + 1 < halves && (rc = launch_half(c + 1))) break;  // half c - 1 is drained
     const int b = int(c & 1);
