@@ -122,6 +122,14 @@ def batch(args):
 MODES["batch"] = batch
 
 
+def _batch_form(st):
+    """How a batch ran, and the flushes it made: searches side by side run
+    several levels a launch and keep no levels (their ent_batch_stats.flushes
+    is the count a joint search would make)."""
+    side = st["phases"] < st["levels"]
+    return {"form": "side by side" if side else "joint", "flushes": 0 if side else st["flushes"]}
+
+
 def grid(args):
     """Config 3: 4096 x 4096 4-neighbour grid, 2% of edges deleted (seed
     4096), largest component kept, 16 seeded roots. Compares the launch forms
@@ -193,9 +201,9 @@ def grid(args):
         single_hash.append(int(dg.row_hash(dg.depth_device_ptr(), 1, g.n)[0]))
         single_levels.append(st["levels"])
     best = min(res, key=lambda k: res[k]["ms_per_bfs"])
-    # The same graph as one 64-source batch keeping 250 levels (the most the
-    # level ring holds: it flushes to the rows about every 251 levels),
-    # against 64 searches at the best form's mean time; four rows checked
+    # The same graph as one 64-source batch on a workspace that keeps 250 levels
+    # (the most the level ring holds; a joint search flushes to the rows about
+    # every 251 levels, searches side by side keep none), against 64 searches at the best form's mean time; four rows checked
     # against the single-source path. Then the 16 roots above as one 16-source
     # batch: every row against its single-source row, and the batch time per
     # root and per level of a root (a multi-source form of the same 16
@@ -228,7 +236,7 @@ def grid(args):
                        # the best form's cost per level times the 16 roots' mean depth
                        "speedup_vs_best_form": round(res[best]["us_per_level"] * float(np.mean(single_levels))
                                                      / (per_root * 1e3), 2),
-                       "levels": st16["levels"], "flushes": st16["flushes"],
+                       "levels": st16["levels"], **_batch_form(st16),
                        "rows_checked": k16,
                        "rows_mismatching_single_source": int(sum(int(h16[i]) != single_hash[i]
                                                                  for i in range(k16)))}
@@ -237,7 +245,7 @@ def grid(args):
             dg.device_free(out)
             dg.batch_release()
         batch = {"k": k, "roots_seed": 1007, "batch_ms": round(bms, 1), "levels": st["levels"],
-                 "flushes": st["flushes"], "kept_levels": 250,
+                 **_batch_form(st), "kept_levels": 250,
                  "speedup_vs_plain": round(k * res[best]["ms_per_bfs"] / bms, 2),
                  "rows_checked": 4, "rows_mismatching_plain": mism}
         log(f"[grid] batch of {k}: {batch}")
@@ -411,20 +419,18 @@ def csr(args):
     parity = bool(np.array_equal(beg, h.beg_pos) and np.array_equal(adj, h.adj))
     dev_ms = float(np.median(ms))
     alg = 8 * ne + 4 * m + 8 * (n + 1)
-    passes = (st["key_bits"] + 7) // 8
     return {"mode": "csr", "metric": "CSR construction from raw tuples, million tuples/s", "unit": "Mtuples/s",
             "value": round(ne / (dev_ms * 1e3), 1), "higher_is_better": True, "ms": round(dev_ms, 3),
             "ms_all": [round(x, 3) for x in ms],
             "config": {"workload": f"R-MAT scale {scale} ef 16 raw tuples (seed {scale}, relabelled) -> "
                                    "symmetric CSR, loops and duplicates dropped, rows sorted",
                        "n": n, "tuples": ne, "m": int(m), "records": int(st["records"]),
-                       "key_bits": int(st["key_bits"]), "radix_passes": int(passes)},
+                       "key_bits": int(st["key_bits"])},
             "parity_vs_host_generator": parity,
             "roofline": {"bound": "hbm", "achieved": round(alg / (dev_ms * 1e-3) / 1e9, 1), "peak": 8000.0,
                          "unit": "GB/s", "frac": round(alg / (dev_ms * 1e-3) / 8e12, 4),
                          "traffic": None,
-                         "algorithmic_bytes": int(alg),
-                         "sort_bytes_estimate": int(st["records"]) * 2 * 8 * passes},
+                         "algorithmic_bytes": int(alg)},
             "cpu_host_builder": {"value": round(ne / (host_s * 1e6), 1), "unit": "Mtuples/s",
                                  "threads": min(os.cpu_count() or 1, 16),
                                  "sample": f"library host builder (ent_csr_from_edges) on the same {ne} tuples",

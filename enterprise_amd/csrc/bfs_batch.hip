@@ -1346,8 +1346,8 @@ __global__ void k_binit_src(BArgs a, const int *roots, BInit in) {
 // 2^64). Block (c, r) sums chunk c of row r and adds it to out[r]. Four values
 // per lane and step, in one 16-byte load where the rows allow it (VEC: the
 // first row 16-byte aligned and cols a multiple of four). Bound: the two
-// 64-bit products a value takes (about 60 us for 64 rows of 2^20), as much as
-// the 268 MB of loads; XXX.
+// 64-bit products a value takes and the loads, about alike: 64 rows of 2^20
+// (268 MB) take 61.5 us, 4.4 TB/s; 144 with one value per lane and step.
 __device__ __forceinline__ unsigned long long hash_mix(long long i, int value) {
   unsigned long long z = ((unsigned long long)i << 32) ^ (unsigned int)value;
   z += 0x9E3779B97F4A7C15ull;

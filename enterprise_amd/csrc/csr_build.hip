@@ -1,7 +1,13 @@
 // Edge list to CSR on the device, behind include/ent_convert.h. The
 // reference builds its CSR on the host, tuple by tuple, in file order
 // (tuple_text_to_binary_csr/tuple_text_to_bin.cpp:190-248); this file
-// gives every stored entry one 64-bit record and radix-sorts the records:
+// sorts one record per stored entry.
+//
+// Sorted rows without weights, the form that the searches use, take the
+// partition of csr_msd.h, as long as csr_plan.h's rules hold. Every other
+// form, and what those rules leave out (n above 2^24, few or very long rows,
+// record counts next to 2^32), gives each entry a 64-bit record and
+// radix-sorts the records:
 //
 //   record r (tuple i = r / 2 with ENT_CSR_REVERSE, else i = r; the odd
 //   record of a reversed tuple is (dst, src)):
@@ -9,16 +15,16 @@
 //     sorted rows : key = row << cb | col          (cb = bits of n)
 //   a dropped self-loop gets row = n and sorts behind every row.
 //
-// Sorted rows without weights sort the keys alone; the other forms carry the
+// There, sorted rows without weights sort the keys alone; the others carry the
 // record index (u32) to fetch the column and weight afterwards. Then, per
 // tile of 4096 sorted records: the count of kept records (real row, and with
 // dedup a key unlike its predecessor's), a scan of the tile counts, and one
 // assembly pass that writes each kept record at its rank: its column and
 // weight, and beg_pos at the row boundaries.
 //
-// HBM traffic per record: the radix sort's passes over 8-byte keys (and
-// 4-byte indices), one pass per 8 key bits; the record and assembly kernels
-// read the tuples once and write the CSR once.
+// HBM traffic per record of that form: the radix sort's passes over 8-byte keys
+// (and 4-byte indices), one pass per 8 key bits; the record and assembly
+// kernels read the tuples once and write the CSR once.
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
