@@ -675,6 +675,14 @@ int ent_csr_release_scratch(int32_t device) {
   return ENT_OK;
 }
 
+// For tests, not in the public headers: bytes of scratch kept idle on `device`.
+int64_t ent_internal_scratch_bytes(int32_t device) {
+  std::lock_guard<std::mutex> lk(g_idle_mu);
+  for (const BuildContext *c = g_idle; c; c = c->next)
+    if (c->device == device) return int64_t(c->bytes);
+  return 0;
+}
+
 int ent_csr_build_device(int32_t device, int64_t n, int64_t ne, const int32_t *src_dev, const int32_t *dst_dev,
                          int32_t flags, int64_t *beg_pos_dev, int32_t *adj_dev, int64_t adj_capacity,
                          int64_t *m_out, ent_build_stats *st) {

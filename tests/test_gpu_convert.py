@@ -3,10 +3,10 @@ oracle: every flag combination bit for bit (offsets, adjacency, weights),
 the raw R-MAT tuples against the host generator's CSR, the ent_convert CLI
 against the reference converter's committed outputs, and BFS on a handle
 built from tuples."""
+import ctypes as C
 import os
 import subprocess
 import sys
-import time
 
 import numpy as np
 import pytest
@@ -219,44 +219,26 @@ def test_partition_drops_every_record():
 def test_scratch_is_kept_and_given_back():
     """The scratch of a construction serves the next one, and goes back when
     the program asks for it and when a handle of the device is freed."""
-    import torch
-    n, ne = 1 << 20, 1 << 24
-    src = torch.randint(0, n, (ne,), dtype=torch.int32, device="cuda")
-    dst = torch.randint(0, n, (ne,), dtype=torch.int32, device="cuda")
-    beg = torch.empty(n + 1, dtype=torch.int64, device="cuda")
-    adj = torch.empty(2 * ne, dtype=torch.int32, device="cuda")
+    kept = L.lib().ent_internal_scratch_bytes
+    kept.argtypes, kept.restype = [C.c_int32], C.c_int64
+    src, dst = _tuples(17, 1 << 16, 200000)
 
-    def build():
-        torch.cuda.synchronize()
-        m, _ = convert.csr_build_device(n, ne, src.data_ptr(), dst.data_ptr(), convert.SIMPLE, beg.data_ptr(),
-                                        adj.data_ptr(), 2 * ne)
-        return m
+    def build(tuples):
+        g, _, _ = convert.csr_build(1 << 16, src[:tuples], dst[:tuples], convert.SIMPLE)
+        return g.m
 
-    def free():
-        """Free device memory once it has settled: the driver clears what was
-        freed, by earlier tests too, in its own time before it counts."""
-        torch.cuda.synchronize()
-        seen = []
-        for _ in range(100):
-            seen.append(torch.cuda.mem_get_info()[0])
-            if len(seen) > 8 and len(set(seen[-8:])) == 1:
-                break
-            time.sleep(0.2)
-        return seen[-1]
-
-    m = build()
     convert.release_scratch()
-    start = free()
-    slack = 64 << 20
+    assert kept(0) == 0
     for give_back in (convert.release_scratch, lambda: DeviceGraph(HostGraph.rmat(8, 4, seed=1)).free()):
         _say("[gpu] construction scratch")
-        assert build() == m
-        kept = start - free()
-        assert kept > 8 * 2 * ne  # more than the records' keys
-        assert build() == m
-        assert abs(start - free() - kept) < slack
+        m = build(src.size)
+        size = kept(0)
+        assert 8 * 2 * src.size < size < 1 << 30  # more than the records' keys
+        assert build(src.size) == m and kept(0) == size
+        build(1000)  # a smaller one runs in the same block
+        assert kept(0) == size
         give_back()
-        assert abs(start - free()) < slack
+        assert kept(0) == 0
     convert.release_scratch()  # nothing left: no error
     for device in (-1, 1 << 20):
         with pytest.raises(EntError):
